@@ -354,15 +354,20 @@ static void launch_stencil(bool pv2, dim3 g, hipStream_t st, const StencilArgs &
 /* device: Gram on the matrix cores                                           */
 /* ------------------------------------------------------------------------- */
 
+/* elements before row i of a packed lower triangle (and of a whole triangle of i rows): partial Gram matrices hold
+ * only element (i, j <= i) of the parameters, 91 of the 256 for 13 parameters */
+__host__ __device__ constexpr int gram_tri(int i) { return i * (i + 1) / 2; }
+
 /* The operand rows of a point lie in planes (detector, real / imaginary part), component-major: component i of
  * bin k at plane[i * N + k], so the stencil kernels write whole waves of consecutive bins.  Each block: up to
  * GWH_GRAM_ROWS bins of one plane of one point, 4 waves; each wave accumulates a 16x16 tile of a a^T over its
  * bins, 4 bins per MFMA (lane l supplies component l%16 of bin k0 + l/16 as both A and B operand; eight
- * MFMAs' operands are loaded first, 32 consecutive bins of each component).  Output: per block 256 FP64
- * partial sums. */
+ * MFMAs' operands are loaded first, 32 consecutive bins of each component).  Output: per block the FP64 partial
+ * sums of the lower triangle of the dim parameters (gram_tri). */
 template <typename T>
 __global__ __launch_bounds__(GWH_TPB) void gwh_gram_kernel(const T *__restrict__ rows, int N, int nplanes,
-                                                           int blk_per_plane, double *__restrict__ partial, int nblk)
+                                                           int blk_per_plane, double *__restrict__ partial, int nblk,
+                                                           int dim)
 {
     __shared__ double lds[GWH_TPB / 64][256];
     const int pt = blockIdx.y, blk = blockIdx.x;
@@ -407,12 +412,20 @@ __global__ __launch_bounds__(GWH_TPB) void gwh_gram_kernel(const T *__restrict__
         lds[wv][row * 16 + (lane & 15)] = out[j];
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < 256; e += GWH_TPB) {
-        double s = lds[0][e];
-        for (int w = 1; w < GWH_TPB / 64; w++) s += lds[w][e];
-        partial[((size_t)pt * nblk + blk) * 256 + e] = s;
+    const int ei = threadIdx.x >> 4, ej = threadIdx.x & 15;
+    if (ei < dim && ej <= ei) {
+        double s = lds[0][threadIdx.x];
+        for (int w = 1; w < GWH_TPB / 64; w++) s += lds[w][threadIdx.x];
+        partial[((size_t)pt * nblk + blk) * gram_tri(dim) + gram_tri(ei) + ej] = s;
     }
 }
+
+/* Column of the LDS plane that holds bin `col` of operand row `row` in the fused kernel: rows are rotated by two
+ * bins each, so that the 32 lanes of a half wave, which read bins 4 q + {0, 1} or {2, 3} of all 16 rows, touch 32
+ * different bank pairs.  Unrotated, the 16 rows (512 bytes apart) share their banks: SQ_LDS_BANK_CONFLICT was 9.4e7
+ * of 1.2e8 LDS cycles of a 128-point pass of the 13-parameter IMRPhenomPv2 Fisher (846 -> 838 us: the vector ALU
+ * covered most of them). */
+__device__ __forceinline__ int fused_col(int row, int col) { return (col + 2 * row) & (GWH_FUSED_BINS - 1); }
 
 /* The stencil and the FP64 Gram in one kernel: one block of GWH_FROWS waves per (point, chunk of 64 bins).  Wave
  * i evaluates operand row i -- the S stencil evaluations of component i, unrolled, projected on every detector and
@@ -489,8 +502,8 @@ __global__ __launch_bounds__(WAVES * 64) void gwh_fisher_fused_kernel(StencilArg
         }
         for (int dd = 0; dd < GWH_MAXDET; dd++) {
             if (dd >= a.d_count) break;
-            lds[2 * dd][i][lane] = dr[dd];
-            lds[2 * dd + 1][i][lane] = di[dd];
+            lds[2 * dd][i][fused_col(i, lane)] = dr[dd];
+            lds[2 * dd + 1][i][fused_col(i, lane)] = di[dd];
         }
     }
     __syncthreads();
@@ -498,40 +511,53 @@ __global__ __launch_bounds__(WAVES * 64) void gwh_fisher_fused_kernel(StencilArg
     const int nslice = 2 * a.d_count * (GWH_FUSED_BINS / 4);
     for (int t = wv; t < nslice; t += WAVES) {
         const int pl = t / (GWH_FUSED_BINS / 4), q = t % (GWH_FUSED_BINS / 4);
-        const double x = lds[pl][lane & 15][4 * q + (lane >> 4)];
+        const int row = lane & 15;
+        const double x = lds[pl][row][fused_col(row, 4 * q + (lane >> 4))];
         acc = __builtin_amdgcn_mfma_f64_16x16x4f64(x, x, acc, 0, 0, 0);
     }
     __syncthreads(); /* the planes are read: the LDS now holds the waves' partial matrices */
     double(*part)[256] = reinterpret_cast<double(*)[256]>(&lds[0][0][0]);
     for (int j = 0; j < 4; j++) part[wv][((lane >> 4) + 4 * j) * 16 + (lane & 15)] = acc[j];
     __syncthreads();
-    if (threadIdx.x < 256) {
+    /* the product of the operand with itself is symmetric bit for bit: the lower triangle of the parameters */
+    const int ei = threadIdx.x >> 4, ej = threadIdx.x & 15;
+    if (ei < a.dim && ej <= ei) {
         double sum = part[0][threadIdx.x];
         for (int w = 1; w < WAVES; w++) sum += part[w][threadIdx.x];
-        partial[((size_t)pt * nbc + bc) * 256 + threadIdx.x] = sum;
+        partial[((size_t)pt * nbc + bc) * gram_tri(a.dim) + gram_tri(ei) + ej] = sum;
     }
 }
 
-/* Fixed-order FP64 sum of the Gram partials, one block of 1024 threads per point: thread (q, e) sums element e of
- * the 16x16 partials of blocks q, q + 4, ... in increasing order, the four sums are added as (s0 + s1) + (s2 + s3),
- * and the output is symmetric (the upper and lower triangles are averaged, as calculate_fisher_elements assigns
- * out[k][j] = out[j][k]). */
+/* Fixed-order FP64 sum of the Gram partials: one block of 1024 threads per (point, 16 elements of the packed lower
+ * triangle).  Thread (q, e) sums its element over blocks q, q + 64, ... in increasing order (16 consecutive elements
+ * per load, 128 bytes), the 64 sums are added pairwise in LDS, and each element is written to both halves of the
+ * matrix, as calculate_fisher_elements assigns out[k][j] = out[j][k].  The loads of a thread are a serial chain, so
+ * the blocks are spread over 64 threads per element and not over four: 12 points of 1025 blocks 68 -> 8.5 us, 128
+ * points of 254 blocks 18.7 -> 7.3 us. */
 __global__ __launch_bounds__(1024) void gwh_gram_reduce_kernel(const double *__restrict__ partial, int nblk, int dim,
                                                                double scale, double *__restrict__ out)
 {
-    __shared__ double red[4][256];
-    const int pt = blockIdx.x;
-    const int e = threadIdx.x & 255, q = threadIdx.x >> 8;
-    const double *pp = partial + (size_t)pt * nblk * 256 + e;
+    __shared__ double red[64][17];
+    const int pt = blockIdx.x, tri = gram_tri(dim);
+    const int e = blockIdx.y * 16 + (threadIdx.x & 15), q = threadIdx.x >> 4;
+    const double *pp = partial + (size_t)pt * nblk * tri + e;
     double acc = 0;
-    for (int b = q; b < nblk; b += 4) acc += pp[(size_t)b * 256];
-    red[q][e] = acc;
+    if (e < tri)
+        for (int b = q; b < nblk; b += 64) acc += pp[(size_t)b * tri];
+    red[q][threadIdx.x & 15] = acc;
     __syncthreads();
-    if (q == 0) red[0][e] = (red[0][e] + red[1][e]) + (red[2][e] + red[3][e]);
-    __syncthreads();
-    if (q == 0) {
-        const int i = e >> 4, j = e & 15;
-        if (i < dim && j < dim) out[(size_t)pt * dim * dim + i * dim + j] = 0.5 * (red[0][e] + red[0][j * 16 + i]) * scale;
+    for (int w = 32; w > 0; w >>= 1) {
+        if (q < w) red[q][threadIdx.x & 15] += red[q + w][threadIdx.x & 15];
+        __syncthreads();
+    }
+    if (q == 0 && e < tri) {
+        int i = 0;
+        while (gram_tri(i + 1) <= e) i++;
+        const int j = e - gram_tri(i);
+        const double v = red[0][threadIdx.x] * scale;
+        double *o = out + (size_t)pt * dim * dim;
+        o[i * dim + j] = v;
+        o[j * dim + i] = v;
     }
 }
 
@@ -668,14 +694,15 @@ static int fisher_run(int event, int model, int basis, int precision, const gwh_
     const int nplanes = (int)(nrows / N); /* (detector, re/im) planes of a point's operand rows */
     const int blk_per_plane = (N + GWH_GRAM_ROWS - 1) / GWH_GRAM_ROWS;
     int nblk = fused ? (N + GWH_FUSED_BINS - 1) / GWH_FUSED_BINS : nplanes * blk_per_plane;
-    if (fused) per_pt_bytes = (size_t)nblk * 256 * 8;
+    const size_t part_bytes = (size_t)nblk * gram_tri(dim) * 8; /* partial Gram matrices of a point */
+    if (fused) per_pt_bytes = part_bytes;
     int chunk = (int)std::max<size_t>(1, F.max_operand / per_pt_bytes);
     if (chunk > n) chunk = n;
     if (chunk > 65535) chunk = 65535;
     if (fused && chunk > GWH_FUSED_MAX_POINTS) chunk = GWH_FUSED_MAX_POINTS;
     int rc;
     if (!fused && (rc = F.deriv.ensure((size_t)chunk * per_pt_bytes)) != GWH_OK) return rc;
-    if ((rc = F.gram.ensure((size_t)chunk * nblk * 256 * 8)) != GWH_OK) return rc;
+    if ((rc = F.gram.ensure((size_t)chunk * part_bytes)) != GWH_OK) return rc;
     if ((rc = F.out.ensure((size_t)n * dim * dim * 8)) != GWH_OK) return rc;
     std::vector<gwh_params> inst;
     std::vector<unsigned char> no_tof;
@@ -771,15 +798,15 @@ static int fisher_run(int event, int model, int basis, int precision, const gwh_
             launch_stencil<double>(pv2, g, F.stream, a, evp, event, F.deriv.as<double>());
             GWH_HIP(hipGetLastError());
             hipLaunchKernelGGL(gwh_gram_kernel<double>, dim3(nblk, np), dim3(GWH_TPB), 0, F.stream,
-                               F.deriv.as<const double>(), N, nplanes, blk_per_plane, F.gram.as<double>(), nblk);
+                               F.deriv.as<const double>(), N, nplanes, blk_per_plane, F.gram.as<double>(), nblk, dim);
         } else {
             launch_stencil<float>(pv2, g, F.stream, a, evp, event, F.deriv.as<float>());
             GWH_HIP(hipGetLastError());
             hipLaunchKernelGGL(gwh_gram_kernel<float>, dim3(nblk, np), dim3(GWH_TPB), 0, F.stream,
-                               F.deriv.as<const float>(), N, nplanes, blk_per_plane, F.gram.as<double>(), nblk);
+                               F.deriv.as<const float>(), N, nplanes, blk_per_plane, F.gram.as<double>(), nblk, dim);
         }
         GWH_HIP(hipGetLastError());
-        hipLaunchKernelGGL(gwh_gram_reduce_kernel, dim3(np), dim3(1024), 0, F.stream, F.gram.as<const double>(),
+        hipLaunchKernelGGL(gwh_gram_reduce_kernel, dim3(np, (gram_tri(dim) + 15) / 16), dim3(1024), 0, F.stream, F.gram.as<const double>(),
                            nblk, dim, scale, F.out.as<double>() + (size_t)p0 * dim * dim);
         GWH_HIP(hipGetLastError());
     }
@@ -844,13 +871,14 @@ size_t gwh_fisher_batch_bytes(int event, int model, int basis, int precision, co
     const bool fused = !sky && precision != GWH_FISHER_GRAM_FP32;
     const size_t nblk = fused ? (ev.N + GWH_FUSED_BINS - 1) / GWH_FUSED_BINS
                               : (nrows / ev.N) * ((ev.N + GWH_GRAM_ROWS - 1) / GWH_GRAM_ROWS);
-    const size_t per_pt_bytes = fused ? nblk * 256 * 8 : nrows * GWH_FROWS * ((precision == GWH_FISHER_GRAM_FP32) ? 4 : 8);
+    const size_t part_bytes = nblk * gram_tri(dim) * 8;
+    const size_t per_pt_bytes = fused ? part_bytes : nrows * GWH_FROWS * ((precision == GWH_FISHER_GRAM_FP32) ? 4 : 8);
     size_t chunk = std::max<size_t>(1, max_operand / per_pt_bytes);
     chunk = std::min<size_t>(chunk, std::min(n, 65535));
     if (fused) chunk = std::min<size_t>(chunk, GWH_FUSED_MAX_POINTS);
     const size_t ni = chunk * per_point;
     return (fused ? F.deriv.cap : gwh_grown_capacity(chunk * per_pt_bytes, F.deriv.cap)) +
-           gwh_grown_capacity(chunk * nblk * 256 * 8, F.gram.cap) +
+           gwh_grown_capacity(chunk * part_bytes, F.gram.cap) +
            gwh_grown_capacity((size_t)n * dim * dim * 8, F.out.cap) +
            (want_sigma ? gwh_grown_capacity((size_t)n * dim * 8, F.sig.cap) : F.sig.cap) +
            gwh_grown_capacity(ni * sizeof(gwh_params), F.params.cap) +
