@@ -11,6 +11,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -125,6 +126,7 @@ struct Event {
     uint64_t last_use = 0;
     int pins = 0;          /* step graphs holding this event's buffers: no destroy, eviction or re-tiling */
     int method = 0, log10F = 0; /* integration rule of the stored weights */
+    std::shared_ptr<const std::vector<double>> chunk_fmin; /* host: smallest frequency of every chunk of 64 bins */
 };
 
 /* grow-only device buffer; a fixed one is a view of memory the buffer does not own (never grown or freed:

@@ -394,6 +394,9 @@ int gwh_event_create_ex(const double *f, int N, int ndet, const int *dets, const
     ds.lanes = gwh_choose_lanes(N);
     /* Gauss-Legendre weights carry no step: nothing to rescale */
     ds.snr_scale = (method == GWH_GAUSSLEG) ? 1.0 : df_f / ev.df_like;
+    auto chunk_fmin = std::make_shared<std::vector<double>>((N + 63) / 64, HUGE_VAL);
+    for (int k = 0; k < N; k++) (*chunk_fmin)[k / 64] = std::fmin((*chunk_fmin)[k / 64], f[k]);
+    ev.chunk_fmin = chunk_fmin;
     ds.sorted = 1;
     for (int k = 1; k < N; k++)
         if (!(f[k] >= f[k - 1])) {
@@ -1051,8 +1054,8 @@ __global__ void gwh_waveform_kernel(const double *__restrict__ f, int N, const I
     if (fk <= C.fcut) {
         const BinPow bp = gwh_bin_powers(fk);
         if (MODEL == GWH_IMRPHENOMD) {
-            double A, phi, u, lx;
-            gwh_phenomd_fp64(C, fk, bp, A, phi, u, lx);
+            double A, phi, u;
+            gwh_phenomd_fp64(C, fk, bp, A, phi, u);
             double s, c;
             gwh_sincos_table(phi, s, c);
             double hr = A * c, hi = -A * s; /* h = A e^{-i phi} */

@@ -4,11 +4,12 @@
  *   host      unpack the point into the basis of the generation method, build the central-difference
  *             stencil (the perturbed parameter sets, fisher.cpp:148-557), run the FP64 setup for all of
  *             them in one launch
- *   stencil   one lane per bin and point: every perturbed waveform/response evaluated in FP64, the FP64
- *             difference quotients D_i(f) scaled by sqrt(w/S) written as rows of 16 (parameters padded
- *             to 16) -- the operand layout of the matrix-core Gram
- *   gram      F = sum_rows a a^T with v_mfma_f64_16x16x4 (FP64 path) or v_mfma_f32_16x16x4 (mixed path),
- *             64 rows of 4 per instruction per wave, FP64 sums across waves and row chunks
+ *   fused     one block per (point, 64 bins): the stencil evaluations of every parameter projected on every detector,
+ *             the FP64 difference quotients scaled by sqrt(w/S) as operand rows (parameters padded to 16) in LDS, and
+ *             F = sum_rows a a^T of the block with v_mfma_f64_16x16x4
+ *   reduce    the blocks' partial matrices of every point, FP64, in a fixed order
+ *   FP32 Gram and bare derivatives: a stencil kernel (one lane per bin, point and row) writes the rows to memory,
+ *             v_mfma_f32_16x16x4 contracts them with FP64 sums across waves and row chunks
  *   invert    FP64 LU inverse per point (util.cpp:828-855) -> marginal sigmas
  *
  * Reference: src/fisher.cpp:81-145 (fisher_numerical), :148-557 (calculate_derivatives),
@@ -16,6 +17,7 @@
  */
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -35,6 +37,8 @@ typedef float gwh_f4 __attribute__((ext_vector_type(4)));
 #ifndef GWH_FUSED_WAVES
 #define GWH_FUSED_WAVES 8 /* waves per block of the fused kernel: GWH_FROWS / GWH_FUSED_WAVES operand rows each */
 #endif
+
+#define GWH_FUSED_SLOTS 3 /* operand rows a wave of the fused kernel can take */
 
 #include "gwh_basis.h"
 
@@ -141,10 +145,18 @@ static double host_dtoa(double ra, double dec, double gmst, int d1, int d2)
     return ((l1[0] - l2[0]) * e0 + (l1[1] - l2[1]) * e1 + (l1[2] - l2[2]) * e2) / GWH_C_SI;
 }
 
+/* Bits of one stencil evaluation.  The GWH_EV_SAME_* ones compare it with the evaluation that its wave of the fused
+ * kernel does just before it (of the previous row of the wave for the first evaluation of a row): the records are
+ * functions of the parameter sets, so parts that depend on fields with equal bits only are equal bit for bit. */
+#define GWH_EV_NO_TOF 1     /* order 4, +-2 eps: no time-of-flight phase (tc is shifted instead) */
+#define GWH_EV_SAME_CORE 2  /* masses and spins: amplitude without prefactor, phase without shifts, Euler angles */
+#define GWH_EV_SAME_TWIST 4 /* core and frame: the IMRPhenomPv2 twist-up factors */
+#define GWH_EV_SAME_PHASE 8 /* core, time and phase shift: the phase at the first detector */
+
 /* Stencil of one point: for every parameter i, S evaluations with weights c[i][s] (the difference
  * quotient including 1/eps and the log factor theta_i); instance parameter sets are appended to
- * `inst`, `no_tof` marks the order-4 +-2 eps evaluations that shift tc instead of using the time-of-flight
- * phase (fisher.cpp:433-453). */
+ * `inst`, their GWH_EV_* bits to `flags`: GWH_EV_NO_TOF marks the order-4 +-2 eps evaluations that shift tc instead
+ * of using the time-of-flight phase (fisher.cpp:433-453). */
 struct PointStencil {
     int S;
     double c[GWH_FROWS][GWH_MAXSTEN];
@@ -159,7 +171,7 @@ static double coordinate_step(double step, double v)
 }
 
 static int build_stencil(const gwh_params &p, int basis, int var, int nmod, int order, double step, int det,
-                         int ref_det, std::vector<gwh_params> &inst, std::vector<unsigned char> &no_tof,
+                         int ref_det, std::vector<gwh_params> &inst, std::vector<int> &flags,
                          PointStencil &ps)
 {
     int dim = basis_dim(basis) + nmod;
@@ -202,19 +214,115 @@ static int build_stencil(const gwh_params &p, int basis, int var, int nmod, int 
             bool two = (S == 4) && (s == 0 || s == 3);
             if (two && det != ref_det) q.tc -= host_dtoa(q.RA, q.DEC, q.gmst, ref_det, det);
             inst.push_back(q);
-            no_tof.push_back(two ? 1 : 0);
+            flags.push_back(two ? GWH_EV_NO_TOF : 0);
         }
     }
     return dim;
+}
+
+/* The GWH_EV_SAME_* bits of parameter set b evaluated right after a: which parts of its record (gwh_setup_kernel)
+ * follow from fields with equal bits.  Core: masses, spins, the chi_p given, the ringdown option, the ppE / gIMR terms
+ * (and for a theory's terms the distance, through its redshift).  IMRPhenomPv2 frame: core, phi_p, f_ref, inclination
+ * and phase.  Phase: core, t_c and the reference: for IMRPhenomD the phase and f_ref, for IMRPhenomPv2 phi_p and f_ref
+ * (its phase offset is the azimuth of J, in which inclination and phase do not enter). */
+static int shared_parts(const gwh_params &a, const gwh_params &b, bool pv2)
+{
+    auto eq = [](const void *x, const void *y, size_t n) { return memcmp(x, y, n) == 0; };
+#define GWH_SAME(F) eq(&a.F, &b.F, sizeof(a.F))
+    if (!(GWH_SAME(mass1) && GWH_SAME(mass2) && GWH_SAME(spin1) && GWH_SAME(spin2) && GWH_SAME(chip) &&
+          GWH_SAME(dep_postmerger) && GWH_SAME(ppe_nmod) && GWH_SAME(ppe_theory) && GWH_SAME(cosmology) &&
+          GWH_SAME(ppe_b) && GWH_SAME(ppe_beta) && GWH_SAME(gimr_dphi) && GWH_SAME(gimr_dsigma) &&
+          GWH_SAME(gimr_dbeta) && GWH_SAME(gimr_dalpha) && (!a.ppe_theory || GWH_SAME(DL))))
+        return 0;
+    int bits = GWH_EV_SAME_CORE;
+    const bool ref = GWH_SAME(f_ref) && GWH_SAME(phip);
+    if (ref && GWH_SAME(incl) && GWH_SAME(phiRef)) bits |= GWH_EV_SAME_TWIST;
+    if (ref && GWH_SAME(tc) && GWH_SAME(shift_time) && GWH_SAME(shift_phase) && (pv2 || GWH_SAME(phiRef)))
+        bits |= GWH_EV_SAME_PHASE;
+    return bits;
+}
+
+/* vector operations of one evaluation after another (the fused kernel's code, counted by hand; only the proportions
+ * matter): the projections always, the rest where it is not shared */
+static int evaluation_cost(const gwh_params *prev, const gwh_params &p, bool pv2, int ndet)
+{
+    const int same = prev ? shared_parts(*prev, p, pv2) : 0;
+    int c = 20 + 14 * ndet;
+    if (!(same & GWH_EV_SAME_CORE)) c += pv2 ? 330 : 150;
+    if (pv2 && !(same & GWH_EV_SAME_TWIST)) c += 130;
+    if (!(same & GWH_EV_SAME_PHASE))
+        c += 10 + 28 * ndet;
+    else if (memcmp(&prev->RA, &p.RA, sizeof(p.RA)) || memcmp(&prev->DEC, &p.DEC, sizeof(p.DEC)))
+        c += 28 * (ndet - 1); /* the arrival times; the first detector is their reference */
+    return c;
+}
+
+/* Rows of the waves of the fused kernel: rows in decreasing order of their cost alone, each to the wave that ends
+ * earliest with it, where what it shares with the wave's last row costs nothing.  inst: the dim * S parameter sets of
+ * one point.  The choice changes only the time: an operand's value does not depend on its wave. */
+static void assign_rows(const gwh_params *inst, int dim, int S, bool pv2, int ndet, int slots,
+                        int (*row)[GWH_FUSED_SLOTS])
+{
+    int load[GWH_FUSED_WAVES] = {0}, used[GWH_FUSED_WAVES] = {0}, order[GWH_FROWS], alone[GWH_FROWS];
+    auto cost = [&](int last, int i) { /* row i after row `last` (-1: first of its wave) */
+        int c = 0;
+        for (int s = 0; s < S; s++) {
+            const gwh_params *prev = s ? &inst[i * S + s - 1] : (last >= 0 ? &inst[last * S + S - 1] : nullptr);
+            c += evaluation_cost(prev, inst[i * S + s], pv2, ndet);
+        }
+        return c;
+    };
+    for (int i = 0; i < dim; i++) {
+        order[i] = i;
+        alone[i] = cost(-1, i);
+    }
+    std::stable_sort(order, order + dim, [&](int x, int y) { return alone[x] > alone[y]; });
+    for (int w = 0; w < GWH_FUSED_WAVES; w++)
+        for (int h = 0; h < GWH_FUSED_SLOTS; h++) row[w][h] = -1;
+    for (int n = 0; n < dim; n++) {
+        int best = -1, end = 0;
+        for (int w = 0; w < GWH_FUSED_WAVES; w++) {
+            if (used[w] >= slots) continue;
+            const int e = load[w] + cost(used[w] ? row[w][used[w] - 1] : -1, order[n]);
+            if (best < 0 || e < end) {
+                best = w;
+                end = e;
+            }
+        }
+        row[best][used[best]++] = order[n];
+        load[best] = end;
+    }
 }
 
 /* ------------------------------------------------------------------------- */
 /* device: stencil                                                            */
 /* ------------------------------------------------------------------------- */
 
+/* One stencil evaluation's share in the difference quotient of a detector, dr + i di += c h, with the fused
+ * multiply-adds written out: the operand rows and the bare derivatives round it alike wherever they are inlined (at
+ * the reference's step of 1e-8 the quotient magnifies a last-bit difference a millionfold). */
+#pragma clang fp contract(off)
+/* IMRPhenomD: h = A K e^{-i x} from cos x and sin x */
+__device__ __forceinline__ void add_response_d(double c, double A, double cs, double sn, const double *K, double &dr,
+                                               double &di)
+{
+    const double er = A * cs, ei = A * sn;
+    dr = fma(c, fma(er, K[0], ei * K[1]), dr);
+    di = fma(c, fma(er, K[1], -(ei * K[0])), di);
+}
+/* IMRPhenomPv2: h = A (P h+ + Q hx) e^{-i x} */
+__device__ __forceinline__ void add_response_pv2(double c, double A, double cs, double sn, const double *K, double hpr,
+                                                 double hpi, double hcr, double hci, double &dr, double &di)
+{
+    const double Gr = fma(K[0], hpr, K[1] * hcr), Gi = fma(K[0], hpi, K[1] * hci), cA = c * A;
+    dr = fma(cA, fma(Gr, cs, Gi * sn), dr);
+    di = fma(cA, fma(Gi, cs, -(Gr * sn)), di);
+}
+#pragma clang fp contract(fast)
+
 struct StencilArgs {
     const InstCoef *coef;        /* points x (dim*S [+1 central]) records */
-    const unsigned char *no_tof;
+    const int *flags;            /* points x records: GWH_EV_* bits of every stencil evaluation */
     const double *cw;            /* points x 16 x 4 stencil weights */
     int dim, S, per_point;       /* records per point */
     int d_first, d_count;        /* detectors of the event accumulated */
@@ -222,6 +330,7 @@ struct StencilArgs {
     double sa_sign;              /* +1 (order 2) or -1 (order 4): i d(phase) A sign of fisher.cpp:299-315 */
     double *raw;                 /* non-null: write the bare derivatives dim x N complex (one point, one
                                     detector) instead of weighted Gram operand rows */
+    int row[GWH_FUSED_WAVES][GWH_FUSED_SLOTS]; /* fused kernel: the operand rows of every wave, -1 none */
 };
 
 /* One lane per (bin, point, operand row): blockIdx.z is the row, and the S = 2 or 4 stencil evaluations of that
@@ -241,15 +350,15 @@ __global__ __launch_bounds__(GWH_TPB) void gwh_fisher_stencil_kernel(StencilArgs
     const double f = E.f[k];
     const InstCoef *C = a.coef + (size_t)pt * a.per_point;
     const double *cw = a.cw + (size_t)pt * GWH_FROWS * GWH_MAXSTEN;
-    const unsigned char *nt = a.no_tof + (size_t)pt * a.per_point;
+    const int *nt = a.flags + (size_t)pt * a.per_point;
     const size_t nrows = (size_t)a.d_count * N * 2;
     T *base = rows + (size_t)pt * nrows * GWH_FROWS;
     if (a.skyavg) {
         /* d h = dA + i sign d(phase) A_central (fisher.cpp:292-316); no detector projection */
         const InstCoef &Cc = C[a.dim * S];
         const BinPow bp = gwh_load_bin(E, k);
-        double Ac = 0, u, lx, ph;
-        if (f <= Cc.fcut) gwh_phenomd_fp64(Cc, f, bp, Ac, ph, u, lx);
+        double Ac = 0, u, ph;
+        if (f <= Cc.fcut) gwh_phenomd_fp64(Cc, f, bp, Ac, ph, u);
         double sw = sqrt(E.wS[(size_t)a.d_first * N + k]);
         double dA = 0, dP = 0;
         if (i < a.dim) {
@@ -257,7 +366,7 @@ __global__ __launch_bounds__(GWH_TPB) void gwh_fisher_stencil_kernel(StencilArgs
             for (int s = 0; s < S; s++) {
                 const InstCoef &Ci = C[i * S + s];
                 double A = 0, phi;
-                gwh_phenomd_fp64(Ci, f, bp, A, phi, u, lx);
+                gwh_phenomd_fp64(Ci, f, bp, A, phi, u);
                 if (!(f <= Ci.fcut)) A = 0;
                 dA += cw[i * GWH_MAXSTEN + s] * A;
                 dP += cw[i * GWH_MAXSTEN + s] * (-phi); /* construct_phase returns -(Psi - tc (f-fref) - phic) */
@@ -284,18 +393,16 @@ __global__ __launch_bounds__(GWH_TPB) void gwh_fisher_stencil_kernel(StencilArgs
             const InstCoef &Ci = C[i * S + s];
             if (!(f <= Ci.fcut)) continue; /* h = 0 above 0.2/M of this evaluation */
             const double c = cw[i * GWH_MAXSTEN + s];
-            const bool tof = !nt[i * S + s];
+            const bool tof = !(nt[i * S + s] & GWH_EV_NO_TOF);
             if (MODEL == GWH_IMRPHENOMD) {
-                double A, phi, u, lx;
-                gwh_phenomd_fp64(Ci, f, bp, A, phi, u, lx);
+                double A, phi, u;
+                gwh_phenomd_fp64(Ci, f, bp, A, phi, u);
                 for (int dd = 0; dd < GWH_MAXDET; dd++) {
                     if (dd >= a.d_count) break;
                     int d = a.d_first + dd;
                     double sn, cs;
                     gwh_sincos_table(phi + (tof ? Ci.det[d][3] : 0.0) * f, sn, cs);
-                    double er = A * cs, ei = -A * sn; /* A K e^{-i(phi + 2 pi dt f)} */
-                    dr[dd] += c * (er * Ci.det[d][0] - ei * Ci.det[d][1]);
-                    di[dd] += c * (er * Ci.det[d][1] + ei * Ci.det[d][0]);
+                    add_response_d(c, A, cs, sn, Ci.det[d], dr[dd], di[dd]);
                 }
             } else {
                 double A, Phi, hpr, hpi, hcr, hci;
@@ -303,12 +410,9 @@ __global__ __launch_bounds__(GWH_TPB) void gwh_fisher_stencil_kernel(StencilArgs
                 for (int dd = 0; dd < GWH_MAXDET; dd++) {
                     if (dd >= a.d_count) break;
                     int d = a.d_first + dd;
-                    double Gr = Ci.det[d][0] * hpr + Ci.det[d][1] * hcr;
-                    double Gi = Ci.det[d][0] * hpi + Ci.det[d][1] * hci;
                     double sn, cs;
                     gwh_sincos_table(Phi + (tof ? Ci.det[d][3] : 0.0) * f, sn, cs);
-                    dr[dd] += c * A * (Gr * cs + Gi * sn);
-                    di[dd] += c * A * (Gi * cs - Gr * sn);
+                    add_response_pv2(c, A, cs, sn, Ci.det[d], hpr, hpi, hcr, hci, dr[dd], di[dd]);
                 }
             }
         }
@@ -364,8 +468,7 @@ __host__ __device__ constexpr int gram_tri(int i) { return i * (i + 1) / 2; }
  * bins, 4 bins per MFMA (lane l supplies component l%16 of bin k0 + l/16 as both A and B operand; eight
  * MFMAs' operands are loaded first, 32 consecutive bins of each component).  Output: per block the FP64 partial
  * sums of the lower triangle of the dim parameters (gram_tri). */
-template <typename T>
-__global__ __launch_bounds__(GWH_TPB) void gwh_gram_kernel(const T *__restrict__ rows, int N, int nplanes,
+__global__ __launch_bounds__(GWH_TPB) void gwh_gram_kernel(const float *__restrict__ rows, int N, int nplanes,
                                                            int blk_per_plane, double *__restrict__ partial, int nblk,
                                                            int dim)
 {
@@ -373,44 +476,24 @@ __global__ __launch_bounds__(GWH_TPB) void gwh_gram_kernel(const T *__restrict__
     const int pt = blockIdx.y, blk = blockIdx.x;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int plane = blk / blk_per_plane;
-    const T *a = rows + ((size_t)pt * nplanes + plane) * GWH_FROWS * N + (size_t)(lane & 15) * N;
+    const float *a = rows + ((size_t)pt * nplanes + plane) * GWH_FROWS * N + (size_t)(lane & 15) * N;
     int r0 = (blk % blk_per_plane) * GWH_GRAM_ROWS + wv * (GWH_GRAM_ROWS / 4);
     int r1 = r0 + GWH_GRAM_ROWS / 4;
     if (r1 > N) r1 = N;
-    double out[4];
-    if (sizeof(T) == 8) {
-        gwh_d4 acc = {0, 0, 0, 0};
-        for (int r = r0; r < r1; r += 32) {
-            double x[8];
+    gwh_f4 acc = {0, 0, 0, 0};
+    for (int r = r0; r < r1; r += 32) {
+        float x[8];
 #pragma unroll
-            for (int u = 0; u < 8; u++) {
-                const int rr = r + 4 * u + (lane >> 4);
-                x[u] = (rr < r1) ? (double)a[rr] : 0.0;
-            }
-#pragma unroll
-            for (int u = 0; u < 8; u++) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(x[u], x[u], acc, 0, 0, 0);
+        for (int u = 0; u < 8; u++) {
+            const int rr = r + 4 * u + (lane >> 4);
+            x[u] = (rr < r1) ? a[rr] : 0.0f;
         }
-        for (int j = 0; j < 4; j++) out[j] = acc[j];
-    } else {
-        gwh_f4 acc = {0, 0, 0, 0};
-        for (int r = r0; r < r1; r += 32) {
-            float x[8];
 #pragma unroll
-            for (int u = 0; u < 8; u++) {
-                const int rr = r + 4 * u + (lane >> 4);
-                x[u] = (rr < r1) ? (float)a[rr] : 0.0f;
-            }
-#pragma unroll
-            for (int u = 0; u < 8; u++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[u], x[u], acc, 0, 0, 0);
-        }
-        for (int j = 0; j < 4; j++) out[j] = acc[j];
+        for (int u = 0; u < 8; u++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[u], x[u], acc, 0, 0, 0);
     }
-    /* result layout on gfx950 (checked on the device): column l % 16; row l / 16 + 4 j for the FP64
-     * instruction, 4 (l / 16) + j for the FP32 one */
-    for (int j = 0; j < 4; j++) {
-        int row = (sizeof(T) == 8) ? ((lane >> 4) + 4 * j) : (4 * (lane >> 4) + j);
-        lds[wv][row * 16 + (lane & 15)] = out[j];
-    }
+    /* result layout on gfx950 (checked on the device): column l % 16; row 4 (l / 16) + j for the FP32 instruction
+     * (l / 16 + 4 j for the FP64 one of the fused kernel) */
+    for (int j = 0; j < 4; j++) lds[wv][(4 * (lane >> 4) + j) * 16 + (lane & 15)] = acc[j];
     __syncthreads();
     const int ei = threadIdx.x >> 4, ej = threadIdx.x & 15;
     if (ei < dim && ej <= ei) {
@@ -427,23 +510,35 @@ __global__ __launch_bounds__(GWH_TPB) void gwh_gram_kernel(const T *__restrict__
  * covered most of them). */
 __device__ __forceinline__ int fused_col(int row, int col) { return (col + 2 * row) & (GWH_FUSED_BINS - 1); }
 
-/* The stencil and the FP64 Gram in one kernel: one block of GWH_FROWS waves per (point, chunk of 64 bins).  Wave
- * i evaluates operand row i -- the S stencil evaluations of component i, unrolled, projected on every detector and
- * weighted by sqrt(4 w / S_n) -- for the chunk's bins, one per lane, into LDS planes (detector, re/im) x row x bin
- * (zero for padding rows and bins past the grid); then the waves contract every plane on the FP64 matrix cores
- * (v_mfma_f64_16x16x4f64: 4 bins per instruction, lane l supplying component l % 16 of bin l / 16 as both
- * operands; wave w takes the (plane, 4-bin) slices w, w + 16, ...), and the block writes one 16x16 partial Gram,
- * summed over its waves in a fixed order.  The operand rows never leave the CU: the two-kernel path writes and
- * re-reads them through HBM (2 x 1.07 GB per 86-point pass of the 13-parameter IMRPhenomPv2 Fisher on the
- * 16225-bin 3-detector event). */
-template <int MODEL, int S, int WAVES>
+/* The stencil and the FP64 Gram in one kernel: one block of WAVES waves per (point, chunk of 64 bins).  Each wave
+ * evaluates the operand rows the host gave it (a.row) -- the S stencil evaluations of a component, unrolled,
+ * projected on every detector and weighted by sqrt(4 w / S_n) -- for the chunk's bins, one per lane, into LDS planes
+ * (detector, re/im) x row x bin (zero for padding rows and bins past the grid); then the waves contract every plane
+ * on the FP64 matrix cores (v_mfma_f64_16x16x4f64: 4 bins per instruction, lane l supplying component l % 16 of bin
+ * l / 16 as both operands; wave w takes the (plane, 4-bin) slices w, w + WAVES, ...), and the block writes one
+ * partial Gram, summed over its waves in a fixed order.  The operand rows never leave the CU.
+ *
+ * Most parameters of a basis leave most of the waveform as it is: sky position, polarisation, inclination, phase,
+ * time and distance move neither the amplitude's shape nor the phase's, and polarisation and distance not even the
+ * phase in a detector.  What an evaluation shares with the one its wave did before (GWH_EV_SAME_*, equal bits by
+ * construction) is kept in registers instead of computed again, and rows that share are given to the same wave:
+ * 12 instead of 22 evaluations of the waveform for the 11 IMRPhenomD parameters (4 rows change it, the other 7 lie
+ * in 4 waves), 13 instead of 26 for the 13 of IMRPhenomPv2.  The arithmetic of an operand does not depend on which wave does it or after
+ * what.  Bound by the vector ALU; per launch, every evaluation in full -> shared, over the live chunks only:
+ * IMRPhenomPv2, 128 points x 16225 bins x 3 detectors 838 -> 307 us, IMRPhenomD, 12 points x 65539 bins x 3 418 -> 238
+ * us; the 7-parameter sky-averaged matrix of one point on 4017 bins, which went through operand rows in HBM, 36 ->
+ * 8.5 us.
+ *
+ * SKY: the sky-averaged IMRPhenomD basis, d h = dA + i sign d(phase) A_central (fisher.cpp:292-316) in planes
+ * (dA, d(phase) A) of one detector row. */
+template <int MODEL, int S, int WAVES, int SLOTS, bool SKY>
 __global__ __launch_bounds__(WAVES * 64) void gwh_fisher_fused_kernel(StencilArgs a,
                                                                      const EventDesc *__restrict__ events,
                                                                      int event0, double *__restrict__ partial, int nbc)
 {
     __shared__ double lds[2 * GWH_MAXDET][GWH_FROWS][GWH_FUSED_BINS]; /* 64 KiB */
     const int pt = blockIdx.y, bc = blockIdx.x;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const EventDesc &E = events[event0];
     const int N = E.N;
     const int k0 = bc * GWH_FUSED_BINS + lane;
@@ -451,64 +546,91 @@ __global__ __launch_bounds__(WAVES * 64) void gwh_fisher_fused_kernel(StencilArg
     const int k = in ? k0 : N - 1;
     const InstCoef *C = a.coef + (size_t)pt * a.per_point;
     const double *cw = a.cw + (size_t)pt * GWH_FROWS * GWH_MAXSTEN;
-    const unsigned char *nt = a.no_tof + (size_t)pt * a.per_point;
-    /* wave wv evaluates rows wv, wv + WAVES, ... (unrolled: no loop for the compiler to hoist values across) */
+    const int *fl = a.flags + (size_t)pt * a.per_point;
+    const int nplanes = 2 * a.d_count;
+    for (int e = threadIdx.x; e < nplanes * (GWH_FROWS - a.dim) * GWH_FUSED_BINS; e += WAVES * 64) {
+        const int r = e / GWH_FUSED_BINS;
+        lds[r % nplanes][a.dim + r / nplanes][e % GWH_FUSED_BINS] = 0.0; /* padding rows */
+    }
+    double f = 0, sw[GWH_MAXDET] = {0, 0, 0, 0}, Ac = 0;
+    BinPow bp = {0, 0, 0, 0, 0};
+    /* the previous evaluation of this wave */
+    double a0 = 0, psi = 0, u = 0, Phi = 0, hpr = 0, hpi = 0, hcr = 0, hci = 0;
+    Pv2Angles ang = {0, 0, 0, 0};
+    double zc[GWH_MAXDET] = {0, 0, 0, 0}, zs[GWH_MAXDET] = {0, 0, 0, 0}, kz[GWH_MAXDET] = {0, 0, 0, 0};
+    if (a.row[wv][0] >= 0) {
+        f = gwh_g(E.f)[k];
+        bp = gwh_load_bin(E, k);
 #pragma unroll
-    for (int h = 0; h < GWH_FROWS / WAVES; h++) {
-        const int i = wv + WAVES * h;
+        for (int dd = 0; dd < (SKY ? 1 : GWH_MAXDET); dd++)
+            if (dd < a.d_count) sw[dd] = in ? sqrt(gwh_g(E.wS)[(size_t)(a.d_first + dd) * N + k]) : 0.0;
+        if (SKY) {
+            const InstCoef &Cc = C[a.dim * S];
+            double ph;
+            if (f <= Cc.fcut) gwh_phenomd_fp64(Cc, f, bp, Ac, ph, u);
+        }
+    }
+    /* unrolled: no loop for the compiler to hoist values across */
+#pragma unroll
+    for (int h = 0; h < SLOTS; h++) {
+        const int i = a.row[wv][h]; /* uniform over the wave */
+        if (i < 0) break;
         double dr[GWH_MAXDET] = {0, 0, 0, 0}, di[GWH_MAXDET] = {0, 0, 0, 0};
-        if (i < a.dim) { /* uniform over the wave */
-            const double f = gwh_g(E.f)[k];
-            const BinPow bp = gwh_load_bin(E, k);
 #pragma unroll
-            for (int s = 0; s < S; s++) {
-                const InstCoef &Ci = C[i * S + s];
-                if (!(f <= Ci.fcut)) continue; /* h = 0 above 0.2/M of this evaluation */
-                const double c = cw[i * GWH_MAXSTEN + s];
-                const bool tof = !nt[i * S + s];
-                if (MODEL == GWH_IMRPHENOMD) {
-                    double A, phi, u, lx;
-                    gwh_phenomd_fp64(Ci, f, bp, A, phi, u, lx);
-                    for (int dd = 0; dd < GWH_MAXDET; dd++) {
-                        if (dd >= a.d_count) break;
-                        const int d = a.d_first + dd;
-                        double sn, cs;
-                        gwh_sincos_table(phi + (tof ? Ci.det[d][3] : 0.0) * f, sn, cs);
-                        const double er = A * cs, ei = -A * sn; /* A K e^{-i(phi + 2 pi dt f)} */
-                        dr[dd] += c * (er * Ci.det[d][0] - ei * Ci.det[d][1]);
-                        di[dd] += c * (er * Ci.det[d][1] + ei * Ci.det[d][0]);
-                    }
-                } else {
-                    double A, Phi, hpr, hpi, hcr, hci;
-                    gwh_pv2_fp64(Ci, f, bp, A, Phi, hpr, hpi, hcr, hci);
-                    for (int dd = 0; dd < GWH_MAXDET; dd++) {
-                        if (dd >= a.d_count) break;
-                        const int d = a.d_first + dd;
-                        const double Gr = Ci.det[d][0] * hpr + Ci.det[d][1] * hcr;
-                        const double Gi = Ci.det[d][0] * hpi + Ci.det[d][1] * hci;
-                        double sn, cs;
-                        gwh_sincos_table(Phi + (tof ? Ci.det[d][3] : 0.0) * f, sn, cs);
-                        dr[dd] += c * A * (Gr * cs + Gi * sn);
-                        di[dd] += c * A * (Gi * cs - Gr * sn);
-                    }
-                }
+        for (int s = 0; s < S; s++) {
+            const InstCoef &Ci = C[i * S + s];
+            const int same = fl[i * S + s];
+            const double c = cw[i * GWH_MAXSTEN + s];
+            const bool live = f <= Ci.fcut; /* h = 0 above 0.2/M of this evaluation */
+            if (SKY) {
+                /* the phase counts up to the cutoff of the central amplitude */
+                if (!__ballot(!(f > Ci.fcut) || !(f > C[a.dim * S].fcut))) continue;
+                if (!(same & GWH_EV_SAME_CORE)) gwh_phenomd_core(Ci, f, bp, a0, psi, u);
+                dr[0] += c * (live ? Ci.amp_pref * a0 : 0.0);
+                di[0] += c * -gwh_phase_shift(Ci, f, psi); /* construct_phase returns -(Psi - tc (f-fref) - phic) */
+                continue;
             }
+            if (!__ballot(live)) continue;
+            if (!(same & GWH_EV_SAME_CORE)) {
+                gwh_phenomd_core(Ci, f, bp, a0, psi, u);
+                if (MODEL == GWH_IMRPHENOMPV2) ang = gwh_pv2_angles(Ci, u, bp);
+            }
+            if (MODEL == GWH_IMRPHENOMPV2 && !(same & GWH_EV_SAME_TWIST)) gwh_pv2_twist(Ci, ang, hpr, hpi, hcr, hci);
+            if (!(same & GWH_EV_SAME_PHASE)) {
+                Phi = gwh_phase_shift(Ci, f, psi);
+                if (MODEL == GWH_IMRPHENOMPV2) Phi = gwh_pv2_phase(Ci, f, Phi, ang);
+            }
+            const double A = live ? Ci.amp_pref * a0 : 0.0;
+#pragma unroll
             for (int dd = 0; dd < GWH_MAXDET; dd++) {
                 if (dd >= a.d_count) break;
-                const double sw = in ? sqrt(gwh_g(E.wS)[(size_t)(a.d_first + dd) * N + k]) : 0.0;
-                dr[dd] *= sw;
-                di[dd] *= sw;
+                const int d = a.d_first + dd;
+                const double kd = (same & GWH_EV_NO_TOF) ? 0.0 : Ci.det[d][3];
+                if (!(same & GWH_EV_SAME_PHASE) || __double_as_longlong(kd) != __double_as_longlong(kz[dd])) {
+                    gwh_sincos_table(Phi + kd * f, zs[dd], zc[dd]);
+                    kz[dd] = kd;
+                }
+                if (MODEL == GWH_IMRPHENOMD)
+                    add_response_d(c, A, zc[dd], zs[dd], Ci.det[d], dr[dd], di[dd]);
+                else
+                    add_response_pv2(c, A, zc[dd], zs[dd], Ci.det[d], hpr, hpi, hcr, hci, dr[dd], di[dd]);
             }
         }
-        for (int dd = 0; dd < GWH_MAXDET; dd++) {
-            if (dd >= a.d_count) break;
-            lds[2 * dd][i][fused_col(i, lane)] = dr[dd];
-            lds[2 * dd + 1][i][fused_col(i, lane)] = di[dd];
+        if (SKY) {
+            lds[0][i][fused_col(i, lane)] = dr[0] * sw[0];
+            lds[1][i][fused_col(i, lane)] = a.sa_sign * di[0] * Ac * sw[0];
+        } else {
+#pragma unroll
+            for (int dd = 0; dd < GWH_MAXDET; dd++) {
+                if (dd >= a.d_count) break;
+                lds[2 * dd][i][fused_col(i, lane)] = dr[dd] * sw[dd];
+                lds[2 * dd + 1][i][fused_col(i, lane)] = di[dd] * sw[dd];
+            }
         }
     }
     __syncthreads();
     gwh_d4 acc = {0, 0, 0, 0};
-    const int nslice = 2 * a.d_count * (GWH_FUSED_BINS / 4);
+    const int nslice = nplanes * (GWH_FUSED_BINS / 4);
     for (int t = wv; t < nslice; t += WAVES) {
         const int pl = t / (GWH_FUSED_BINS / 4), q = t % (GWH_FUSED_BINS / 4);
         const int row = lane & 15;
@@ -526,6 +648,31 @@ __global__ __launch_bounds__(WAVES * 64) void gwh_fisher_fused_kernel(StencilArg
         for (int w = 1; w < WAVES; w++) sum += part[w][threadIdx.x];
         partial[((size_t)pt * nbc + bc) * gram_tri(a.dim) + gram_tri(ei) + ej] = sum;
     }
+}
+
+/* the fused kernel of a model, stencil size and basis; grid: chunks of 64 bins x points.  Order 2 gives a wave up to
+ * three rows; order 4 (single points only) two, which keeps its unrolled code within the instruction cache. */
+static void launch_fused(bool pv2, bool sky, dim3 g, hipStream_t st, const StencilArgs &a, const EventDesc *evp,
+                         int event, double *partial)
+{
+    constexpr int W = GWH_FUSED_WAVES;
+    const dim3 b(W * 64);
+    const int nbc = (int)g.x;
+#define GWH_FUSED(M, S, SLOTS, SKY)                                                                                 \
+    hipLaunchKernelGGL((gwh_fisher_fused_kernel<M, S, W, SLOTS, SKY>), g, b, 0, st, a, evp, event, partial, nbc)
+    if (sky && a.S == 4)
+        GWH_FUSED(GWH_IMRPHENOMD, 4, 2, true);
+    else if (sky)
+        GWH_FUSED(GWH_IMRPHENOMD, 2, 2, true);
+    else if (!pv2 && a.S == 4)
+        GWH_FUSED(GWH_IMRPHENOMD, 4, 2, false);
+    else if (!pv2)
+        GWH_FUSED(GWH_IMRPHENOMD, 2, GWH_FUSED_SLOTS, false);
+    else if (a.S == 4)
+        GWH_FUSED(GWH_IMRPHENOMPV2, 4, 2, false);
+    else
+        GWH_FUSED(GWH_IMRPHENOMPV2, 2, GWH_FUSED_SLOTS, false);
+#undef GWH_FUSED
 }
 
 /* Fixed-order FP64 sum of the Gram partials: one block of 1024 threads per (point, 16 elements of the packed lower
@@ -684,10 +831,10 @@ static int fisher_run(int event, int model, int basis, int precision, const gwh_
     int per_point = dim * S + (sky ? 1 : 0);
     const int N = ev.N;
     const size_t nrows = (size_t)(sky ? 1 : d_count) * N * 2;
-    const size_t row_bytes = GWH_FROWS * ((precision == GWH_FISHER_GRAM_FP32) ? 4 : 8);
-    /* the FP64 Gram of a network Fisher runs fused with the stencil (no operand rows in HBM); the sky-averaged
-       basis, the FP32 Gram and the bare derivatives go through operand rows */
-    const bool fused = !raw && !sky && precision != GWH_FISHER_GRAM_FP32;
+    const size_t row_bytes = GWH_FROWS * (raw ? 8 : 4); /* operand rows: FP32 Gram, bare derivatives */
+    /* the FP64 Gram runs fused with the stencil (no operand rows in HBM); the FP32 Gram and the bare derivatives go
+       through operand rows */
+    const bool fused = !raw && precision != GWH_FISHER_GRAM_FP32;
     /* points per pass: bounded operand buffer (F.max_operand, 1 GiB unless a caller's budget says less); fused,
        the partial Gram matrices take its place */
     size_t per_pt_bytes = nrows * row_bytes;
@@ -705,22 +852,34 @@ static int fisher_run(int event, int model, int basis, int precision, const gwh_
     if ((rc = F.gram.ensure((size_t)chunk * part_bytes)) != GWH_OK) return rc;
     if ((rc = F.out.ensure((size_t)n * dim * dim * 8)) != GWH_OK) return rc;
     std::vector<gwh_params> inst;
-    std::vector<unsigned char> no_tof;
+    std::vector<int> flags; /* GWH_EV_* bits of every record */
     std::vector<double> cw;
+    StencilArgs a;
+    const int slots = (S == 4 || sky) ? 2 : GWH_FUSED_SLOTS; /* as launch_fused */
     int slot = 0;
     for (int p0 = 0; p0 < n; p0 += chunk, slot ^= 1) {
         int np = std::min(chunk, n - p0);
         inst.clear();
-        no_tof.clear();
+        flags.clear();
         cw.assign((size_t)np * GWH_FROWS * GWH_MAXSTEN, 0.0);
         inst.reserve((size_t)np * per_point);
         for (int q = 0; q < np; q++) {
             PointStencil ps;
             build_stencil(params[p0 + q], basis, gwh_ppe_variant(model), nmod, order, eps, det_for_tof, ref_det,
-                          inst, no_tof, ps);
+                          inst, flags, ps);
             if (sky) {
                 inst.push_back(params[p0 + q]); /* central amplitude: the caller's parameters */
-                no_tof.push_back(0);
+                flags.push_back(0);
+            }
+            if (fused) {
+                const gwh_params *rec = &inst[(size_t)q * per_point];
+                if (p0 == 0 && q == 0) assign_rows(rec, dim, S, pv2, sky ? 1 : d_count, slots, a.row);
+                for (int w = 0; w < GWH_FUSED_WAVES; w++) {
+                    int prev = -1;
+                    for (int h = 0; h < slots && a.row[w][h] >= 0; h++)
+                        for (int e = a.row[w][h] * S; e < (a.row[w][h] + 1) * S; prev = e++)
+                            if (prev >= 0) flags[(size_t)q * per_point + e] |= shared_parts(rec[prev], rec[e], pv2);
+                }
             }
             for (int i = 0; i < GWH_FROWS; i++)
                 for (int s = 0; s < GWH_MAXSTEN; s++) cw[((size_t)q * GWH_FROWS + i) * GWH_MAXSTEN + s] = ps.c[i][s];
@@ -728,9 +887,10 @@ static int fisher_run(int event, int model, int basis, int precision, const gwh_
         int ni = (int)inst.size();
         if ((rc = F.params.ensure((size_t)ni * sizeof(gwh_params))) != GWH_OK) return rc;
         if ((rc = F.coef.ensure((size_t)ni * sizeof(InstCoef))) != GWH_OK) return rc;
-        if ((rc = F.misc.ensure(cw.size() * 8 + no_tof.size() + 256)) != GWH_OK) return rc;
+        if ((rc = F.misc.ensure(cw.size() * 8 + flags.size() * 4 + 256)) != GWH_OK) return rc;
         /* stage the pass in pinned memory (asynchronous copies; the device buffers are reused in stream order) */
-        const size_t rec_bytes = (size_t)ni * sizeof(gwh_params), stage_bytes = rec_bytes + cw.size() * 8 + no_tof.size();
+        const size_t rec_bytes = (size_t)ni * sizeof(gwh_params), misc_bytes = cw.size() * 8 + flags.size() * 4,
+                     stage_bytes = rec_bytes + misc_bytes;
         if (F.stage_done[slot]) GWH_HIP(hipEventSynchronize(F.stage_done[slot])); /* its last copy has run */
         else GWH_HIP(hipEventCreateWithFlags(&F.stage_done[slot], hipEventDisableTiming));
         if (F.stage_cap[slot] < stage_bytes) {
@@ -743,18 +903,17 @@ static int fisher_run(int event, int model, int basis, int precision, const gwh_
         char *st = (char *)F.stage[slot];
         memcpy(st, inst.data(), rec_bytes);
         memcpy(st + rec_bytes, cw.data(), cw.size() * 8);
-        memcpy(st + rec_bytes + cw.size() * 8, no_tof.data(), no_tof.size());
+        memcpy(st + rec_bytes + cw.size() * 8, flags.data(), flags.size() * 4);
         GWH_HIP(hipMemcpyAsync(F.params.p, st, rec_bytes, hipMemcpyHostToDevice, F.stream));
         char *misc = (char *)F.misc.p;
-        GWH_HIP(hipMemcpyAsync(misc, st + rec_bytes, cw.size() * 8 + no_tof.size(), hipMemcpyHostToDevice, F.stream));
+        GWH_HIP(hipMemcpyAsync(misc, st + rec_bytes, misc_bytes, hipMemcpyHostToDevice, F.stream));
         GWH_HIP(hipEventRecord(F.stage_done[slot], F.stream));
         if ((rc = gwh_setup_launch(nullptr, event, model, F.params.as<const gwh_params>(), ni, F.coef.as<InstCoef>(),
                                    F.stream)) != GWH_OK)
             return rc;
-        StencilArgs a;
         a.coef = F.coef.as<const InstCoef>();
         a.cw = (const double *)misc;
-        a.no_tof = (const unsigned char *)(misc + cw.size() * 8);
+        a.flags = (const int *)(misc + cw.size() * 8);
         a.dim = dim;
         a.S = S;
         a.per_point = per_point;
@@ -777,37 +936,28 @@ static int fisher_run(int event, int model, int basis, int precision, const gwh_
             GWH_HIP(hipStreamSynchronize(F.stream));
             return GWH_OK;
         }
+        int nb = nblk; /* partial Gram matrices of a point */
         if (fused) {
-            const dim3 gf(nblk, np), bf(GWH_FUSED_WAVES * 64);
-            if (!pv2) {
-                if (S == 4)
-                    hipLaunchKernelGGL((gwh_fisher_fused_kernel<GWH_IMRPHENOMD, 4, GWH_FUSED_WAVES>), gf, bf, 0, F.stream, a, evp, event,
-                                       F.gram.as<double>(), nblk);
-                else
-                    hipLaunchKernelGGL((gwh_fisher_fused_kernel<GWH_IMRPHENOMD, 2, GWH_FUSED_WAVES>), gf, bf, 0, F.stream, a, evp, event,
-                                       F.gram.as<double>(), nblk);
-            } else {
-                if (S == 4)
-                    hipLaunchKernelGGL((gwh_fisher_fused_kernel<GWH_IMRPHENOMPV2, 4, GWH_FUSED_WAVES>), gf, bf, 0, F.stream, a, evp,
-                                       event, F.gram.as<double>(), nblk);
-                else
-                    hipLaunchKernelGGL((gwh_fisher_fused_kernel<GWH_IMRPHENOMPV2, 2, GWH_FUSED_WAVES>), gf, bf, 0, F.stream, a, evp,
-                                       event, F.gram.as<double>(), nblk);
+            /* only the 64-bin chunks that begin at or below some record's cutoff 0.2/M hold anything (a margin covers
+               the rounding of the device's own cutoff, which decides bin by bin): 77 of 254 chunks for 65 solar masses
+               on 20-2048 Hz */
+            double fcut = 0;
+            for (const gwh_params &p : inst) {
+                const double c = .2 / (p.mass1 * GWH_MSOL_SEC + p.mass2 * GWH_MSOL_SEC);
+                fcut = (c <= fcut) ? fcut : c; /* NaN: every chunk */
             }
-        } else if (precision != GWH_FISHER_GRAM_FP32) {
-            launch_stencil<double>(pv2, g, F.stream, a, evp, event, F.deriv.as<double>());
-            GWH_HIP(hipGetLastError());
-            hipLaunchKernelGGL(gwh_gram_kernel<double>, dim3(nblk, np), dim3(GWH_TPB), 0, F.stream,
-                               F.deriv.as<const double>(), N, nplanes, blk_per_plane, F.gram.as<double>(), nblk, dim);
+            const std::vector<double> &cf = *ev.chunk_fmin;
+            while (nb > 1 && cf[nb - 1] > fcut * (1 + 1e-9)) nb--;
+            launch_fused(pv2, sky, dim3(nb, np), F.stream, a, evp, event, F.gram.as<double>());
         } else {
             launch_stencil<float>(pv2, g, F.stream, a, evp, event, F.deriv.as<float>());
             GWH_HIP(hipGetLastError());
-            hipLaunchKernelGGL(gwh_gram_kernel<float>, dim3(nblk, np), dim3(GWH_TPB), 0, F.stream,
-                               F.deriv.as<const float>(), N, nplanes, blk_per_plane, F.gram.as<double>(), nblk, dim);
+            hipLaunchKernelGGL(gwh_gram_kernel, dim3(nblk, np), dim3(GWH_TPB), 0, F.stream, F.deriv.as<const float>(), N,
+                               nplanes, blk_per_plane, F.gram.as<double>(), nblk, dim);
         }
         GWH_HIP(hipGetLastError());
         hipLaunchKernelGGL(gwh_gram_reduce_kernel, dim3(np, (gram_tri(dim) + 15) / 16), dim3(1024), 0, F.stream, F.gram.as<const double>(),
-                           nblk, dim, scale, F.out.as<double>() + (size_t)p0 * dim * dim);
+                           nb, dim, scale, F.out.as<double>() + (size_t)p0 * dim * dim);
         GWH_HIP(hipGetLastError());
     }
     if (sigma) {
@@ -868,7 +1018,7 @@ size_t gwh_fisher_batch_bytes(int event, int model, int basis, int precision, co
     const bool sky = (basis == GWH_BASIS_PHENOMD_SKYAVG);
     const size_t per_point = (size_t)dim * 2 + (sky ? 1 : 0);
     const size_t nrows = (size_t)(sky ? 1 : ev.D) * ev.N * 2;
-    const bool fused = !sky && precision != GWH_FISHER_GRAM_FP32;
+    const bool fused = precision != GWH_FISHER_GRAM_FP32;
     const size_t nblk = fused ? (ev.N + GWH_FUSED_BINS - 1) / GWH_FUSED_BINS
                               : (nrows / ev.N) * ((ev.N + GWH_GRAM_ROWS - 1) / GWH_GRAM_ROWS);
     const size_t part_bytes = nblk * gram_tri(dim) * 8;
@@ -883,7 +1033,7 @@ size_t gwh_fisher_batch_bytes(int event, int model, int basis, int precision, co
            (want_sigma ? gwh_grown_capacity((size_t)n * dim * 8, F.sig.cap) : F.sig.cap) +
            gwh_grown_capacity(ni * sizeof(gwh_params), F.params.cap) +
            gwh_grown_capacity(ni * sizeof(InstCoef), F.coef.cap) +
-           gwh_grown_capacity(chunk * GWH_FROWS * GWH_MAXSTEN * 8 + ni + 256, F.misc.cap) + F.raw.cap;
+           gwh_grown_capacity(chunk * GWH_FROWS * GWH_MAXSTEN * 8 + ni * 4 + 256, F.misc.cap) + F.raw.cap;
 }
 
 extern "C" {

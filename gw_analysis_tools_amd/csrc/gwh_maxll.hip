@@ -75,8 +75,8 @@ __global__ __launch_bounds__(GWH_MX_TPB) void gwh_maxll_fill_kernel(const EventD
         if (f <= C.fcut) {
             const BinPow bp = gwh_load_bin(E, k);
             if (MODEL == GWH_IMRPHENOMD) {
-                double A, phi, u, lx;
-                gwh_phenomd_fp64(C, f, bp, A, phi, u, lx);
+                double A, phi, u;
+                gwh_phenomd_fp64(C, f, bp, A, phi, u);
                 double s, c;
                 gwh_sincos_table(phi, s, c);
                 hp = make_double2(A * c * C.wf_a, -A * s * C.wf_a); /* h+ = A e^{-i phi} (1 + cos^2 i) / 2 */

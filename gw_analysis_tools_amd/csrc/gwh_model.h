@@ -1120,8 +1120,6 @@ __device__ __forceinline__ double gwh_setup_knot(double fRD, int j)
 /* per-bin FP64 evaluation                                                    */
 /* ------------------------------------------------------------------------- */
 
-/* IMRPhenomD amplitude A(f) and phase phi(f) = Psi(f) - tc_total (f - f_ref) - phic
- * (IMRPhenomD.cpp:471-501); caller guarantees 0 < f <= fcut. */
 /* gIMR inspiral phase terms at one bin from 1/v, v = (pi M f)^(1/3) */
 __device__ __forceinline__ double gwh_gimr_bin(const InstCoef &C, double iv)
 {
@@ -1138,13 +1136,15 @@ __device__ __forceinline__ double gwh_ppe_bin(const InstCoef &C, double lf)
     return t;
 }
 
+/* The part of IMRPhenomD that depends on the intrinsic parameters only: the amplitude a(f) without its prefactor
+ * (distance, chirp mass) and the phase psi(f) without the time and phase shift; u = (M f)^{1/3}. */
 template <bool FP32_EXP = false>
-__device__ __forceinline__ void gwh_phenomd_fp64(const InstCoef &C, double f, const BinPow &bp, double &A, double &phi,
-                                                 double &u_out, double &lx_out, const double2 *tab = gwh_turn_table,
+__device__ __forceinline__ void gwh_phenomd_core(const InstCoef &C, double f, const BinPow &bp, double &a, double &psi,
+                                                 double &u, const double2 *tab = gwh_turn_table,
                                                  const double *etab = gwh_exp2_table)
 {
     double Mf = C.M * f;
-    double u = C.M13 * bp.f13;      /* (Mf)^{1/3} */
+    u = C.M13 * bp.f13;              /* (Mf)^{1/3} */
     double inv76 = C.Mm76 * bp.fm76; /* (Mf)^{-7/6} */
     double ar;
     if (f < C.f1) {
@@ -1158,12 +1158,10 @@ __device__ __forceinline__ void gwh_phenomd_fp64(const InstCoef &C, double f, co
     } else {
         ar = C.delta[0] + Mf * (C.delta[1] + Mf * (C.delta[2] + Mf * (C.delta[3] + Mf * C.delta[4])));
     }
-    A = C.amp_pref * ar * inv76;
-    double psi;
-    double lx = 0;
+    a = ar * inv76;
     if (f < C.f1p) {
         double v = u * 1.4645918875615231; /* pi^{1/3} */
-        lx = C.lgPiM + bp.lf;             /* log(pi M f) */
+        double lx = C.lgPiM + bp.lf;       /* log(pi M f) */
         double c5 = C.c8 + lx * C.c9;
         double c6 = C.c10 - C.c11 * lx;
         double v2 = v * v;
@@ -1179,20 +1177,34 @@ __device__ __forceinline__ void gwh_phenomd_fp64(const InstCoef &C, double f, co
         psi = C.beta[0] + C.beta[1] * Mf + C.beta[2] * (C.lgM + bp.lf) - C.beta[3] * rcp_newton(Mf * Mf * Mf);
     }
     if (C.ppe_n > 0 && (C.ppe_imr || f < C.f1p)) psi += gwh_ppe_bin(C, bp.lf);
-    phi = psi - (C.tc_total * (f - C.f_ref) + C.phic);
-    u_out = u;
-    lx_out = lx;
 }
 
-/* IMRPhenomPv2 twist-up at one bin (IMRPhenomP.cpp:290-361): returns the common amplitude
- * (already including the 1/2), the total phase and the complex h+ / hx twist-up factors. */
-__device__ __forceinline__ void gwh_pv2_fp64(const InstCoef &C, double f, const BinPow &bp, double &A, double &Phi,
-                                             double &hpr, double &hpi, double &hcr, double &hci,
-                                             const double2 *tab = gwh_turn_table, const double *etab = gwh_exp2_table)
+/* psi(f) with the instance's time and phase shift */
+__device__ __forceinline__ double gwh_phase_shift(const InstCoef &C, double f, double psi)
 {
-    double u, lx;
-    gwh_phenomd_fp64(C, f, bp, A, Phi, u, lx, tab, etab);
-    /* gwh_phenomd_fp64 already applied -tc (f - f_ref) - phic; Pv2 adds 2 eps and the t_c correction */
+    return psi - (C.tc_total * (f - C.f_ref) + C.phic);
+}
+
+/* IMRPhenomD amplitude A(f) and phase phi(f) = Psi(f) - tc_total (f - f_ref) - phic
+ * (IMRPhenomD.cpp:471-501); caller guarantees 0 < f <= fcut. */
+template <bool FP32_EXP = false>
+__device__ __forceinline__ void gwh_phenomd_fp64(const InstCoef &C, double f, const BinPow &bp, double &A, double &phi,
+                                                 double &u, const double2 *tab = gwh_turn_table,
+                                                 const double *etab = gwh_exp2_table)
+{
+    double a, psi;
+    gwh_phenomd_core<FP32_EXP>(C, f, bp, a, psi, u, tab, etab);
+    A = C.amp_pref * a;
+    phi = gwh_phase_shift(C, f, psi);
+}
+
+/* What the IMRPhenomPv2 twist-up (IMRPhenomP.cpp:290-361) takes from the intrinsic parameters at one bin: cosine and
+ * sine of half the opening angle, and the Euler angles without their offsets. */
+struct Pv2Angles {
+    double cbh, sbh, alpha, eps;
+};
+__device__ __forceinline__ Pv2Angles gwh_pv2_angles(const InstCoef &C, double u, const BinPow &bp)
+{
     double v = u * 1.4645918875615231;
     double logw = C.lgPiM + bp.lf; /* log(pi M f) */
     double x = v * v;
@@ -1201,13 +1213,23 @@ __device__ __forceinline__ void gwh_pv2_fp64(const InstCoef &C, double f, const 
     double cb = rsqrt_seeded(1.0 + s * s);
     /* cos and sin of beta/2: 1 - cos b = s^2 cos^2 b / (1 + cos b), so sin(b/2) = |s| cos b / (2 cos(b/2)), free of
        the cancellation of sqrt((1 - cos b) / 2) for small s and one square root fewer */
-    double cbh = sqrt((1.0 + cb) / 2.0), sbh = fabs(s) * cb * (0.5 * rcp_newton(cbh));
+    Pv2Angles P;
+    P.cbh = sqrt((1.0 + cb) / 2.0);
+    P.sbh = fabs(s) * cb * (0.5 * rcp_newton(P.cbh));
+    P.alpha = gwh_euler_eval(C.a_c, v, logw);
+    P.eps = gwh_euler_eval(C.e_c, v, logw);
+    return P;
+}
+
+/* the complex h+ / hx twist-up factors */
+__device__ __forceinline__ void gwh_pv2_twist(const InstCoef &C, const Pv2Angles &P, double &hpr, double &hpi,
+                                              double &hcr, double &hci, const double2 *tab = gwh_turn_table)
+{
+    const double cbh = P.cbh, sbh = P.sbh;
     double c2 = cbh * cbh, s2 = sbh * sbh, c3 = c2 * cbh, s3 = s2 * sbh;
     double d2[5] = {s3 * sbh, 2 * cbh * s3, GWH_SQRT_6 * s2 * c2, 2 * c3 * sbh, c3 * cbh};
-    double alpha = gwh_euler_eval(C.a_c, v, logw) + C.alpha_add;
-    double eps = gwh_euler_eval(C.e_c, v, logw) + C.eps_add;
     double sa, ca;
-    gwh_sincos_tab(alpha, sa, ca, tab);
+    gwh_sincos_tab(P.alpha + C.alpha_add, sa, ca, tab);
     /* e^{i m alpha}, m=-2..2 */
     double er[5], ei[5];
     er[2] = 1;
@@ -1232,7 +1254,25 @@ __device__ __forceinline__ void gwh_pv2_fp64(const InstCoef &C, double f, const 
         hcr -= t2i - tmi;
         hci += t2r - tmr;
     }
-    Phi = Phi + 2. * eps + C.t_corr_2pi * f;
+}
+
+/* phase of IMRPhenomPv2 from the shifted IMRPhenomD phase: 2 epsilon and the t_c correction */
+__device__ __forceinline__ double gwh_pv2_phase(const InstCoef &C, double f, double phi, const Pv2Angles &P)
+{
+    return phi + 2. * (P.eps + C.eps_add) + C.t_corr_2pi * f;
+}
+
+/* IMRPhenomPv2 at one bin (IMRPhenomP.cpp:290-361): returns the common amplitude
+ * (already including the 1/2), the total phase and the complex h+ / hx twist-up factors. */
+__device__ __forceinline__ void gwh_pv2_fp64(const InstCoef &C, double f, const BinPow &bp, double &A, double &Phi,
+                                             double &hpr, double &hpi, double &hcr, double &hci,
+                                             const double2 *tab = gwh_turn_table, const double *etab = gwh_exp2_table)
+{
+    double u, phi;
+    gwh_phenomd_fp64(C, f, bp, A, phi, u, tab, etab);
+    const Pv2Angles P = gwh_pv2_angles(C, u, bp);
+    gwh_pv2_twist(C, P, hpr, hpi, hcr, hci, tab);
+    Phi = gwh_pv2_phase(C, f, phi, P);
 }
 
 #endif

@@ -159,9 +159,9 @@ __device__ __forceinline__ void gwh_loglike_tile(const WorkMap &W, const EventDe
                 if (!__ballot(live)) continue;
                 const BinPow bp = gwh_load_bin(E, k);
                 if (MODEL == GWH_IMRPHENOMD) {
-                    double a, phi, u, lx;
+                    double a, phi, u;
                     /* mixed: the merger-ringdown exponential in FP32, everything else as FP64 */
-                    gwh_phenomd_fp64<PREC == GWH_MIXED>(C, f, bp, a, phi, u, lx, tab, etab);
+                    gwh_phenomd_fp64<PREC == GWH_MIXED>(C, f, bp, a, phi, u, tab, etab);
                     a = live ? a : 0.0;
                     phi = live ? phi : 0.0;
 #pragma unroll
