@@ -23,8 +23,7 @@
  * where FP32 is faster on gfx950: with packed FP32 disabled, FP32 and FP64 FMAs
  * issue at the same rate, so only FP32 hardware transcendentals can pay --
  * the IMRPhenomD merger-ringdown exponential (FP32 exp2 with an FP64 exponent
- * split) and the IMRPhenomPv2 reciprocal square root's seed.  Phases, products
- * and sums stay FP64.
+ * split).  Phases, products and sums stay FP64; IMRPhenomPv2 runs the FP64 kernels.
  *
  * Reference: src/mcmc_gw.cpp:2374-2489 (MCMC_likelihood_extrinsic),
  * :801-868 (Log_Likelihood_internal), src/waveform_util.cpp:152-184
@@ -209,7 +208,7 @@ int gwh_ensure_init()
     E.events.assign(GWH_MAX_EVENTS, Event());
     GWH_HIP(hipGetSymbolAddress((void **)&E.noalloc_scratch, HIP_SYMBOL(scratch)));
     if (gwh_tiles_load<GWH_IMRPHENOMD, GWH_FP64>() || gwh_tiles_load<GWH_IMRPHENOMD, GWH_MIXED>() ||
-        gwh_tiles_load<GWH_IMRPHENOMPV2, GWH_FP64>() || gwh_tiles_load<GWH_IMRPHENOMPV2, GWH_MIXED>())
+        gwh_tiles_load<GWH_IMRPHENOMPV2, GWH_FP64>())
         return gwh_set_error(GWH_ERR_HIP, "loading the likelihood kernels failed");
     E.ready = true;
     return GWH_OK;
@@ -526,11 +525,12 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__rest
                 X.phi_aligned = F.phi_aligned;
                 zeta = F.zeta;
                 double ct = cos(F.thetaJN), st = sin(F.thetaJN);
-                C->ylm[0] = sqrt(5.0 / (64.0 * GWH_PI)) * (1.0 - ct) * (1.0 - ct);
-                C->ylm[1] = sqrt(5.0 / (16.0 * GWH_PI)) * st * (1.0 - ct);
-                C->ylm[2] = sqrt(15.0 / (32.0 * GWH_PI)) * st * st;
-                C->ylm[3] = sqrt(5.0 / (16.0 * GWH_PI)) * st * (1.0 + ct);
-                C->ylm[4] = sqrt(5.0 / (64.0 * GWH_PI)) * (1.0 + ct) * (1.0 + ct);
+                /* sums and differences of -2Y_2m(thetaJN, 0), m and -m (gwh_pv2_twist) */
+                C->tw[0] = sqrt(5.0 / (64.0 * GWH_PI)) * 2.0 * (1.0 + ct * ct);
+                C->tw[1] = sqrt(5.0 / (64.0 * GWH_PI)) * 4.0 * ct;
+                C->tw[2] = sqrt(5.0 / (16.0 * GWH_PI)) * 2.0 * st;
+                C->tw[3] = sqrt(5.0 / (16.0 * GWH_PI)) * 2.0 * st * ct;
+                C->tw[4] = sqrt(15.0 / (32.0 * GWH_PI)) * (GWH_SQRT_6 / 2.0) * st * st;
             }
             const EventDesc &E = events[ev];
             gwh_setup_detectors(p, pv2, zeta, geo, E.det, E.D, *C);
@@ -585,8 +585,9 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__rest
                 }
                 double vr = cbrt(GWH_PI * S.M * p.f_ref);
                 double lw = log(vr * vr * vr);
-                eul_a = gwh_euler_eval(a_c, vr, lw);
-                eul_e = gwh_euler_eval(e_c, vr, lw);
+                const double ivr = rcp_newton(vr);
+                eul_a = gwh_euler_eval(a_c, vr, ivr, lw);
+                eul_e = gwh_euler_eval(e_c, vr, ivr, lw);
             }
         }
         /* the tile count (a dependent chain of loads) on a role with a short chain: the detectors role for
@@ -898,10 +899,8 @@ static void launch_tiles(int model, int precision, int cls, long long items, con
         else
             gwh_launch_tiles<GWH_IMRPHENOMD, GWH_MIXED>(bpl, lanes, items, work, st, W, ev, c, part, act, count);
     } else {
-        if (precision == GWH_FP64)
-            gwh_launch_tiles<GWH_IMRPHENOMPV2, GWH_FP64>(bpl, lanes, items, work, st, W, ev, c, part, act, count);
-        else
-            gwh_launch_tiles<GWH_IMRPHENOMPV2, GWH_MIXED>(bpl, lanes, items, work, st, W, ev, c, part, act, count);
+        /* mixed precision keeps nothing in FP32 here: no FP32 part of the precessing evaluation pays */
+        gwh_launch_tiles<GWH_IMRPHENOMPV2, GWH_FP64>(bpl, lanes, items, work, st, W, ev, c, part, act, count);
     }
 }
 

@@ -592,7 +592,7 @@ __global__ __launch_bounds__(WAVES * 64) void gwh_fisher_fused_kernel(StencilArg
             }
             if (!__ballot(live)) continue;
             if (!(same & GWH_EV_SAME_CORE)) {
-                gwh_phenomd_core(Ci, f, bp, a0, psi, u);
+                gwh_phenomd_core<false, MODEL == GWH_IMRPHENOMPV2>(Ci, f, bp, a0, psi, u);
                 if (MODEL == GWH_IMRPHENOMPV2) ang = gwh_pv2_angles(Ci, u, bp);
             }
             if (MODEL == GWH_IMRPHENOMPV2 && !(same & GWH_EV_SAME_TWIST)) gwh_pv2_twist(Ci, ang, hpr, hpi, hcr, hci);

@@ -235,7 +235,7 @@ struct InstCoef {
     double a_c[5], e_c[5];   /* Euler alpha / epsilon coefficients */
     double alpha_add;        /* alpha0 - alpha(f_ref) */
     double eps_add;          /* -epsilon(f_ref) */
-    double ylm[5];           /* -2Y_2m(thetaJN, 0), m = -2..2 */
+    double tw[5];            /* twist-up constants from -2Y_2m(thetaJN, 0): gwh_pv2_twist */
     /* per detector: PhenomD: (Re K, Im K, |K|^2, 2 pi dt) ; Pv2: (P, Q, 0, 2 pi dt) */
     double det[GWH_MAXDET][4];
     double wf_a, wf_b; /* polarisation constants: PhenomD ((1+cos^2 i)/2, cos i); Pv2 (cos 2 zeta, sin 2 zeta) */
@@ -647,12 +647,11 @@ __device__ inline void gwh_euler_coeffs(double q, double chil, double chip, doub
             (1645 * m2_4 * chil2) / (192. * eta));
 }
 
-__device__ __forceinline__ double gwh_euler_eval(const double *c, double v, double logw)
+/* iv = 1 / v (a bin takes it from its tabulated f^{-1/3}).  The sum as explicit fused multiply-adds, so every kernel
+ * that inlines it (the GR and the modified-gravity setup among them) rounds it the same way */
+__device__ __forceinline__ double gwh_euler_eval(const double *c, double v, double iv, double logw)
 {
-    /* the negative powers of v from one Newton-refined reciprocal (the two angles of a bin share it once inlined)
-       instead of three FP64 division sequences; the sum as explicit fused multiply-adds, so every kernel that
-       inlines it (the GR and the modified-gravity setup among them) rounds it the same way */
-    const double iv = rcp_newton(v), iv2 = iv * iv;
+    const double iv2 = iv * iv;
     return fma(c[0], iv2 * iv, fma(c[1], iv2, fma(c[2], iv, fma(c[3], logw, c[4] * v))));
 }
 
@@ -1137,13 +1136,18 @@ __device__ __forceinline__ double gwh_ppe_bin(const InstCoef &C, double lf)
 }
 
 /* The part of IMRPhenomD that depends on the intrinsic parameters only: the amplitude a(f) without its prefactor
- * (distance, chirp mass) and the phase psi(f) without the time and phase shift; u = (M f)^{1/3}. */
-template <bool FP32_EXP = false>
+ * (distance, chirp mass) and the phase psi(f) without the time and phase shift; u = (M f)^{1/3}.
+ * TABLE_R: negative powers of M f from the tabulated f^{-1/3} instead of a reciprocal.  IMRPhenomPv2, which reads that
+ * table for its Euler angles anyway, takes them from there; IMRPhenomD needs one reciprocal per bin and would pay 8
+ * more bytes (256 uneven events, bound by the event data: 200 -> 215 us). */
+template <bool FP32_EXP = false, bool TABLE_R = false>
 __device__ __forceinline__ void gwh_phenomd_core(const InstCoef &C, double f, const BinPow &bp, double &a, double &psi,
                                                  double &u, const double2 *tab = gwh_turn_table,
                                                  const double *etab = gwh_exp2_table)
 {
     double Mf = C.M * f;
+    const double r = TABLE_R ? C.Mm13 * bp.fm13 : 0.0; /* (Mf)^{-1/3} */
+    const double r3 = r * r * r;
     u = C.M13 * bp.f13;              /* (Mf)^{1/3} */
     double inv76 = C.Mm76 * bp.fm76; /* (Mf)^{-7/6} */
     double ar;
@@ -1166,15 +1170,16 @@ __device__ __forceinline__ void gwh_phenomd_core(const InstCoef &C, double f, co
         double c6 = C.c10 - C.c11 * lx;
         double v2 = v * v;
         double poly = C.cp[0] + v2 * (C.cp[2] + v * (C.cp[3] + v * (C.cp[4] + v * (c5 + v * (c6 + v * C.cp[7])))));
+        const double iv = TABLE_R ? r * 0.68278406325529568 : 0.0, iv2 = iv * iv; /* 1/v = pi^{-1/3} (Mf)^{-1/3} */
         double Mf43 = Mf * u;
-        psi = -GWH_PI / 4. + C.K * poly * rcp_newton(v2 * v2 * v) +
+        psi = -GWH_PI / 4. + C.K * poly * (TABLE_R ? iv2 * iv2 * iv : rcp_newton(v2 * v2 * v)) +
               (C.sig[0] * Mf + C.sig[1] * Mf43 + C.sig[2] * Mf43 * u + C.sig[3] * Mf * Mf);
-        if (C.gimr) psi += gwh_gimr_bin(C, rcp_newton(v));
+        if (C.gimr) psi += gwh_gimr_bin(C, TABLE_R ? iv : rcp_newton(v));
     } else if (f > C.f2p) {
-        psi = C.alpha[0] + C.alpha[1] * Mf - C.alpha[2] * rcp_newton(Mf) + C.alpha[3] * (C.M34 * bp.f34) +
+        psi = C.alpha[0] + C.alpha[1] * Mf - C.alpha[2] * (TABLE_R ? r3 : rcp_newton(Mf)) + C.alpha[3] * (C.M34 * bp.f34) +
               C.alpha[4] * gwh_atan_seeded((f - C.alpha[5]) * C.inv_fdamp, tab);
     } else {
-        psi = C.beta[0] + C.beta[1] * Mf + C.beta[2] * (C.lgM + bp.lf) - C.beta[3] * rcp_newton(Mf * Mf * Mf);
+        psi = C.beta[0] + C.beta[1] * Mf + C.beta[2] * (C.lgM + bp.lf) - C.beta[3] * (TABLE_R ? r3 * r3 * r3 : rcp_newton(Mf * Mf * Mf));
     }
     if (C.ppe_n > 0 && (C.ppe_imr || f < C.f1p)) psi += gwh_ppe_bin(C, bp.lf);
 }
@@ -1187,73 +1192,55 @@ __device__ __forceinline__ double gwh_phase_shift(const InstCoef &C, double f, d
 
 /* IMRPhenomD amplitude A(f) and phase phi(f) = Psi(f) - tc_total (f - f_ref) - phic
  * (IMRPhenomD.cpp:471-501); caller guarantees 0 < f <= fcut. */
-template <bool FP32_EXP = false>
+template <bool FP32_EXP = false, bool TABLE_R = false>
 __device__ __forceinline__ void gwh_phenomd_fp64(const InstCoef &C, double f, const BinPow &bp, double &A, double &phi,
                                                  double &u, const double2 *tab = gwh_turn_table,
                                                  const double *etab = gwh_exp2_table)
 {
     double a, psi;
-    gwh_phenomd_core<FP32_EXP>(C, f, bp, a, psi, u, tab, etab);
+    gwh_phenomd_core<FP32_EXP, TABLE_R>(C, f, bp, a, psi, u, tab, etab);
     A = C.amp_pref * a;
     phi = gwh_phase_shift(C, f, psi);
 }
 
 /* What the IMRPhenomPv2 twist-up (IMRPhenomP.cpp:290-361) takes from the intrinsic parameters at one bin: cosine and
- * sine of half the opening angle, and the Euler angles without their offsets. */
+ * sine of the opening angle beta, and the Euler angles without their offsets. */
 struct Pv2Angles {
-    double cbh, sbh, alpha, eps;
+    double cb, sb, alpha, eps;
 };
 __device__ __forceinline__ Pv2Angles gwh_pv2_angles(const InstCoef &C, double u, const BinPow &bp)
 {
-    double v = u * 1.4645918875615231;
-    double logw = C.lgPiM + bp.lf; /* log(pi M f) */
-    double x = v * v;
-    double L = C.eta * (1.0 + C.L_c1 * x + C.L_c2 * x * x) * rcp_newton(v);
-    double s = C.SP * rcp_newton(L + C.SL);
-    double cb = rsqrt_seeded(1.0 + s * s);
-    /* cos and sin of beta/2: 1 - cos b = s^2 cos^2 b / (1 + cos b), so sin(b/2) = |s| cos b / (2 cos(b/2)), free of
-       the cancellation of sqrt((1 - cos b) / 2) for small s and one square root fewer */
+    const double v = u * 1.4645918875615231, iv = C.Mm13 * bp.fm13 * 0.68278406325529568; /* (pi M f)^{+-1/3} */
+    const double logw = C.lgPiM + bp.lf;                                                /* log(pi M f) */
+    const double x = v * v;
+    /* tan beta = S_perp / (L + S_L) with L = eta (1 + ...) / v, one reciprocal for both */
+    const double s = C.SP * v * rcp_newton(C.eta * (1.0 + C.L_c1 * x + C.L_c2 * x * x) + C.SL * v);
     Pv2Angles P;
-    P.cbh = sqrt((1.0 + cb) / 2.0);
-    P.sbh = fabs(s) * cb * (0.5 * rcp_newton(P.cbh));
-    P.alpha = gwh_euler_eval(C.a_c, v, logw);
-    P.eps = gwh_euler_eval(C.e_c, v, logw);
+    P.cb = rsqrt_seeded(1.0 + s * s);
+    P.sb = fabs(s) * P.cb;
+    P.alpha = gwh_euler_eval(C.a_c, v, iv, logw);
+    P.eps = gwh_euler_eval(C.e_c, v, iv, logw);
     return P;
 }
 
-/* the complex h+ / hx twist-up factors */
+/* The complex h+ / hx twist-up factors sum_m e^{-i m alpha} d_{-m} Y_m + e^{i m alpha} d_m Y_m (and their difference times
+ * i) over m = -2..2, with the rotation elements d_m of spin 2 to m' = +-2 at beta.  Collected by powers of e^{i alpha}
+ * only sums and differences of d_m and d_{-m} remain, and these are polynomials in cos beta and sin beta:
+ * d_2 + d_{-2} = (1 + cos^2 beta) / 2, d_2 - d_{-2} = cos beta, d_1 + d_{-1} = sin beta, d_1 - d_{-1} = sin beta cos beta,
+ * d_0 = sqrt(6)/4 sin^2 beta.  No half angles, no cancellation; 26 operations where the sum over m took 90 and the half
+ * angle another 30 (a square root and a reciprocal).  C.tw = {Y_2 + Y_{-2}, Y_2 - Y_{-2}, Y_1 + Y_{-1}, Y_1 - Y_{-1},
+ * sqrt(6)/2 Y_0}. */
 __device__ __forceinline__ void gwh_pv2_twist(const InstCoef &C, const Pv2Angles &P, double &hpr, double &hpi,
                                               double &hcr, double &hci, const double2 *tab = gwh_turn_table)
 {
-    const double cbh = P.cbh, sbh = P.sbh;
-    double c2 = cbh * cbh, s2 = sbh * sbh, c3 = c2 * cbh, s3 = s2 * sbh;
-    double d2[5] = {s3 * sbh, 2 * cbh * s3, GWH_SQRT_6 * s2 * c2, 2 * c3 * sbh, c3 * cbh};
     double sa, ca;
     gwh_sincos_tab(P.alpha + C.alpha_add, sa, ca, tab);
-    /* e^{i m alpha}, m=-2..2 */
-    double er[5], ei[5];
-    er[2] = 1;
-    ei[2] = 0;
-    er[3] = ca;
-    ei[3] = sa;
-    er[1] = ca;
-    ei[1] = -sa;
-    er[4] = ca * ca - sa * sa;
-    ei[4] = 2 * ca * sa;
-    er[0] = er[4];
-    ei[0] = -ei[4];
-    hpr = hpi = hcr = hci = 0;
-#pragma unroll
-    for (int m = -2; m <= 2; m++) {
-        double dm2 = (m == -2) ? d2[4] : (m == -1) ? -d2[3] : (m == 0) ? d2[2] : (m == 1) ? -d2[1] : d2[0];
-        double y = C.ylm[m + 2];
-        double t2r = er[-m + 2] * dm2 * y, t2i = ei[-m + 2] * dm2 * y;
-        double tmr = er[m + 2] * d2[m + 2] * y, tmi = ei[m + 2] * d2[m + 2] * y;
-        hpr += t2r + tmr;
-        hpi += t2i + tmi;
-        hcr -= t2i - tmi;
-        hci += t2r - tmr;
-    }
+    const double c2 = ca * ca - sa * sa, s2 = 2.0 * sa * ca;
+    const double e = 0.5 + 0.5 * P.cb * P.cb, g = P.sb * P.cb;
+    hpr = C.tw[0] * (e * c2) + C.tw[3] * (g * ca) + C.tw[4] * (P.sb * P.sb);
+    hpi = C.tw[0] * (P.cb * s2) + C.tw[3] * (P.sb * sa);
+    hcr = C.tw[1] * (e * s2) + C.tw[2] * (g * sa);
+    hci = -(C.tw[1] * (P.cb * c2) + C.tw[2] * (P.sb * ca));
 }
 
 /* phase of IMRPhenomPv2 from the shifted IMRPhenomD phase: 2 epsilon and the t_c correction */
@@ -1269,7 +1256,7 @@ __device__ __forceinline__ void gwh_pv2_fp64(const InstCoef &C, double f, const 
                                              const double2 *tab = gwh_turn_table, const double *etab = gwh_exp2_table)
 {
     double u, phi;
-    gwh_phenomd_fp64(C, f, bp, A, phi, u, tab, etab);
+    gwh_phenomd_fp64<false, true>(C, f, bp, A, phi, u, tab, etab);
     const Pv2Angles P = gwh_pv2_angles(C, u, bp);
     gwh_pv2_twist(C, P, hpr, hpi, hcr, hci, tab);
     Phi = gwh_pv2_phase(C, f, phi, P);

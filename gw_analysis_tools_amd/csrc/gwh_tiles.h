@@ -1,9 +1,9 @@
 /*
  * gwh_tiles.h -- the per-bin network log-likelihood kernels: one (instance, tile) work item per block, a tile of
- * TPB lanes x BPL bins per lane (TPB in 64..1024, BPL in 1..8, chosen per event: fixed default or autotuned), and
- * the mixed-precision pieces of the per-bin evaluation.  Included by the engine (declarations, the block reduction
- * and the work map) and by the four translation units that instantiate the kernels of one (model, precision) each,
- * so the 160 kernels compile in parallel.
+ * TPB lanes x BPL bins per lane (TPB in 64..1024, BPL in 1..8, chosen per event: fixed default or autotuned).
+ * Included by the engine (declarations, the block reduction and the work map) and by the three translation units that
+ * instantiate the kernels of one (model, precision) each (IMRPhenomPv2 runs in FP64 in both modes), so the 120 kernels
+ * compile in parallel.
  */
 #pragma once
 
@@ -48,64 +48,6 @@ __device__ __forceinline__ void block_reduce_store(double (&acc)[NV], double *__
     }
 }
 
-
-/* ------------------------------------------------------------------------- */
-/* per-bin mixed-precision evaluators                                         */
-/* ------------------------------------------------------------------------- */
-
-/* IMRPhenomD in mixed precision: the FP64 evaluator with the merger-ringdown amplitude's exponential in FP32
- * (TABLE_EXP false: ~6e-8 relative per bin) or through the FP64 table (true: a few ulp); the phase, including its
- * arctangent, stays FP64 (an FP32 atan there was the largest error of the path, ~7e-4 in logL for heavy
- * binaries). */
-template <bool TABLE_EXP>
-__device__ __forceinline__ void gwh_phenomd_mixed(const InstCoef &C, double f, const BinPow &bp, double &a, double &phi,
-                                                  double &u_out, double &lx_out, const double2 *tab = gwh_turn_table,
-                                                  const double *etab = gwh_exp2_table)
-{
-    double Mf = C.M * f;
-    double r = C.Mm13 * bp.fm13;     /* (Mf)^{-1/3} */
-    double u = C.M13 * bp.f13;       /* (Mf)^{1/3} */
-    double r2 = r * r;
-    double inv76 = C.Mm76 * bp.fm76; /* (Mf)^{-7/6} */
-    double ar;
-    if (f < C.f1) {
-        double pn = C.ca[0] + u * u * (C.ca[2] + u * (C.ca[3] + u * (C.ca[4] + u * (C.ca[5] + u * C.ca[6]))));
-        double u3 = u * u * u;
-        ar = pn + u3 * u3 * u * (C.rho[0] + u * (C.rho[1] + u * C.rho[2]));
-    } else if (f > C.f3) {
-        double dl = f - C.fRD;
-        ar = C.mr_k * (TABLE_EXP ? gwh_exp_table(-C.mr_g2 * dl, etab) : exp_fp32(-C.mr_g2 * dl)) * rcp_newton(dl * dl + C.mr_w2);
-    } else {
-        ar = C.delta[0] + Mf * (C.delta[1] + Mf * (C.delta[2] + Mf * (C.delta[3] + Mf * C.delta[4])));
-    }
-    a = C.amp_pref * ar * inv76;
-    double psi;
-    double lx = 0;
-    if (f < C.f1p) {
-        double v = u * 1.4645918875615231;
-        lx = C.lgPiM + bp.lf; /* log(pi M f) */
-        double c5 = C.c8 + lx * C.c9;
-        double c6 = C.c10 - C.c11 * lx;
-        double v2 = v * v;
-        double poly = C.cp[0] + v2 * (C.cp[2] + v * (C.cp[3] + v * (C.cp[4] + v * (c5 + v * (c6 + v * C.cp[7])))));
-        double iv = r * 0.68278406325529568; /* 1/v = pi^{-1/3} (Mf)^{-1/3} */
-        double iv2 = iv * iv;
-        double Mf43 = Mf * u;
-        psi = -GWH_PI / 4. + C.K * poly * (iv2 * iv2 * iv) +
-              (C.sig[0] * Mf + C.sig[1] * Mf43 + C.sig[2] * Mf43 * u + C.sig[3] * Mf * Mf);
-        if (C.gimr) psi += gwh_gimr_bin(C, iv);
-    } else if (f > C.f2p) {
-        psi = C.alpha[0] + C.alpha[1] * Mf - C.alpha[2] * (r2 * r) + C.alpha[3] * (C.M34 * bp.f34) +
-              C.alpha[4] * gwh_atan_seeded((f - C.alpha[5]) * C.inv_fdamp, tab);
-    } else {
-        double r3 = r2 * r;
-        psi = C.beta[0] + C.beta[1] * Mf + C.beta[2] * (C.lgM + bp.lf) - C.beta[3] * (r3 * r3 * r3);
-    }
-    if (C.ppe_n > 0 && (C.ppe_imr || f < C.f1p)) psi += gwh_ppe_bin(C, bp.lf); /* FP64: phase accuracy */
-    phi = psi - (C.tc_total * (f - C.f_ref) + C.phic);
-    u_out = u;
-    lx_out = lx;
-}
 
 /* ------------------------------------------------------------------------- */
 /* the batched likelihood kernels                                             */
@@ -177,55 +119,7 @@ __device__ __forceinline__ void gwh_loglike_tile(const WorkMap &W, const EventDe
                     }
                 } else {
                     double A, Phi, hpr, hpi, hcr, hci;
-                    if (PREC == GWH_FP64) {
-                        gwh_pv2_fp64(C, f, bp, A, Phi, hpr, hpi, hcr, hci, tab, etab);
-                    } else {
-                        double u, lx;
-                        gwh_phenomd_mixed<true>(C, f, bp, A, Phi, u, lx, tab, etab);
-                        /* precession angles and the sin/cos of the Euler angle alpha in FP64 (alpha's rounding
-                         * would enter |h|^2 directly), like the detector phases below: table-driven sin/cos and
-                         * exponential (the FP32 ones left ~2.5e-4 in logL on short, loud precessing events) */
-                        const double v = u * 1.4645918875615231;
-                        const double logw = C.lgPiM + bp.lf; /* log(pi M f) */
-                        const double x = v * v;
-                        const double L = C.eta * (1.0 + C.L_c1 * x + C.L_c2 * x * x) * rcp_newton(v);
-                        const double sv = C.SP * rcp_newton(L + C.SL);
-                        const double cbd = rsqrt_seeded(1.0 + sv * sv);
-                        /* sin(beta/2) = |s| cos b / (2 cos(beta/2)): no cancellation, one square root */
-                        const double cbhd = sqrt(0.5 * (1.0 + cbd)), sbhd = fabs(sv) * cbd * (0.5 * rcp_newton(cbhd));
-                        const double c2d = cbhd * cbhd, s2d = sbhd * sbhd;
-                        const double d2[5] = {s2d * s2d, 2. * cbhd * s2d * sbhd, GWH_SQRT_6 * s2d * c2d,
-                                              2. * c2d * cbhd * sbhd, c2d * c2d};
-                        const double alpha = gwh_euler_eval(C.a_c, v, logw) + C.alpha_add;
-                        const double eps = gwh_euler_eval(C.e_c, v, logw) + C.eps_add;
-                        double sa, ca;
-                        gwh_sincos_tab(alpha, sa, ca, tab);
-                        double er[5], ei[5];
-                        er[2] = 1.;
-                        ei[2] = 0.;
-                        er[3] = ca;
-                        ei[3] = sa;
-                        er[1] = ca;
-                        ei[1] = -sa;
-                        er[4] = ca * ca - sa * sa;
-                        ei[4] = 2. * ca * sa;
-                        er[0] = er[4];
-                        ei[0] = -ei[4];
-                        hpr = hpi = hcr = hci = 0;
-#pragma unroll
-                        for (int m = -2; m <= 2; m++) {
-                            const double dm2 =
-                                (m == -2) ? d2[4] : (m == -1) ? -d2[3] : (m == 0) ? d2[2] : (m == 1) ? -d2[1] : d2[0];
-                            const double y = C.ylm[m + 2];
-                            const double t2r = er[-m + 2] * dm2 * y, t2i = ei[-m + 2] * dm2 * y;
-                            const double tmr = er[m + 2] * d2[m + 2] * y, tmi = ei[m + 2] * d2[m + 2] * y;
-                            hpr += t2r + tmr;
-                            hpi += t2i + tmi;
-                            hcr -= t2i - tmi;
-                            hci += t2r - tmr;
-                        }
-                        Phi = Phi + 2. * eps + C.t_corr_2pi * f;
-                    }
+                    gwh_pv2_fp64(C, f, bp, A, Phi, hpr, hpi, hcr, hci, tab, etab);
                     A = live ? A : 0.0;
                     Phi = live ? Phi : 0.0;
 #pragma unroll
@@ -360,4 +254,3 @@ template <int MODEL, int PREC> int gwh_tiles_load()
 GWH_TILES_DECLARE(GWH_IMRPHENOMD, GWH_FP64)
 GWH_TILES_DECLARE(GWH_IMRPHENOMD, GWH_MIXED)
 GWH_TILES_DECLARE(GWH_IMRPHENOMPV2, GWH_FP64)
-GWH_TILES_DECLARE(GWH_IMRPHENOMPV2, GWH_MIXED)
