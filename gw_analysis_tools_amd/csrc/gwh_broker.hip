@@ -171,7 +171,7 @@ size_t lane_bytes_after(const Lane &L, const std::vector<int> &events, int n)
     const size_t m = (size_t)n;
     return gwh_grown_capacity(m * sizeof(InstCoef), S.coef.cap) +
            gwh_grown_capacity(m * maxtiles * GWH_PARTIAL_STRIDE * sizeof(double), S.partial.cap) +
-           gwh_grown_capacity(m * sizeof(int), S.active.cap) + gwh_grown_capacity(tiles * sizeof(int2), S.work.cap) +
+           gwh_grown_capacity(m * sizeof(int), S.active.cap) + gwh_grown_capacity(gwh_worklist_bytes(tiles), S.work.cap) +
            gwh_grown_capacity(GWH_NCLASS * sizeof(int), S.wcount.cap) +
            gwh_grown_capacity(m * sizeof(gwh_params), L.d_params.cap) +
            gwh_grown_capacity(m * sizeof(int), L.d_events.cap) + gwh_grown_capacity(m * sizeof(double), L.d_logl.cap);

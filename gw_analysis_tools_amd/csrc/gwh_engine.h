@@ -55,6 +55,10 @@ static inline int gwh_tiles_of(const EventDesc &d)
     return (d.N + t - 1) / t;
 }
 
+/* device bytes of the work lists of a multi-event batch with `items` (instance, tile) items at most: one list per number
+ * of lanes per tile, each with room for 7 holes */
+static inline size_t gwh_worklist_bytes(size_t items) { return (items + 5 * 7) * sizeof(int2); }
+
 /* Loads through global-address-space pointers.  Pointers held in device structs are generic, and generic
  * (flat) loads count against the scalar-memory counter as well as the vector one, so every wait for a
  * scalar load of the instance coefficients would also wait for the bin data in flight. */

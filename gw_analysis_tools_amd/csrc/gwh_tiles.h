@@ -2,7 +2,7 @@
  * gwh_tiles.h -- the per-bin network log-likelihood kernels: one (instance, tile) work item per block, a tile of
  * TPB lanes x BPL bins per lane (TPB in 64..1024, BPL in 1..8, chosen per event: fixed default or autotuned).
  * Included by the engine (declarations, the block reduction and the work map) and by the three translation units that
- * instantiate the kernels of one (model, precision) each (IMRPhenomPv2 runs in FP64 in both modes), so the 120 kernels
+ * instantiate the kernels of one (model, precision) each (IMRPhenomPv2 runs in FP64 in both modes), so the 75 kernels
  * compile in parallel.
  */
 #pragma once
@@ -59,19 +59,21 @@ struct WorkMap {
 };
 
 /* One (instance, tile) work item: TPB lanes x BPL bins of one instance's network log-likelihood, reduced
- * to the instance's partial sums for that tile.  Every early return is uniform over the block. */
-template <int MODEL, int PREC, int BPL, int TPB>
+ * to the instance's partial sums for that tile.  Every early return is uniform over the block.
+ * ANY: an item of a work list, whose event has TPB lanes and any number of bins per lane up to BPL = 8 (the unrolled
+ * steps past it are skipped). */
+template <int MODEL, int PREC, int BPL, int TPB, bool ANY = false>
 __device__ __forceinline__ void gwh_loglike_tile(const WorkMap &W, const EventDesc *__restrict__ events,
                                                  const InstCoef *__restrict__ coefs, double *__restrict__ partial,
-                                                 const int *__restrict__ active, const int inst, const int tile,
+                                                 const int *__restrict__ active, const int ev, const int inst, const int tile,
                                                  double (*lds)[GWH_PARTIAL_STRIDE], double2 *__restrict__ tab,
                                                  double *__restrict__ etab)
 {
     {
-        const int ev = W.inst_event ? W.inst_event[inst] : W.event0;
         const EventDesc &E = events[ev];
-        if (E.bpl != BPL || E.lanes != TPB) return; /* the instance's event is tiled by another launch */
-        if (tile >= active[inst]) return; /* above 0.2/M on an ascending grid: h = 0, nothing to add */
+        if (!ANY && (E.bpl != BPL || E.lanes != TPB)) return; /* the instance's event is tiled by another launch */
+        if (!ANY && tile >= active[inst]) return; /* above 0.2/M on an ascending grid: h = 0, nothing to add */
+        const int bpl = ANY ? E.bpl : BPL;
         const int w = inst * W.tiles0 + tile;
         const InstCoef &C = coefs[inst];
         const int N = E.N, D = E.D;
@@ -79,8 +81,8 @@ __device__ __forceinline__ void gwh_loglike_tile(const WorkMap &W, const EventDe
 #pragma unroll
         for (int j = 0; j < GWH_PARTIAL_STRIDE; j++) acc[j] = 0;
         /* skip tiles entirely above the 0.2/M cutoff (h = 0 there, IMRPhenomD.cpp:475) */
-        constexpr int kLevel = gwh_tile_level(TPB * BPL);
-        const double fmin_tile = gwh_g(E.tile_fmin)[E.fmin_off[kLevel] + tile];
+        const int level = ANY ? gwh_tile_level(TPB) + (__ffs(bpl) - 1) : gwh_tile_level(TPB * BPL);
+        const double fmin_tile = gwh_g(E.tile_fmin)[E.fmin_off[level] + tile];
         if (!(fmin_tile > C.fcut)) {
             /* the sin/cos and exponential tables in LDS: the detector phases (one gather per detector and bin), the
                merger-ringdown arctangent's correction and exponential and the IMRPhenomPv2 Euler angle read them
@@ -90,10 +92,11 @@ __device__ __forceinline__ void gwh_loglike_tile(const WorkMap &W, const EventDe
             __syncthreads();
 #pragma unroll
             for (int j = 0; j < BPL; j++) {
+                if (ANY && j >= bpl) break;
                 /* Lanes past the end of the grid or above 0.2/M evaluate the last grid bin with a zero amplitude
                  * (and phase), so the accumulators never sit under divergent control flow; a wave without any
                  * bin at or below the cutoff skips the step on a uniform branch. */
-                const int k0 = tile * TPB * BPL + j * TPB + threadIdx.x;
+                const int k0 = tile * TPB * bpl + j * TPB + threadIdx.x;
                 const bool in = k0 < N;
                 const int k = in ? k0 : N - 1;
                 const double f = gwh_g(E.f)[k];
@@ -141,13 +144,13 @@ __device__ __forceinline__ void gwh_loglike_tile(const WorkMap &W, const EventDe
     }
 }
 
-/* the flattened (instance, tile) work list of one tiling class: one block per live work item, so batches mixing
- * 10^3- and 10^5-bin events launch no empty blocks; entries fold over y beyond 2^20 blocks */
-template <int MODEL, int PREC, int BPL, int TPB>
+/* the flattened (instance, tile) work list of one number of lanes per tile (gwh_worklist_kernel): one block per live
+ * work item, so batches mixing 10^3- and 10^5-bin events launch no empty blocks; entries fold over y beyond 2^20
+ * blocks */
+template <int MODEL, int PREC, int TPB>
 __global__ __launch_bounds__(TPB) void gwh_loglike_wl_kernel(WorkMap W, const EventDesc *__restrict__ events,
                                                              const InstCoef *__restrict__ coefs,
                                                              double *__restrict__ partial,
-                                                             const int *__restrict__ active,
                                                              const int2 *__restrict__ work,
                                                              const int *__restrict__ count)
 {
@@ -157,7 +160,9 @@ __global__ __launch_bounds__(TPB) void gwh_loglike_wl_kernel(WorkMap W, const Ev
     const int w = blockIdx.y * gridDim.x + blockIdx.x;
     if (w >= *count) return;
     const int2 wi = work[w];
-    gwh_loglike_tile<MODEL, PREC, BPL, TPB>(W, events, coefs, partial, active, wi.x, wi.y, lds, tab, etab);
+    if (wi.x < 0) return; /* a hole at the end of a column */
+    gwh_loglike_tile<MODEL, PREC, 8, TPB, true>(W, events, coefs, partial, nullptr, wi.x >> 16, wi.x & 0xffff, wi.y, lds,
+                                                tab, etab);
 }
 
 /* One block per (instance, tile) item, in tile-major order (item w = tile * n + instance).  Consecutive blocks go
@@ -183,57 +188,69 @@ __global__ __launch_bounds__(TPB) void gwh_loglike_grid_kernel(WorkMap W, const 
     const int nn = count ? min(*count, W.n) : W.n;
     const int w = blockIdx.y * gridDim.x + blockIdx.x; /* items fold over y beyond 2^20 blocks */
     if (nn <= 0 || w >= nn * W.tiles0) return;
-    gwh_loglike_tile<MODEL, PREC, BPL, TPB>(W, events, coefs, partial, active, w % nn, w / nn, lds, tab, etab);
+    const int inst = w % nn;
+    gwh_loglike_tile<MODEL, PREC, BPL, TPB>(W, events, coefs, partial, active, W.inst_event ? W.inst_event[inst] : W.event0,
+                                            inst, w / nn, lds, tab, etab);
 }
 
 /* ------------------------------------------------------------------------- */
 /* launch of one tiling class                                                 */
 /* ------------------------------------------------------------------------- */
 
-template <int MODEL, int PREC, int BPL, int TPB>
-static void gwh_launch_tiles_one(long long items, const int2 *work, hipStream_t st, const WorkMap &W,
-                                 const EventDesc *ev, const InstCoef *c, double *part, const int *act,
-                                 const int *count)
+/* a dispatch counts work-items in 32 bits per dimension: at most 2^20 blocks along x */
+static inline dim3 gwh_tile_grid(long long items)
 {
-    /* a dispatch counts work-items in 32 bits per dimension: at most 2^20 blocks along x */
     const long long gx = std::max(1LL, std::min(items, 1LL << 20)), gy = std::max(1LL, (items + gx - 1) / gx);
-    const dim3 g((unsigned)gx, (unsigned)gy);
-    if (work)
-        hipLaunchKernelGGL((gwh_loglike_wl_kernel<MODEL, PREC, BPL, TPB>), g, dim3(TPB), 0, st, W, ev, c, part, act,
-                           work, count);
-    else
-        hipLaunchKernelGGL((gwh_loglike_grid_kernel<MODEL, PREC, BPL, TPB>), g, dim3(TPB), 0, st, W, ev, c, part,
-                           act, count);
+    return dim3((unsigned)gx, (unsigned)gy);
 }
 
 template <int MODEL, int PREC, int TPB>
-static void gwh_launch_tiles_lanes(int bpl, long long items, const int2 *work, hipStream_t st, const WorkMap &W,
-                                   const EventDesc *ev, const InstCoef *c, double *part, const int *act,
-                                   const int *count)
+static void gwh_launch_tiles_lanes(int bpl, long long items, hipStream_t st, const WorkMap &W, const EventDesc *ev,
+                                   const InstCoef *c, double *part, const int *act, const int *count)
 {
+    const dim3 g = gwh_tile_grid(items), b(TPB);
+#define GWH_GRID(BPL) hipLaunchKernelGGL((gwh_loglike_grid_kernel<MODEL, PREC, BPL, TPB>), g, b, 0, st, W, ev, c, part, act, count)
     switch (bpl) {
-    case 1: gwh_launch_tiles_one<MODEL, PREC, 1, TPB>(items, work, st, W, ev, c, part, act, count); break;
-    case 2: gwh_launch_tiles_one<MODEL, PREC, 2, TPB>(items, work, st, W, ev, c, part, act, count); break;
-    case 4: gwh_launch_tiles_one<MODEL, PREC, 4, TPB>(items, work, st, W, ev, c, part, act, count); break;
-    default: gwh_launch_tiles_one<MODEL, PREC, 8, TPB>(items, work, st, W, ev, c, part, act, count); break;
+    case 1: GWH_GRID(1); break;
+    case 2: GWH_GRID(2); break;
+    case 4: GWH_GRID(4); break;
+    default: GWH_GRID(8); break;
+    }
+#undef GWH_GRID
+}
+
+/* The per-bin kernel of one tiling class (bpl bins per lane x lanes per tile) over a batch on one event tiling: one
+ * block per (instance, tile) item (items = n x tiles; count = the optional device instance count).  Each (MODEL, PREC)
+ * is instantiated in its own translation unit (gwh_tiles_*.hip). */
+template <int MODEL, int PREC>
+void gwh_launch_tiles(int bpl, int lanes, long long items, hipStream_t st, const WorkMap &W, const EventDesc *ev,
+                      const InstCoef *c, double *part, const int *act, const int *count)
+{
+    switch (lanes) {
+    case 64: gwh_launch_tiles_lanes<MODEL, PREC, 64>(bpl, items, st, W, ev, c, part, act, count); break;
+    case 128: gwh_launch_tiles_lanes<MODEL, PREC, 128>(bpl, items, st, W, ev, c, part, act, count); break;
+    case 512: gwh_launch_tiles_lanes<MODEL, PREC, 512>(bpl, items, st, W, ev, c, part, act, count); break;
+    case 1024: gwh_launch_tiles_lanes<MODEL, PREC, 1024>(bpl, items, st, W, ev, c, part, act, count); break;
+    default: gwh_launch_tiles_lanes<MODEL, PREC, 256>(bpl, items, st, W, ev, c, part, act, count); break;
     }
 }
 
-/* The per-bin kernel of one tiling class (bpl bins per lane x lanes per tile).  work == nullptr: one block per
- * (instance, tile) item of a batch over one event tiling (items = n x tiles; count = the optional device instance
- * count); otherwise one block per entry of the class's work list (items = its upper bound; count = its device
- * length).  Each (MODEL, PREC) is instantiated in its own translation unit (gwh_tiles_*.hip). */
+/* The per-bin kernel over a work list of one number of lanes per tile: one block per entry (items = the list's upper
+ * bound; count = its device length). */
 template <int MODEL, int PREC>
-void gwh_launch_tiles(int bpl, int lanes, long long items, const int2 *work, hipStream_t st, const WorkMap &W,
-                      const EventDesc *ev, const InstCoef *c, double *part, const int *act, const int *count)
+void gwh_launch_worklist(int lanes, long long items, const int2 *work, hipStream_t st, const WorkMap &W,
+                         const EventDesc *ev, const InstCoef *c, double *part, const int *count)
 {
+    const dim3 g = gwh_tile_grid(items);
+#define GWH_WL(TPB) hipLaunchKernelGGL((gwh_loglike_wl_kernel<MODEL, PREC, TPB>), g, dim3(TPB), 0, st, W, ev, c, part, work, count)
     switch (lanes) {
-    case 64: gwh_launch_tiles_lanes<MODEL, PREC, 64>(bpl, items, work, st, W, ev, c, part, act, count); break;
-    case 128: gwh_launch_tiles_lanes<MODEL, PREC, 128>(bpl, items, work, st, W, ev, c, part, act, count); break;
-    case 512: gwh_launch_tiles_lanes<MODEL, PREC, 512>(bpl, items, work, st, W, ev, c, part, act, count); break;
-    case 1024: gwh_launch_tiles_lanes<MODEL, PREC, 1024>(bpl, items, work, st, W, ev, c, part, act, count); break;
-    default: gwh_launch_tiles_lanes<MODEL, PREC, 256>(bpl, items, work, st, W, ev, c, part, act, count); break;
+    case 64: GWH_WL(64); break;
+    case 128: GWH_WL(128); break;
+    case 512: GWH_WL(512); break;
+    case 1024: GWH_WL(1024); break;
+    default: GWH_WL(256); break;
     }
+#undef GWH_WL
 }
 /* Load the code object holding the kernels of one (MODEL, PREC) on the current device: the runtime loads a
  * translation unit's kernels at the first use of any of them, a few milliseconds that would otherwise fall on the
@@ -247,9 +264,11 @@ template <int MODEL, int PREC> int gwh_tiles_load()
                : -1;
 }
 #define GWH_TILES_DECLARE(M, P)                                                                                    \
-    extern template void gwh_launch_tiles<M, P>(int, int, long long, const int2 *, hipStream_t, const WorkMap &,    \
+    extern template void gwh_launch_tiles<M, P>(int, int, long long, hipStream_t, const WorkMap &,                  \
                                                 const EventDesc *, const InstCoef *, double *, const int *,         \
                                                 const int *);                                                       \
+    extern template void gwh_launch_worklist<M, P>(int, long long, const int2 *, hipStream_t, const WorkMap &,      \
+                                                   const EventDesc *, const InstCoef *, double *, const int *);     \
     extern template int gwh_tiles_load<M, P>();
 GWH_TILES_DECLARE(GWH_IMRPHENOMD, GWH_FP64)
 GWH_TILES_DECLARE(GWH_IMRPHENOMD, GWH_MIXED)
