@@ -113,10 +113,15 @@ GWH_HD static void unpack(const gwh_params &p, int basis, double *v, int *lf)
     }
 }
 
-/* a: a gen_params carrying only the non-parameter options (fisher.cpp:2513-2572) */
-GWH_HD static void repack(const double *v, int basis, gwh_params &a)
+/* parts of a basis vector's record that do not depend on each other (a kernel gives each its own wave) */
+#define GWH_REPACK_PARTS 3
+
+/* a: a gen_params carrying only the non-parameter options (fisher.cpp:2513-2572).  Part 0: sky position, orientation,
+ * phase, time; 1: distance and (cosine of) inclination, IMRPhenomPv2's first spin; 2: masses and spins */
+GWH_HD static void repack_part(const double *v, int basis, int part, gwh_params &a)
 {
     if (basis == GWH_BASIS_PHENOMD_SKYAVG) {
+        if (part != 2) return;
         a.mass1 = mass1_of(v[3], v[4]);
         a.mass2 = mass2_of(v[3], v[4]);
         double mcs = v[3] * kMsolSec;
@@ -127,24 +132,33 @@ GWH_HD static void repack(const double *v, int basis, gwh_params &a)
         a.spin2[2] = v[5] - v[6];
         return;
     }
-    bool mcmc = (basis == GWH_BASIS_PHENOMD_MCMC || basis == GWH_BASIS_PV2_MCMC);
-    a.mass1 = mass1_of(mcmc ? exp(v[7]) : v[7], v[8]);
-    a.mass2 = mass2_of(mcmc ? exp(v[7]) : v[7], v[8]);
-    a.DL = mcmc ? exp(v[6]) : v[6];
-    a.RA = v[0];
-    a.DEC = mcmc ? asin(v[1]) : v[1];
-    a.psi = v[2];
-    a.incl = mcmc ? acos(v[3]) : v[3];
-    a.phiRef = v[4];
-    a.tc = v[5];
+    const bool mcmc = (basis == GWH_BASIS_PHENOMD_MCMC || basis == GWH_BASIS_PV2_MCMC);
+    if (part == 0) {
+        a.RA = v[0];
+        a.DEC = mcmc ? asin(v[1]) : v[1];
+        a.psi = v[2];
+        a.phiRef = v[4];
+        a.tc = v[5];
+    } else if (part == 1) {
+        a.DL = mcmc ? exp(v[6]) : v[6];
+        a.incl = mcmc ? acos(v[3]) : v[3];
+    } else {
+        const double mc = mcmc ? exp(v[7]) : v[7];
+        a.mass1 = mass1_of(mc, v[8]);
+        a.mass2 = mass2_of(mc, v[8]);
+    }
     if (basis == GWH_BASIS_PV2_MCMC) {
         /* bump cos(theta) back into [-1, 1] (fisher.cpp:2188-2210) */
-        double t1 = v[11] > 1 ? 0 : (v[11] < -1 ? M_PI : acos(v[11]));
-        double t2 = v[12] > 1 ? 0 : (v[12] < -1 ? M_PI : acos(v[12]));
-        double s1[3] = {v[9], t1, v[13]}, s2[3] = {v[10], t2, v[14]};
-        sph_to_cart(s1, a.spin1);
-        sph_to_cart(s2, a.spin2);
-    } else {
+        if (part == 1) {
+            double t1 = v[11] > 1 ? 0 : (v[11] < -1 ? M_PI : acos(v[11]));
+            double s1[3] = {v[9], t1, v[13]};
+            sph_to_cart(s1, a.spin1);
+        } else if (part == 2) {
+            double t2 = v[12] > 1 ? 0 : (v[12] < -1 ? M_PI : acos(v[12]));
+            double s2[3] = {v[10], t2, v[14]};
+            sph_to_cart(s2, a.spin2);
+        }
+    } else if (part == 2) {
         a.spin1[2] = v[9];
         a.spin2[2] = v[10];
         if (basis == GWH_BASIS_PV2_FULL) {
@@ -152,6 +166,10 @@ GWH_HD static void repack(const double *v, int basis, gwh_params &a)
             a.phip = v[12];
         }
     }
+}
+GWH_HD static void repack(const double *v, int basis, gwh_params &a)
+{
+    for (int part = 0; part < GWH_REPACK_PARTS; part++) repack_part(v, basis, part, a);
 }
 
 #endif

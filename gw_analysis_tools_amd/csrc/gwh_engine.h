@@ -116,6 +116,85 @@ __device__ __forceinline__ double wave_sum(double v)
     return (read_lane(v, 0) + read_lane(v, 16)) + (read_lane(v, 32) + read_lane(v, 48));
 }
 
+/* instances of one batch: their events and the tile stride of the partial sums */
+struct WorkMap {
+    const int *inst_event; /* NULL: every instance uses event0 */
+    int event0, n, tiles0; /* tiles0: tile stride of the partial buffer */
+};
+
+/* what the last kernel of a batched likelihood reads */
+struct FinalizeArgs {
+    WorkMap W;
+    const EventDesc *events;
+    const InstCoef *coefs;
+    const double *partial;
+    const int *active;
+    int model, what;
+};
+
+/* The log-likelihood of instance i (valid in lane 0) by one whole wave: lane l sums tiles l, l + 64, ... in order, then
+ * a fixed xor-shuffle tree; the order depends only on the instance's own tile count, so results do not depend on the
+ * batch. */
+__device__ __forceinline__ double gwh_finalize_instance(const FinalizeArgs &F, int i)
+{
+    /* The instance index is uniform over the wave (scalar loads).  Each lane's first tile record (every tile slot
+       lies inside the buffer) is requested first, then the loads that do not depend on each other (tile count,
+       event id, the instance's detector constants); slots at or past the tile count are added as zeros, so the
+       sums are those of the tiles in order, without a round trip for the count before the partial sums. */
+    const int lane = threadIdx.x & 63;
+    const size_t t0 = (size_t)i * F.W.tiles0;
+    double v0[GWH_PARTIAL_STRIDE];
+    const bool has0 = lane < F.W.tiles0; /* lanes without a tile slot read nothing */
+#pragma unroll
+    for (int j = 0; j < GWH_PARTIAL_STRIDE; j++) v0[j] = 0.0;
+    if (has0) {
+        const double *p = F.partial + (t0 + lane) * GWH_PARTIAL_STRIDE;
+#pragma unroll
+        for (int j = 0; j < GWH_PARTIAL_STRIDE; j++) v0[j] = p[j];
+    }
+    const int nt = F.active[i];
+    const int ev = F.W.inst_event ? F.W.inst_event[i] : F.W.event0;
+    const InstCoef &C = F.coefs[i];
+    double cdet[GWH_MAXDET][3];
+#pragma unroll
+    for (int d = 0; d < GWH_MAXDET; d++)
+        for (int q = 0; q < 3; q++) cdet[d][q] = C.det[d][q];
+    const EventDesc &E = F.events[ev];
+    if (nt < 0) return __longlong_as_double(0x7ff8000000000000ll); /* not evaluated (count or mask of the launch) */
+    /* every slot of a tile's partial record is summed (slots past 3 D are unused), so the loads need not wait
+       for the event's detector count */
+    double s[GWH_PARTIAL_STRIDE];
+    const bool use0 = has0 && lane < nt;
+#pragma unroll
+    for (int j = 0; j < GWH_PARTIAL_STRIDE; j++) s[j] = use0 ? v0[j] : 0.0;
+    for (int t = lane + 64; t < nt; t += 64) {
+        const double *p = F.partial + (t0 + t) * GWH_PARTIAL_STRIDE;
+#pragma unroll
+        for (int j = 0; j < GWH_PARTIAL_STRIDE; j++) s[j] += p[j];
+    }
+    const int D = E.D, nv = 3 * D;
+#pragma unroll
+    for (int j = 0; j < GWH_PARTIAL_STRIDE; j++)
+        if (j < nv) s[j] = wave_sum(s[j]);
+    double ll = 0;
+#pragma unroll
+    for (int d = 0; d < GWH_MAXDET; d++) {
+        if (d >= D) break;
+        double hh, dh;
+        if (!gwh_is_pv2(F.model)) {
+            double ha = s[3 * d], zr = s[3 * d + 1], zi = s[3 * d + 2];
+            hh = cdet[d][2] * ha;
+            dh = cdet[d][0] * zr + cdet[d][1] * zi;
+        } else {
+            hh = s[3 * d];
+            dh = s[3 * d + 1];
+        }
+        ll += (F.what == 0) ? -0.5 * (hh - 2 * dh) : hh;
+    }
+    /* what 1: network optimal SNR sqrt(sum_d (h_d|h_d)) with the SNR's Simpson step */
+    return (F.what == 0) ? ll : sqrt(ll * E.snr_scale);
+}
+
 struct Event {
     bool live = false;
     int N = 0, D = 0;
@@ -164,12 +243,14 @@ struct Scratch {
  *   d_mask        device ints, n: only instances with d_mask[i] != 0 are evaluated
  *   reserve_only  size the scratch buffers for this launch and return without launching
  *   capturing     the stream is being captured into a graph: no timing events are recorded
+ *   finalize_later  the last kernel (partial sums -> log-likelihoods) is left to the caller, with these arguments
  * Instances that are not evaluated get a NaN result. */
 struct LaunchExtra {
     const int *d_count = nullptr;
     const int *d_mask = nullptr;
     bool reserve_only = false;
     bool capturing = false;
+    FinalizeArgs *finalize_later = nullptr;
 };
 
 /* Device scratch and stream of one Fisher computation (the engine's own, or a broker worker's). */

@@ -818,76 +818,13 @@ __global__ __launch_bounds__(1024) void gwh_worklist_kernel(WorkMap W, const Eve
     }
 }
 
-/* One wave per instance: lane l sums tiles l, l + 64, ... in order, then a fixed xor-shuffle tree; the
- * order depends only on the instance's own tile count, so results do not depend on the batch. */
-__global__ __launch_bounds__(GWH_TPB) void gwh_finalize_kernel(WorkMap W, const EventDesc *__restrict__ events,
-                                                               const InstCoef *__restrict__ coefs,
-                                                               const double *__restrict__ partial,
-                                                               const int *__restrict__ active, int model, int what,
-                                                               double *__restrict__ logl, const int *__restrict__ count)
+__global__ __launch_bounds__(GWH_TPB) void gwh_finalize_kernel(FinalizeArgs F, double *__restrict__ logl,
+                                                               const int *__restrict__ count)
 {
-    /* The instance index is uniform over the wave (scalar loads).  Each lane's first tile record (every tile slot
-       lies inside the buffer) is requested first, then the loads that do not depend on each other (tile count,
-       event id, the instance's detector constants); slots at or past the tile count are added as zeros, so the
-       sums are those of the tiles in order, without a round trip for the count before the partial sums. */
     const int i = __builtin_amdgcn_readfirstlane(blockIdx.x * (GWH_TPB / 64) + (threadIdx.x >> 6));
-    const int lane = threadIdx.x & 63;
-    if (i >= W.n || (count && i >= *count)) return; /* whole waves leave together */
-    const size_t t0 = (size_t)i * W.tiles0;
-    double v0[GWH_PARTIAL_STRIDE];
-    const bool has0 = lane < W.tiles0; /* lanes without a tile slot read nothing */
-#pragma unroll
-    for (int j = 0; j < GWH_PARTIAL_STRIDE; j++) v0[j] = 0.0;
-    if (has0) {
-        const double *p = partial + (t0 + lane) * GWH_PARTIAL_STRIDE;
-#pragma unroll
-        for (int j = 0; j < GWH_PARTIAL_STRIDE; j++) v0[j] = p[j];
-    }
-    const int nt = active[i];
-    const int ev = W.inst_event ? W.inst_event[i] : W.event0;
-    const InstCoef &C = coefs[i];
-    double cdet[GWH_MAXDET][3];
-#pragma unroll
-    for (int d = 0; d < GWH_MAXDET; d++)
-        for (int q = 0; q < 3; q++) cdet[d][q] = C.det[d][q];
-    const EventDesc &E = events[ev];
-    if (nt < 0) { /* instance not evaluated (count or mask of the launch) */
-        if (lane == 0) logl[i] = __longlong_as_double(0x7ff8000000000000ll);
-        return;
-    }
-    /* every slot of a tile's partial record is summed (slots past 3 D are unused), so the loads need not wait
-       for the event's detector count */
-    double s[GWH_PARTIAL_STRIDE];
-    const bool use0 = has0 && lane < nt;
-#pragma unroll
-    for (int j = 0; j < GWH_PARTIAL_STRIDE; j++) s[j] = use0 ? v0[j] : 0.0;
-    for (int t = lane + 64; t < nt; t += 64) {
-        const double *p = partial + (t0 + t) * GWH_PARTIAL_STRIDE;
-#pragma unroll
-        for (int j = 0; j < GWH_PARTIAL_STRIDE; j++) s[j] += p[j];
-    }
-    const int D = E.D, nv = 3 * D;
-#pragma unroll
-    for (int j = 0; j < GWH_PARTIAL_STRIDE; j++)
-        if (j < nv) s[j] = wave_sum(s[j]);
-    if (lane != 0) return;
-    double ll = 0;
-#pragma unroll
-    for (int d = 0; d < GWH_MAXDET; d++) {
-        if (d >= D) break;
-        double hh, dh;
-        if (!gwh_is_pv2(model)) {
-            double ha = s[3 * d], zr = s[3 * d + 1], zi = s[3 * d + 2];
-            hh = cdet[d][2] * ha;
-            dh = cdet[d][0] * zr + cdet[d][1] * zi;
-        } else {
-            hh = s[3 * d];
-            dh = s[3 * d + 1];
-        }
-        ll += (what == 0) ? -0.5 * (hh - 2 * dh) : hh;
-    }
-    /* what 1: network optimal SNR sqrt(sum_d (h_d|h_d)) with the SNR's Simpson step */
-    logl[i] = (what == 0) ? ll : sqrt(ll * E.snr_scale);
+    if (i >= F.W.n || (count && i >= *count)) return; /* whole waves leave together */
+    const double ll = gwh_finalize_instance(F, i);
+    if ((threadIdx.x & 63) == 0) logl[i] = ll;
 }
 
 int gwh_choose_bpl(int N)
@@ -1042,9 +979,13 @@ int gwh_loglike_launch(const int *d_events, int events0, int model, int precisio
     GWH_HIP(hipGetLastError());
     if (timed) GWH_HIP(hipEventRecord(E.ev1, stream));
     if (live) GWH_HIP(hipEventRecord(E.kt_ev[2 * E.kt_used++ + 1], stream));
-    hipLaunchKernelGGL(gwh_finalize_kernel, dim3((n + GWH_TPB / 64 - 1) / (GWH_TPB / 64)), dim3(GWH_TPB), 0, stream,
-                       W, evp, cp,
-                       (const double *)pp, ap, model, what, d_logl, X.d_count);
+    const FinalizeArgs F{W, evp, cp, pp, ap, model, what};
+    if (X.finalize_later) { /* the caller's own kernel takes it from here */
+        *X.finalize_later = F;
+        return GWH_OK;
+    }
+    hipLaunchKernelGGL(gwh_finalize_kernel, dim3((n + GWH_TPB / 64 - 1) / (GWH_TPB / 64)), dim3(GWH_TPB), 0, stream, F,
+                       d_logl, X.d_count);
     GWH_HIP(hipGetLastError());
     if (timed && kernel_ms) {
         GWH_HIP(hipEventSynchronize(E.ev1));

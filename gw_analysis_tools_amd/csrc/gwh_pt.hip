@@ -88,7 +88,6 @@ struct PtArgs {
     double *theta, *ll;    /* current states */
     double *prop, *llp;    /* this step's proposals and their log-likelihoods */
     double *logu;          /* n: this step's log U */
-    double *tmp;           /* n x dim: ladder permutation staging */
     gwh_params *params;    /* n: records of the proposals */
     int *mask;             /* n: proposal inside the prior box */
     int *acc;              /* n: 1 accepted, 0 rejected, 2 pending FP64 re-decision */
@@ -124,11 +123,15 @@ __global__ void gwh_pt_init_kernel(PtArgs a)
 }
 
 /* gaussian_step (mcmc_sampler_internals.cpp:364-409): one dimension chosen uniformly, moved by
- * width * N(0, 1); the prior box decides whether the likelihood is needed at all (mcmc_step :83-92) */
+ * width * N(0, 1); the prior box decides whether the likelihood is needed at all (mcmc_step :83-92).
+ * 64 chains per block, four waves with one lane of each per chain: all draw the proposal, then wave 0 writes it with
+ * log U and the mask, waves 1 to 3 a part of its record each (repack_part), so the logarithms, powers and arctangents
+ * run side by side: with one lane per chain the step's chain of them took 11.2 us, now 5.6. */
 __global__ __launch_bounds__(256) void gwh_pt_propose_kernel(PtArgs a)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i == 0) {
+    const int role = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i = blockIdx.x * 64 + (threadIdx.x & 63);
+    if (i == 0 && role == 0) {
         a.gcount[0] = 0;
         a.gcount[1] = 0;
     }
@@ -140,35 +143,36 @@ __global__ __launch_bounds__(256) void gwh_pt_propose_kernel(PtArgs a)
     const int beta = (int)(((uint64_t)A.x * (uint64_t)a.dim) >> 32);
     const double u1 = u53(A.y, A.z), u2 = u53(A.w, B.x);
     const double z = sqrt(-2.0 * log(1.0 - u1)) * cospi(2.0 * u2);
-    a.logu[i] = log(u53(B.y, B.z));
     const double *th = a.theta + (size_t)i * a.dim;
-    double *pr = a.prop + (size_t)i * a.dim;
+    const double t_beta = th[beta], x_beta = __dadd_rn(__dmul_rn(a.width[(size_t)i * a.dim + beta], z), t_beta);
     /* fixed trip count: every index of v is a compile-time constant, so v lives in registers */
-    double v[GWH_PT_MAXDIM], t_beta = 0;
+    double v[GWH_PT_MAXDIM];
     int ok = 1;
 #pragma unroll
-    for (int d = 0; d < GWH_PT_MAXDIM; d++) {
-        v[d] = 0;
-        if (d < a.dim) {
-            double x = th[d];
-            if (d == beta) {
-                t_beta = x;
-                x = __dadd_rn(__dmul_rn(a.width[(size_t)i * a.dim + d], z), x);
-            }
-            v[d] = x;
-            pr[d] = x;
-            ok &= (x >= a.lower[d]) & (x <= a.upper[d]);
-        }
-    }
-    a.mask[i] = ok;
-    if (!ok) { /* outside the prior box: the record of the current state (its likelihood is not used) */
+    for (int d = 0; d < GWH_PT_MAXDIM; d++) v[d] = d < a.dim ? th[d] : 0.0;
 #pragma unroll
-        for (int d = 0; d < GWH_PT_MAXDIM; d++)
-            if (d == beta) v[d] = t_beta;
+    for (int d = 0; d < GWH_PT_MAXDIM; d++) {
+        if (d >= a.dim) break;
+        v[d] = (d == beta) ? x_beta : v[d];
+        if (role == 0) a.prop[(size_t)i * a.dim + d] = v[d];
+        ok &= (v[d] >= a.lower[d]) & (v[d] <= a.upper[d]);
     }
+    if (role == 0) {
+        a.mask[i] = ok;
+        a.logu[i] = log(u53(B.y, B.z));
+        return;
+    }
+    /* outside the prior box: the record of the current state (its likelihood is not used) */
+#pragma unroll
+    for (int d = 0; d < GWH_PT_MAXDIM; d++) v[d] = (!ok && d == beta) ? t_beta : v[d];
     /* a.params[i] holds the template's other fields since the init kernel: only the sampled ones change (the
      * sampling bases' repack reads no field of the record) */
-    repack(v, a.basis, a.params[i]);
+    if (role == 1)
+        repack_part(v, a.basis, 0, a.params[i]);
+    else if (role == 2)
+        repack_part(v, a.basis, 1, a.params[i]);
+    else
+        repack_part(v, a.basis, 2, a.params[i]);
 }
 
 /* Metropolis-Hastings (mcmc_sampler_internals.cpp:96-142): reject iff (ll' - ll) / T < log U; a proposal
@@ -187,16 +191,20 @@ __device__ __forceinline__ bool mh_accept(double ratio, double logu)
     return ratio > -INFINITY && !(ratio < logu);
 }
 
-__global__ void gwh_pt_accept_kernel(PtArgs a)
+/* The proposals' log-likelihoods from their tiles' partial sums (gwh_finalize_instance, one wave per chain), each followed
+ * by its decision in lane 0 -- one launch instead of two -- and the step counter's advance: nothing in this kernel reads
+ * it, the swaps that follow take it less one. */
+__global__ __launch_bounds__(256) void gwh_pt_accept_kernel(PtArgs a, FinalizeArgs F)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+    if (blockIdx.x == 0 && threadIdx.x == 0) ++*a.step;
     if (i >= a.n) return;
+    double lp = gwh_finalize_instance(F, i);
+    if ((threadIdx.x & 63) != 0) return;
+    if (i < (a.nt - 1) * a.nc) a.swp[i] = 0; /* no swap so far in this step */
     const double T = pt_T(a, i), lu = a.logu[i];
-    double lp = a.llp[i];
-    if (!a.mask[i]) {
-        lp = __longlong_as_double(0x7ff8000000000000ll);
-        a.llp[i] = lp;
-    }
+    if (!a.mask[i]) lp = __longlong_as_double(0x7ff8000000000000ll);
+    a.llp[i] = lp;
     const double ratio = (lp == lp) ? (-a.ll[i] + lp) / T : -INFINITY;
     const double margin = ratio - lu;
     if (a.guard && ratio > -INFINITY && isfinite(margin) && fabs(margin) < 2.0 * a.tol / T) {
@@ -223,91 +231,98 @@ __global__ void gwh_pt_accept_guard_kernel(PtArgs a)
 }
 
 /* chain_swap / single_chain_swap (mcmc_sampler_internals.cpp:1086-1180): pairs (k, k+1) of one ladder in
- * increasing k; reject iff exp((ll1 - ll2) / T2 - (ll1 - ll2) / T1) < U.  perm[k] = the temperature index
- * whose state (at the start of the swaps) sits at temperature k. */
-__device__ int pt_ladder(const PtArgs &a, int c, long long s, const double *ll64, int *perm, int *flag)
+ * increasing k; reject iff exp((ll1 - ll2) / T2 - (ll1 - ll2) / T1) < U.
+ *
+ * One wave per ladder.  At pair k the state at temperature k + 1 is the one it started with and the state at k one of
+ * those of temperatures 0..k, so the lanes decide every (pair, state) combination side by side (120 for 16 temperatures,
+ * at most 2016), and lane 0 walks the ladder through the table of decisions; then all lanes move the states.  With one
+ * lane per ladder, each walking its pairs' divisions and exponentials and moving its rows alone, a swap took 100 us for
+ * 32 ladders of 16 temperatures, now 7.3.
+ *
+ * ll64: FP64 log-likelihoods of the ladder's states by temperature; without them a decision inside the guard band on the
+ * walk ends it (-> the states are queued for FP64 evaluation). */
+struct LadderShared {
+    double ll[GWH_PT_MAXTEMPS], T[GWH_PT_MAXTEMPS], theta[GWH_PT_MAXTEMPS * GWH_PT_MAXDIM];
+    unsigned char how[GWH_PT_MAXTEMPS][GWH_PT_MAXTEMPS]; /* pair k, state j: 1 swap, 2 undecided in this precision */
+    int perm[GWH_PT_MAXTEMPS], flag[GWH_PT_MAXTEMPS], slot;
+};
+
+__device__ void pt_ladder(const PtArgs &a, int c, long long s, const double *ll64, LadderShared &sh)
 {
+    const int lane = threadIdx.x, nt = a.nt;
+    if (lane < nt) {
+        sh.ll[lane] = a.ll[lane * a.nc + c];
+        sh.T[lane] = a.temps[lane];
+    }
+    for (int e = lane; e < nt * a.dim; e += 64) sh.theta[e] = a.theta[(size_t)((e / a.dim) * a.nc + c) * a.dim + e % a.dim];
+    __syncthreads();
     const uint32_t slo = (uint32_t)s, shi = (uint32_t)((unsigned long long)s >> 32);
-    for (int k = 0; k < a.nt; k++) perm[k] = k;
-    for (int k = 0; k + 1 < a.nt; k++) {
-        const double T1 = a.temps[k], T2 = a.temps[k + 1];
-        flag[k] = 0;
-        if (T1 == T2) continue;
+    for (int p = lane; p < nt * (nt - 1) / 2; p += 64) {
+        int k = (int)((sqrtf(8.0f * p + 1.0f) - 1.0f) * 0.5f); /* p = k (k + 1) / 2 + j, 0 <= j <= k < nt - 1 */
+        while (k * (k + 1) / 2 > p) k--;
+        while ((k + 1) * (k + 2) / 2 <= p) k++;
+        const int j = p - k * (k + 1) / 2;
         const U4 C = philox4x32_10(U4{(uint32_t)(k * a.nc + c), slo, shi, 2u}, a.key0, a.key1);
         const double alpha = u53(C.x, C.y);
-        const double l1 = a.ll[perm[k] * a.nc + c], l2 = a.ll[perm[k + 1] * a.nc + c];
+        const double T1 = sh.T[k], T2 = sh.T[k + 1], l1 = sh.ll[j], l2 = sh.ll[k + 1];
         double pw = (l1 - l2) / T2 - (l1 - l2) / T1;
-        if (a.guard && alpha > 0 && fabs(pw - log(alpha)) < 2.0 * a.tol * fabs(1.0 / T2 - 1.0 / T1)) {
-            if (!ll64) return -1; /* FP64 values of this ladder's states are needed */
-            const double m1 = ll64[perm[k]], m2 = ll64[perm[k + 1]];
+        bool near = a.guard && alpha > 0 && fabs(pw - log(alpha)) < 2.0 * a.tol * fabs(1.0 / T2 - 1.0 / T1);
+        if (near && ll64) {
+            const double m1 = ll64[j], m2 = ll64[k + 1];
             pw = (m1 - m2) / T2 - (m1 - m2) / T1;
+            near = false;
         }
-        if (!(exp(pw) < alpha)) {
-            const int t = perm[k];
-            perm[k] = perm[k + 1];
-            perm[k + 1] = t;
-            flag[k] = 1;
-        }
+        sh.how[k][j] = near ? 2 : !(exp(pw) < alpha);
     }
-    return 0;
-}
-
-__device__ void pt_permute(const PtArgs &a, int c, const int *perm, const int *flag)
-{
-    double lv[GWH_PT_MAXTEMPS];
-    for (int k = 0; k < a.nt; k++) {
-        const int i = k * a.nc + c;
-        lv[k] = a.ll[i];
-        for (int d = 0; d < a.dim; d++) a.tmp[(size_t)i * a.dim + d] = a.theta[(size_t)i * a.dim + d];
-    }
-    for (int k = 0; k < a.nt; k++) {
-        const int i = k * a.nc + c, j = perm[k] * a.nc + c;
-        a.ll[i] = lv[perm[k]];
-        for (int d = 0; d < a.dim; d++) a.theta[(size_t)i * a.dim + d] = a.tmp[(size_t)j * a.dim + d];
-    }
-    for (int k = 0; k + 1 < a.nt; k++) {
-        a.swp[k * a.nc + c] = flag[k];
-        a.swap_count[k * a.nc + c] += flag[k];
-    }
-}
-
-/* one block of n_chains threads; the last kernel of a step advances the step counter */
-__global__ __launch_bounds__(1024) void gwh_pt_swap_kernel(PtArgs a, int last)
-{
-    const int c = threadIdx.x;
-    const long long s = *a.step;
-    const bool swap_step = a.swap_every > 0 && (s + 1) % a.swap_every == 0;
-    if (c < a.nc) {
-        a.lslot[c] = -1;
-        int perm[GWH_PT_MAXTEMPS], flag[GWH_PT_MAXTEMPS];
-        for (int k = 0; k + 1 < a.nt; k++) a.swp[k * a.nc + c] = 0;
-        if (swap_step) {
-            if (pt_ladder(a, c, s, nullptr, perm, flag) == 0) {
-                pt_permute(a, c, perm, flag);
-            } else {
-                const int slot = atomicAdd(&a.gcount[1], a.nt);
-                a.lslot[c] = slot;
-                for (int k = 0; k < a.nt; k++)
-                    a.lparams[slot + k] = pt_record(a, a.theta + (size_t)(k * a.nc + c) * a.dim);
+    __syncthreads();
+    if (lane == 0) {
+        int cur = 0; /* the temperature whose state has come to temperature k */
+        sh.slot = -1;
+        for (int k = 0; k + 1 < nt; k++) {
+            const int how = (sh.T[k] == sh.T[k + 1]) ? 0 : sh.how[k][cur];
+            if (how == 2) { /* FP64 values of this ladder's states are needed */
+                sh.slot = atomicAdd(&a.gcount[1], nt);
+                break;
             }
+            sh.flag[k] = how;
+            sh.perm[k] = how ? k + 1 : cur;
+            if (!how) cur = k + 1;
         }
+        sh.perm[nt - 1] = cur;
     }
     __syncthreads();
-    if (last && threadIdx.x == 0) *a.step = s + 1;
+    if (sh.slot >= 0) {
+        if (lane == 0) a.lslot[c] = sh.slot;
+        if (lane < nt) a.lparams[sh.slot + lane] = pt_record(a, a.theta + (size_t)(lane * a.nc + c) * a.dim);
+        return;
+    }
+    if (lane < nt) a.ll[lane * a.nc + c] = sh.ll[sh.perm[lane]];
+    for (int e = lane; e < nt * a.dim; e += 64)
+        a.theta[(size_t)((e / a.dim) * a.nc + c) * a.dim + e % a.dim] = sh.theta[sh.perm[e / a.dim] * a.dim + e % a.dim];
+    if (lane + 1 < nt) {
+        a.swp[lane * a.nc + c] = sh.flag[lane];
+        a.swap_count[lane * a.nc + c] += sh.flag[lane];
+    }
 }
 
-__global__ __launch_bounds__(1024) void gwh_pt_swap_guard_kernel(PtArgs a)
+/* one block of one wave per ladder; the accept kernel has advanced the step counter */
+__global__ __launch_bounds__(64) void gwh_pt_swap_kernel(PtArgs a)
 {
-    const int c = threadIdx.x;
-    const long long s = *a.step;
-    if (c < a.nc && a.lslot[c] >= 0) {
-        int perm[GWH_PT_MAXTEMPS], flag[GWH_PT_MAXTEMPS];
-        pt_ladder(a, c, s, a.lll + a.lslot[c], perm, flag);
-        pt_permute(a, c, perm, flag);
-        atomicAdd(a.guard_evals, (unsigned long long)a.nt);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) *a.step = s + 1;
+    __shared__ LadderShared sh;
+    const int c = blockIdx.x, lane = threadIdx.x;
+    const long long s = *a.step - 1;
+    if (lane == 0) a.lslot[c] = -1;
+    if (a.swap_every > 0 && (s + 1) % a.swap_every == 0) pt_ladder(a, c, s, nullptr, sh);
+}
+
+__global__ __launch_bounds__(64) void gwh_pt_swap_guard_kernel(PtArgs a)
+{
+    __shared__ LadderShared sh;
+    const int c = blockIdx.x;
+    const int slot = a.lslot[c];
+    if (slot < 0) return; /* the whole block */
+    pt_ladder(a, c, *a.step - 1, a.lll + slot, sh);
+    if (threadIdx.x == 0) atomicAdd(a.guard_evals, (unsigned long long)a.nt);
 }
 
 /* ------------------------------------------------------------------------- */
@@ -543,7 +558,7 @@ int gwh_pt_create(int event, const gwh_pt_config *cfg, const double *temps, cons
 
     /* one allocation: doubles, then records, then 8-byte counters, then ints */
     const size_t nd = (size_t)nt + (size_t)n * dim + 2 * dim + 1 /* tmpl slot (aligned) */ + 2 * (size_t)n * dim +
-                      3 * (size_t)n + (size_t)n * dim + 2 * (size_t)n + (size_t)n;
+                      3 * (size_t)n + 2 * (size_t)n + (size_t)n;
     const size_t nrec = (size_t)n + 2 * (size_t)n + (size_t)n + 1;
     const size_t ncnt = (size_t)n + (size_t)(nt - 1) * nc + 2;
     const size_t nint = (size_t)n * 3 + (size_t)(nt - 1) * nc + 2 + (size_t)n + (size_t)nc;
@@ -579,7 +594,6 @@ int gwh_pt_create(int event, const gwh_pt_config *cfg, const double *temps, cons
     a.ll = (double *)take(n * 8);
     a.llp = (double *)take(n * 8);
     a.logu = (double *)take(n * 8);
-    a.tmp = (double *)take((size_t)n * dim * 8);
     a.gll = (double *)take(2 * (size_t)n * 8);
     a.lll = (double *)take((size_t)n * 8);
     gwh_params *d_tmpl = (gwh_params *)take(sizeof(gwh_params));
@@ -636,17 +650,18 @@ int gwh_pt_create(int event, const gwh_pt_config *cfg, const double *temps, cons
     if (hipStreamSynchronize(s) != hipSuccess) return fail(gwh_set_error(GWH_ERR_HIP, "initial likelihoods failed"));
 
     x.capturing = true;
-    const int nsw = std::max(nc, 64);
     rc = capture(*g, [&]() -> int {
         int r;
         for (int k = 0; k < g->steps_per_graph; k++) {
-            hipLaunchKernelGGL(gwh_pt_propose_kernel, blocks_of(n), dim3(256), 0, s, a);
+            hipLaunchKernelGGL(gwh_pt_propose_kernel, dim3((n + 63) / 64), dim3(256), 0, s, a);
             LaunchExtra m = x;
+            FinalizeArgs fin;
             m.d_mask = a.mask;
+            m.finalize_later = &fin;
             if ((r = gwh_loglike_launch(nullptr, event, M, P, a.params, n, a.llp, s, false, nullptr, nullptr, 0,
                                         &g->scr, &m)) != GWH_OK)
                 return r;
-            hipLaunchKernelGGL(gwh_pt_accept_kernel, blocks_of(n), dim3(256), 0, s, a);
+            hipLaunchKernelGGL(gwh_pt_accept_kernel, dim3((n + 3) / 4), dim3(256), 0, s, a, fin);
             if (guard) {
                 LaunchExtra c0 = x;
                 c0.d_count = a.gcount;
@@ -655,14 +670,18 @@ int gwh_pt_create(int event, const gwh_pt_config *cfg, const double *temps, cons
                     return r;
                 hipLaunchKernelGGL(gwh_pt_accept_guard_kernel, blocks_of(n), dim3(256), 0, s, a);
             }
-            hipLaunchKernelGGL(gwh_pt_swap_kernel, dim3(1), dim3(nsw), 0, s, a, guard ? 0 : 1);
-            if (guard) {
+            /* runs advance by whole graphs from step 0, so with a swap interval that divides the graph's steps the place
+               in the graph tells whether a step swaps; otherwise the kernel asks the step counter */
+            const bool swaps = cfg->swap_every > 0 && nt > 1 &&
+                               (g->steps_per_graph % cfg->swap_every != 0 || (k + 1) % cfg->swap_every == 0);
+            if (swaps) hipLaunchKernelGGL(gwh_pt_swap_kernel, dim3(nc), dim3(64), 0, s, a);
+            if (swaps && guard) {
                 LaunchExtra c1 = x;
                 c1.d_count = a.gcount + 1;
                 if ((r = gwh_loglike_launch(nullptr, event, M, GWH_FP64, a.lparams, n, a.lll, s, false, nullptr,
                                             nullptr, 0, &g->scr, &c1)) != GWH_OK)
                     return r;
-                hipLaunchKernelGGL(gwh_pt_swap_guard_kernel, dim3(1), dim3(nsw), 0, s, a);
+                hipLaunchKernelGGL(gwh_pt_swap_guard_kernel, dim3(nc), dim3(64), 0, s, a);
             }
             GWH_HIP(hipGetLastError());
         }

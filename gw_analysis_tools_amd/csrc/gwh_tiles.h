@@ -53,11 +53,6 @@ __device__ __forceinline__ void block_reduce_store(double (&acc)[NV], double *__
 /* the batched likelihood kernels                                             */
 /* ------------------------------------------------------------------------- */
 
-struct WorkMap {
-    const int *inst_event; /* NULL: every instance uses event0 */
-    int event0, n, tiles0; /* tiles0: tile stride of the partial buffer */
-};
-
 /* One (instance, tile) work item: TPB lanes x BPL bins of one instance's network log-likelihood, reduced
  * to the instance's partial sums for that tile.  Every early return is uniform over the block.
  * ANY: an item of a work list, whose event has TPB lanes and any number of bins per lane up to BPL = 8 (the unrolled
