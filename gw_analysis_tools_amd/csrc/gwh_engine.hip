@@ -416,12 +416,16 @@ int gwh_event_create_ex(const double *f, int N, int ndet, const int *dets, const
 /* setup                                                                      */
 /* ------------------------------------------------------------------------- */
 
-/* 64 instances per block, four waves (roles) per instance group: each lane computes one part of its
+/* GWH_SETUP_LANES instances per block, four waves (roles) per instance group: each lane computes one part of its
  * instance's record, the parts meet in LDS (see gwh_model.h for the split).  256 threads per block leave
  * each lane the whole register file of its SIMD, so the FP64 working set needs no scratch memory.  Every
- * wave reaches both barriers; lanes without an instance only skip the work.  MOD: the ppE / gIMR / theory
- * modifications are compiled in (the GR models run a kernel without them, which keeps its registers and
+ * wave reaches both barriers; lanes without an instance only skip the work.  Half-filled waves: the records' stores,
+ * 119 of 8 bytes 952 bytes apart per lane, go through twice as many CUs (512 instances 11.3 -> 10.0 us; with a quarter of
+ * the lanes the fetch of the code by ever more CUs costs more than that saves: 11.0, an eighth 15.4).  MOD: the ppE / gIMR /
+ * theory modifications are compiled in (the GR models run a kernel without them, which keeps its registers and
  * code to what GR needs). */
+#define GWH_SETUP_LANES 32
+#pragma clang fp contract(on)
 template <int MODEL, bool MOD>
 __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__restrict__ params,
                                                         const int *__restrict__ inst_event, int event0, int n,
@@ -433,17 +437,17 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__rest
                                                         int ppe_variant)
 {
     const int ppe = MOD ? ppe_variant : 0;
-    __shared__ SetupShared sh[64];
+    __shared__ SetupShared sh[GWH_SETUP_LANES];
     constexpr bool pv2 = (MODEL == GWH_IMRPHENOMPV2);
     const int lane = threadIdx.x & 63;
     const int role = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int i = blockIdx.x * 64 + lane;
-    bool live = i < n;
+    const int i = blockIdx.x * GWH_SETUP_LANES + lane;
+    bool live = lane < GWH_SETUP_LANES && i < n;
     if (live && ((d_count && i >= *d_count) || (d_mask && !d_mask[i]))) {
         if (active && role == 2) active[i] = -1; /* not evaluated: no tiles, NaN result */
         live = false;
     }
-    SetupShared &X = sh[lane];
+    SetupShared &X = sh[lane & (GWH_SETUP_LANES - 1)];
     InstCoef *C = coef + (live ? i : 0);
     gwh_params p;
     SetupState S;
@@ -458,12 +462,15 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__rest
         if (role == 0) {
             const double chip = pv2 ? gwh_setup_chip(p, S) : -1;
             gwh_setup_ringdown(p, pv2, chip, &gwh_phenomd_fit[0][0], qnm, S);
-            gwh_setup_amp_mr(S, S.f3, &X.v3, &X.d3);
+            const double wd = S.g[2] * S.fdamp, iw = 1.0 / wd;
+            gwh_setup_amp_mr(S, S.f3, iw, &X.v3, &X.d3);
             SetupState &T = X.S; /* base, ringdown fits and frequencies */
             T.m1 = S.m1;
             T.m2 = S.m2;
             T.M = S.M;
             T.eta = S.eta;
+            T.ieta = S.ieta;
+            T.iM = S.iM;
             T.chi1 = S.chi1;
             T.chi2 = S.chi2;
             T.chi_s = S.chi_s;
@@ -492,24 +499,25 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__rest
             C->fRD = S.fRD;
             C->fdamp = S.fdamp;
             C->inv_fdamp = 1.0 / S.fdamp;
-            C->mr_k = S.g[0] * S.g[2] * S.fdamp / S.M;
-            C->mr_g2 = S.g[1] / (S.g[2] * S.fdamp);
-            C->mr_w2 = (S.g[2] * S.fdamp) * (S.g[2] * S.fdamp);
+            C->mr_k = S.g[0] * wd * S.iM;
+            C->mr_g2 = S.g[1] * iw;
+            C->mr_w2 = wd * wd;
         } else if (role == 1) {
             gwh_setup_pn(p, S);
             const double xfit = S.chi_pn - 1;
             for (int k = 0; k < 3; k++) S.rho[k] = gwh_fit(&gwh_phenomd_fit[0][0], k, S.eta, xfit);
-            gwh_setup_amp_ins(S, 0.014 / S.M, &X.v1, &X.d1);
+            gwh_setup_amp_ins_f1(S, &X.v1, &X.d1);
             for (int k = 0; k < 3; k++) X.S.rho[k] = S.rho[k];
             for (int k = 0; k < 7; k++) X.S.pa[k] = S.pa[k];
             for (int k = 0; k < 12; k++) X.S.pp[k] = S.pp[k];
-            double pi13 = cbrt(GWH_PI), pw = 1.0;
+            double pw = 1.0;
+#pragma unroll
             for (int k = 0; k < 7; k++) {
                 C->ca[k] = S.pa[k] * pw;
-                pw *= pi13;
+                pw *= 1.4645918875615231; /* pi^{1/3} */
             }
             for (int k = 0; k < 3; k++) C->rho[k] = S.rho[k];
-            C->K = 3. / (128. * S.eta);
+            C->K = 3. / (128. * S.eta); /* scales a phase of up to 1e4 rad: one rounding, not two */
             for (int k = 0; k < 8; k++) C->cp[k] = S.pp[k];
             C->c8 = S.pp[8];
             C->c9 = S.pp[9];
@@ -518,13 +526,14 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__rest
             C->gimr = S.gimr;
             for (int k = 0; k < 4; k++) C->gimr_neg[k] = S.gimr_neg[k];
         } else if (role == 2) {
-            double zeta = 0;
+            double c2z = 1, s2z = 0;
             if (pv2) {
                 const Pv2Frame F = gwh_setup_frame(p, S, gwh_setup_chip(p, S));
                 X.alpha0 = F.alpha0;
                 X.phi_aligned = F.phi_aligned;
-                zeta = F.zeta;
-                double ct = cos(F.thetaJN), st = sin(F.thetaJN);
+                c2z = F.c2z;
+                s2z = F.s2z;
+                const double ct = F.cJN, st = F.sJN;
                 /* sums and differences of -2Y_2m(thetaJN, 0), m and -m (gwh_pv2_twist) */
                 C->tw[0] = sqrt(5.0 / (64.0 * GWH_PI)) * 2.0 * (1.0 + ct * ct);
                 C->tw[1] = sqrt(5.0 / (64.0 * GWH_PI)) * 4.0 * ct;
@@ -533,7 +542,7 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__rest
                 C->tw[4] = sqrt(15.0 / (32.0 * GWH_PI)) * (GWH_SQRT_6 / 2.0) * st * st;
             }
             const EventDesc &E = events[ev];
-            gwh_setup_detectors(p, pv2, zeta, geo, E.det, E.D, *C);
+            gwh_setup_detectors(p, pv2, c2z, s2z, geo, E.det, E.D, *C);
         } else {
             X.alpha1_fit = gwh_setup_phase_fits(p, &gwh_phenomd_fit[0][0], S);
             {
@@ -543,10 +552,10 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__rest
                 for (int k = 0; k < 4; k++) T.beta[k] = S.beta[k];
                 for (int k = 0; k < 6; k++) T.alpha[k] = S.alpha[k];
             }
-            C->sig[0] = S.sigma[1] / S.eta;
-            C->sig[1] = 0.75 * S.sigma[2] / S.eta;
-            C->sig[2] = 0.6 * S.sigma[3] / S.eta;
-            C->sig[3] = 0.5 * S.sigma[4] / S.eta;
+            C->sig[0] = S.sigma[1] * S.ieta;
+            C->sig[1] = 0.75 * S.sigma[2] * S.ieta;
+            C->sig[2] = 0.6 * S.sigma[3] * S.ieta;
+            C->sig[3] = 0.5 * S.sigma[4] * S.ieta;
             gwh_setup_mass(p, ppe, S);
             X.S.Mc = S.Mc;
             X.S.A0 = S.A0;
@@ -554,11 +563,11 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__rest
                 X.S.ppe_e[k] = S.ppe_e[k];
                 X.S.ppe_c[k] = S.ppe_c[k];
             }
-            const double M76 = pow(S.M, 7. / 6.);
-            C->amp_pref = pv2 ? S.A0 * M76 / (2. * sqrt(5. / (64. * GWH_PI))) / 2. : S.A0 * M76;
-            C->M13 = cbrt(S.M);
-            C->Mm13 = 1.0 / C->M13;
-            C->Mm76 = 1.0 / (S.M * sqrt(C->M13));
+            const double M13 = cbrt(S.M), M76 = S.M * sqrt(M13);
+            C->amp_pref = pv2 ? S.A0 * M76 * (1. / (4. * sqrt(5. / (64. * GWH_PI)))) : S.A0 * M76;
+            C->M13 = M13;
+            C->Mm13 = 1.0 / M13;
+            C->Mm76 = 1.0 / M76;
             C->M34 = sqrt(sqrt(S.M * S.M * S.M));
             C->lgM = log(S.M);
             C->lgPiM = log(GWH_PI * S.M);
@@ -571,12 +580,12 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__rest
             if (pv2) { /* precession constants (IMRPhenomP.cpp:64-144, :1081-1211) */
                 const double chip = gwh_setup_chip(p, S);
                 const double q = S.m1 / S.m2;
-                const double chil = (1.0 + q) / q * S.chi_eff;
-                const double mm1 = q / (1 + q), mm2 = 1. / (1 + q);
+                const double chil = S.chi_eff * S.M / S.m1;
+                const double mm1 = S.m1 * S.iM, mm2 = S.m2 * S.iM;
                 C->SP = chip * mm1 * mm1;
                 C->SL = S.chi1 * mm1 * mm1 + S.chi2 * mm2 * mm2;
                 C->L_c1 = 1.5 + S.eta / 6.0;
-                C->L_c2 = 3.375 - (19.0 * S.eta) / 8. - S.eta * S.eta / 24.0;
+                C->L_c2 = 3.375 - (19.0 / 8.) * S.eta - S.eta * S.eta / 24.0;
                 double a_c[5], e_c[5];
                 gwh_euler_coeffs(q, chil, chip, a_c, e_c);
                 for (int k = 0; k < 5; k++) {
@@ -584,7 +593,7 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__rest
                     C->e_c[k] = e_c[k];
                 }
                 double vr = cbrt(GWH_PI * S.M * p.f_ref);
-                double lw = log(vr * vr * vr);
+                double lw = log(GWH_PI * S.M * p.f_ref);
                 const double ivr = rcp_newton(vr);
                 eul_a = gwh_euler_eval(a_c, vr, ivr, lw);
                 eul_e = gwh_euler_eval(e_c, vr, ivr, lw);
@@ -636,17 +645,16 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__rest
         S.beta[0] = S.beta[1] = 0;
         S.alpha[0] = S.alpha[1] = 0;
         if (role == 0) {
-            X.p_ins = gwh_setup_phase_ins(S, S.f1p);
-            X.l1 = log(S.M * S.f1p);
+            X.p_ins = gwh_setup_phase_ins_at(S, S.f1p, GWH_MF1P_V, 1.0 / GWH_MF1P_V, GWH_MF1P_LNPI, GWH_MF1P_U, GWH_MF1P);
+            X.d_ins = gwh_setup_dphase_ins_f1p(S);
         } else if (role == 1) {
-            X.d_ins = gwh_setup_dphase_ins(S, S.f1p);
-            X.l2 = log(S.M * S.f2p);
+            double dl[5];
+            gwh_setup_amp_connection(S.iM, S.f1, S.f3, X.v1, X.d1, S.v2, X.v3, X.d3, dl);
+            for (int k = 0; k < 5; k++) C->delta[k] = dl[k];
         } else if (role == 2) {
             X.q_mr = gwh_setup_phase_mr(S, S.f2p);
             X.dq_mr = gwh_setup_dphase_mr(S, S.f2p);
-            double dl[5];
-            gwh_setup_amp_connection(S.M, S.f1, S.f3, X.v1, X.d1, S.v2, X.v3, X.d3, dl);
-            for (int k = 0; k < 5; k++) C->delta[k] = dl[k];
+            X.l2 = log(S.M * S.f2p);
         } else {
             if (!pv2) {
                 if (p.shift_phase) {
@@ -667,21 +675,22 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__rest
 
     /* ---- phase 3: the phase connection (IMRPhenomD.cpp:1614-1674) and the alignment ---- */
     if (live && role == 0) {
-        const double eta = S.eta, M = S.M;
-        S.beta[1] = (eta / M) * X.d_ins - (eta / M) * gwh_setup_dphase_int(S, S.f1p);
-        S.beta[0] = eta * X.p_ins - eta * gwh_setup_phase_int_l(S, S.f1p, X.l1);
-        S.alpha[1] = (eta / M) * gwh_setup_dphase_int(S, S.f2p) - (eta / M) * X.dq_mr;
-        S.alpha[0] = eta * gwh_setup_phase_int_l(S, S.f2p, X.l2) -
-                     eta * (X.q_mr + (1. / eta) * (S.alpha[1] * (M * S.f2p)));
-        C->beta[0] = S.beta[0] / eta;
-        C->beta[1] = S.beta[1] / eta;
-        C->beta[2] = S.beta[2] / eta;
-        C->beta[3] = S.beta[3] / (3. * eta);
-        C->alpha[0] = S.alpha[0] / eta;
-        C->alpha[1] = S.alpha[1] / eta;
-        C->alpha[2] = S.alpha[2] / eta;
-        C->alpha[3] = (4. / 3.) * S.alpha[3] / eta;
-        C->alpha[4] = S.alpha[4] / eta;
+        const double eta = S.eta, ieta = S.ieta, M = S.M, etaM = eta * S.iM;
+        const double Mf2 = M * S.f2p, iMf2 = 1.0 / Mf2;
+        const double Mf1 = GWH_MF1P, iMf1 = 1.0 / GWH_MF1P;
+        S.beta[1] = etaM * (X.d_ins - gwh_setup_dphase_int(S, S.f1p, iMf1));
+        S.beta[0] = eta * (X.p_ins - gwh_setup_phase_int_l(S, S.f1p, Mf1, iMf1, GWH_MF1P_LN));
+        S.alpha[1] = etaM * (gwh_setup_dphase_int(S, S.f2p, iMf2) - X.dq_mr);
+        S.alpha[0] = eta * (gwh_setup_phase_int_l(S, S.f2p, Mf2, iMf2, X.l2) - X.q_mr) - S.alpha[1] * Mf2;
+        C->beta[0] = S.beta[0] * ieta;
+        C->beta[1] = S.beta[1] * ieta;
+        C->beta[2] = S.beta[2] * ieta;
+        C->beta[3] = S.beta[3] * ieta * (1. / 3.);
+        C->alpha[0] = S.alpha[0] * ieta;
+        C->alpha[1] = S.alpha[1] * ieta;
+        C->alpha[2] = S.alpha[2] * ieta;
+        C->alpha[3] = (4. / 3.) * S.alpha[3] * ieta;
+        C->alpha[4] = S.alpha[4] * ieta;
         C->alpha[5] = S.alpha[5] * S.fRD;
         if (!pv2) {
             /* phase and time alignment (IMRPhenomD.cpp:441-466) */
@@ -692,9 +701,9 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__rest
                 if (fref < S.f1p)
                     b = X.ref;
                 else if (fref > S.f2p)
-                    b = X.ref + (1. / eta) * (S.alpha[0] + S.alpha[1] * (M * fref));
+                    b = X.ref + ieta * (S.alpha[0] + S.alpha[1] * (M * fref));
                 else
-                    b = gwh_setup_phase_int_l(S, fref, X.ref);
+                    b = gwh_setup_phase_int_l(S, fref, M * fref, 1.0 / (M * fref), X.ref);
                 phic = 2 * p.phiRef + b;
             } else {
                 fref = 0;
@@ -702,7 +711,7 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__rest
             }
             double tc_shift = 0;
             if (p.shift_time)
-                tc_shift = (X.dq_mr3 + (1. / eta) * (M * S.alpha[1])) + (-S.alpha[1] + X.alpha1_fit) * M / eta;
+                tc_shift = X.dq_mr3 + ieta * (M * X.alpha1_fit); /* the slope at f3 with the fitted alpha1 */
             C->tc_total = GWH_2PI * p.tc + tc_shift;
             C->phic = phic;
             C->f_ref = fref;
@@ -711,26 +720,29 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__rest
             C->phic = 2 * X.phi_aligned;
             C->tc_total = GWH_2PI * p.tc;
             C->f_ref = p.f_ref;
-            /* t_c alignment: derivative at fRD of a 10-knot natural spline of -Psi_MR (IMRPhenomP.cpp:550-606) */
+            /* t_c alignment: 1 / (2 pi) times the derivative at fRD of a 10-knot natural spline of -Psi_MR
+             * (IMRPhenomP.cpp:550-606); the spline of a line is the line, so its alpha1 part is exact */
             double t_corr = 0;
             if (p.shift_time) {
-                double ph[10];
+                double q[10];
 #pragma unroll
-                for (int j = 0; j < 10; j++)
-                    ph[j] = -(X.tq[j] + (1. / eta) * (S.alpha[0] + S.alpha[1] * (M * gwh_setup_knot(S.fRD, j))));
-                t_corr = gwh_setup_tcorr(S.fRD, ph);
+                for (int j = 0; j < 10; j++) q[j] = X.tq[j];
+                t_corr = -(gwh_setup_tcorr(S.fRD, q) + ieta * (S.alpha[1] * M));
+                if (!(S.fRD > 0)) t_corr = 0;
             }
-            C->t_corr_2pi = GWH_2PI * t_corr;
+            C->t_corr_2pi = t_corr;
         }
     }
 }
+
+#pragma clang fp contract(fast)
 
 static void launch_setup(int model, int n, hipStream_t st, const gwh_params *params, const int *inst_event,
                          int event0, InstCoef *coef, int *active, const int *d_count = nullptr,
                          const int *d_mask = nullptr)
 {
     Engine &E = gwh_engine();
-    dim3 g((n + 63) / 64), b(256);
+    dim3 g((n + GWH_SETUP_LANES - 1) / GWH_SETUP_LANES), b(256);
     const int var = gwh_ppe_variant(model);
     auto k = gwh_is_pv2(model) ? (var ? gwh_setup_kernel<GWH_IMRPHENOMPV2, true> : gwh_setup_kernel<GWH_IMRPHENOMPV2, false>)
                                : (var ? gwh_setup_kernel<GWH_IMRPHENOMD, true> : gwh_setup_kernel<GWH_IMRPHENOMD, false>);

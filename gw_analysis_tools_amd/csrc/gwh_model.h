@@ -285,29 +285,24 @@ struct DetGeom {
 /* ------------------------------------------------------------------------- */
 /* FP64 setup helpers (device)                                                 */
 /* ------------------------------------------------------------------------- */
-
-__device__ __forceinline__ double gwh_spline_eval(const double *x, const double *y, const double *c, int n,
-                                                  double xq)
-{
-    if (!(xq >= x[0] && xq <= x[n - 1])) return __longlong_as_double(0x7ff8000000000000LL);
-    /* interval with x[lo] <= xq < x[lo + 1] (lo = n - 2 at the last knot), the one a bisection finds:
-     * start from the uniform-spacing guess and walk (a step or two on the near-uniform spin grid) */
-    int lo = (int)((xq - x[0]) / (x[n - 1] - x[0]) * (n - 1));
-    lo = lo < 0 ? 0 : (lo > n - 2 ? n - 2 : lo);
-    while (lo > 0 && x[lo] > xq) lo--;
-    while (lo < n - 2 && x[lo + 1] <= xq) lo++;
-    double h = x[lo + 1] - x[lo];
-    double b = (y[lo + 1] - y[lo]) / h - h * (c[lo + 1] + 2.0 * c[lo]) / 3.0;
-    double d = (c[lo + 1] - c[lo]) / (3.0 * h);
-    double dx = xq - x[lo];
-    return y[lo] + dx * (b + dx * (c[lo] + dx * d));
-}
+/*
+ * The setup runs one lane per instance and role, so it is bound by the latency of each role's chain and by fetching its
+ * instructions, which few waves execute once: 78 KB (IMRPhenomD) and 99 KB (IMRPhenomPv2), more than the instruction
+ * cache, while every division, power and logarithm was written out.  Constants stand for those that do not depend on the
+ * instance -- M f is 0.014 and 0.018 at the first transitions whatever M -- and one reciprocal of eta, M, ... for
+ * repeated divisions: 56 KB and 57 KB.  512 instances: IMRPhenomD 11.3 -> 7.5 us, IMRPhenomPv2 17.5 -> 11.2 us (of
+ * which the half-filled blocks of gwh_setup_kernel 1.3 and 0.9).
+ *
+ * Multiply-adds are fused within an expression only (contract(on)), so a function rounds alike wherever it is inlined:
+ * the kernels with and without the modified-gravity terms have to agree bit for bit where the terms vanish.
+ */
+#pragma clang fp contract(on)
 
 /* both QNM splines (M f_ring and M f_damp) at spin a, with the interval x[lo] <= a < x[lo + 1] (lo = n - 2 at
  * the last knot) that a bisection finds.  On the table's near-uniform spin grid that interval lies within one
  * knot of the uniform-spacing guess, so the knots and coefficients of the four-knot window around the guess
- * are loaded together (one memory round trip) and the interval is picked among them; a window that misses it
- * falls back to the walk of gwh_spline_eval.  Same arithmetic as gwh_spline_eval. */
+ * are loaded together (one memory round trip) and the interval is picked among them; a window that misses it is
+ * moved until it does not. */
 __device__ __forceinline__ void gwh_qnm_eval(const QnmTable &q, double a, double &fring, double &fdamp)
 {
     const int n = q.n;
@@ -315,22 +310,21 @@ __device__ __forceinline__ void gwh_qnm_eval(const QnmTable &q, double a, double
         fring = fdamp = __longlong_as_double(0x7ff8000000000000LL);
         return;
     }
-    int g = (int)((a - q.x0) / (q.x1 - q.x0) * (n - 1));
-    g = g < 0 ? 0 : (g > n - 2 ? n - 2 : g);
-    const int b = (g - 1 < 0) ? 0 : (g - 1 > n - 4 ? n - 4 : g - 1);
+    const int g = (int)((a - q.x0) / (q.x1 - q.x0) * (n - 1));
+    int b = (g - 1 < 0) ? 0 : (g - 1 > n - 4 ? n - 4 : g - 1);
     double xs[4], yr[4], cr[4], yd[4], cd[4];
+    for (;;) {
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-        xs[k] = q.spin[b + k];
-        yr[k] = q.fring[b + k];
-        cr[k] = q.c_ring[b + k];
-        yd[k] = q.fdamp[b + k];
-        cd[k] = q.c_damp[b + k];
-    }
-    if (!(xs[0] <= a && (a < xs[3] || b == n - 4))) {
-        fring = gwh_spline_eval(q.spin, q.fring, q.c_ring, n, a);
-        fdamp = gwh_spline_eval(q.spin, q.fdamp, q.c_damp, n, a);
-        return;
+        for (int k = 0; k < 4; k++) {
+            xs[k] = q.spin[b + k];
+            yr[k] = q.fring[b + k];
+            cr[k] = q.c_ring[b + k];
+            yd[k] = q.fdamp[b + k];
+            cd[k] = q.c_damp[b + k];
+        }
+        const int step = (xs[0] > a && b > 0) ? -1 : ((a >= xs[3] && b < n - 4) ? 1 : 0);
+        if (step == 0) break;
+        b += step;
     }
     double x0 = xs[0], x1 = xs[1], r0 = yr[0], r1 = yr[1], rc0 = cr[0], rc1 = cr[1], d0 = yd[0], d1 = yd[1],
            dc0 = cd[0], dc1 = cd[1];
@@ -348,12 +342,12 @@ __device__ __forceinline__ void gwh_qnm_eval(const QnmTable &q, double a, double
             dc0 = cd[k];
             dc1 = cd[k + 1];
         }
-    const double h = x1 - x0, dx = a - x0;
-    double bb = (r1 - r0) / h - h * (rc1 + 2.0 * rc0) / 3.0;
-    double dd = (rc1 - rc0) / (3.0 * h);
+    const double h = x1 - x0, dx = a - x0, ih = 1.0 / h;
+    double bb = (r1 - r0) * ih - h * (rc1 + 2.0 * rc0) * (1.0 / 3.0);
+    double dd = (rc1 - rc0) * (ih * (1.0 / 3.0));
     fring = r0 + dx * (bb + dx * (rc0 + dx * dd));
-    bb = (d1 - d0) / h - h * (dc1 + 2.0 * dc0) / 3.0;
-    dd = (dc1 - dc0) / (3.0 * h);
+    bb = (d1 - d0) * ih - h * (dc1 + 2.0 * dc0) * (1.0 / 3.0);
+    dd = (dc1 - dc0) * (ih * (1.0 / 3.0));
     fdamp = d0 + dx * (bb + dx * (dc0 + dx * dd));
 }
 
@@ -365,24 +359,23 @@ __device__ __forceinline__ double gwh_fit(const double *tab, int row, double eta
            x * x * (p[5] + p[6] * eta + p[7] * eta * eta) + x * x * x * (p[8] + p[9] * eta + p[10] * eta * eta);
 }
 
-__device__ __forceinline__ double gwh_final_spin0815(double eta, double chi1, double chi2)
+/* delta = sqrt(1 - 4 eta), ieta = 1 / eta */
+__device__ __forceinline__ double gwh_final_spin0815(double eta, double ieta, double delta, double chi1, double chi2)
 {
-    double Seta = sqrt(1.0 - 4.0 * eta);
-    double m1 = 0.5 * (1.0 + Seta), m2 = 0.5 * (1.0 - Seta);
+    double m1 = 0.5 * (1.0 + delta), m2 = 0.5 * (1.0 - delta);
     double s = m1 * m1 * chi1 + m2 * m2 * chi2;
     double eta2 = eta * eta, eta3 = eta2 * eta, s2 = s * s, s3 = s2 * s;
     return eta * (3.4641016151377544 - 4.399247300629289 * eta + 9.397292189321194 * eta2 -
                   13.180949901606242 * eta3 +
-                  s * ((1.0 / eta - 0.0850917821418767 - 5.837029316602263 * eta) +
+                  s * ((ieta - 0.0850917821418767 - 5.837029316602263 * eta) +
                        (0.1014665242971878 - 2.0967746996832157 * eta) * s +
                        (-1.3546806617824356 + 4.108962025369336 * eta) * s2 +
                        (-0.8676969352555539 + 2.064046835273906 * eta) * s3));
 }
 
-__device__ __forceinline__ double gwh_erad0815(double eta, double chi1, double chi2)
+__device__ __forceinline__ double gwh_erad0815(double eta, double delta, double chi1, double chi2)
 {
-    double Seta = sqrt(1.0 - 4.0 * eta);
-    double m1 = 0.5 * (1.0 + Seta), m2 = 0.5 * (1.0 - Seta);
+    double m1 = 0.5 * (1.0 + delta), m2 = 0.5 * (1.0 - delta);
     double m1s = m1 * m1, m2s = m2 * m2;
     double s = (m1s * chi1 + m2s * chi2) / (m1s + m2s);
     double eta2 = eta * eta, eta3 = eta2 * eta;
@@ -395,6 +388,7 @@ __device__ __forceinline__ double gwh_erad0815(double eta, double chi1, double c
 /* Everything the setup needs while building the record */
 struct SetupState {
     double m1, m2, M, eta, chi1, chi2, chi_s, chi_a, delta, chi_pn, chi_eff, Mc, A0;
+    double ieta, iM; /* 1 / eta, 1 / M */
     double fRD, fdamp, f1, f3, f1p, f2p;
     double rho[3], v2, g[3], sigma[5], beta[4], alpha[6];
     double pa[7];  /* amplitude PN coefficients (reference numbering) */
@@ -410,15 +404,15 @@ struct SetupState {
 __device__ __forceinline__ double gwh_pn_c8_gr(double eta, double dm, double ca, double cs)
 {
     const double eta2 = eta * eta;
-    return (38645. * GWH_PI / 756 - 65. * GWH_PI * eta / 9 + dm * (-732985. / 2268 - 140. * eta / 9) * ca +
-            (-732985. / 2268 + 24260. * eta / 81 + 340. * eta2 / 9) * cs);
+    return (38645. * GWH_PI / 756 - 65. * GWH_PI / 9 * eta + dm * (-732985. / 2268 - 140. / 9 * eta) * ca +
+            (-732985. / 2268 + 24260. / 81 * eta + 340. / 9 * eta2) * cs);
 }
 
 /* gIMR inspiral phase terms beyond the IMRPhenomD polynomial (gIMRPhenomD.cpp:148-184): the order-1 coefficient
  * (zero in IMRPhenomD) and 3/(128 eta) delta_i (pi M f)^((i - 5)/3) for i = -4..-1, with their f derivative */
 __device__ __forceinline__ double gwh_setup_gimr(const SetupState &S, double f, double *deriv)
 {
-    const double K = 3. / (128. * S.eta);
+    const double K = 3. / 128. * S.ieta;
     const double x = GWH_PI * S.M * f, iv = 1.0 / cbrt(x);
     double iv2 = iv * iv, iv4 = iv2 * iv2;
     double t = S.pp[1] * iv4, d = S.pp[1] * (-4. / 3.) * iv4;
@@ -450,67 +444,72 @@ __device__ __forceinline__ double gwh_setup_ppe(const SetupState &S, double f, d
     return t;
 }
 
-/* TF2 + sigma inspiral phase at f (IMRPhenomD.cpp:1364-1399) */
-__device__ __forceinline__ double gwh_setup_phase_ins(const SetupState &S, double f)
+/* the transition frequencies times M, and what the phases and amplitudes need of them */
+#define GWH_MF1 0.014                        /* amplitude: inspiral up to here */
+#define GWH_MF1_V 0.35298748079802035326     /* (pi M f)^(1/3) */
+#define GWH_MF1_U 0.24101422641752299861     /* (M f)^(1/3) */
+#define GWH_MF1P 0.018                       /* phase: inspiral up to here */
+#define GWH_MF1P_V 0.38383165853550260132    /* (pi M f)^(1/3) */
+#define GWH_MF1P_U 0.26207413942088966071    /* (M f)^(1/3) */
+#define GWH_MF1P_LNPI -2.8726536352365721857 /* ln(pi M f) */
+#define GWH_MF1P_LN -4.0173835210859723598   /* ln(M f) */
+
+/* TF2 + sigma inspiral phase at f (IMRPhenomD.cpp:1364-1399) from v = (pi M f)^(1/3), 1 / v, ln v^3, u = (M f)^(1/3), M f */
+__device__ __forceinline__ double gwh_setup_phase_ins_at(const SetupState &S, double f, double v, double iv, double lx,
+                                                         double u, double Mf)
 {
-    double x = GWH_PI * S.M * f;
-    double v = cbrt(x);
-    double lx = log(x);
     double c5 = S.pp[8] + lx * S.pp[9];
     double c6 = S.pp[10] - S.pp[11] * lx;
-    double v2 = v * v;
+    double v2 = v * v, iv2 = iv * iv;
     double poly = S.pp[0] + v2 * (S.pp[2] + v * (S.pp[3] + v * (S.pp[4] + v * (c5 + v * (c6 + v * S.pp[7])))));
-    double Mf = S.M * f;
-    double u = cbrt(Mf);
     double Mf43 = Mf * u, Mf53 = Mf43 * u;
-    double ph = -GWH_PI / 4. + 3. / (128. * S.eta) * poly / (v2 * v2 * v) +
-                (1. / S.eta) * (S.sigma[1] * Mf + 0.75 * S.sigma[2] * Mf43 + 0.6 * S.sigma[3] * Mf53 +
-                                0.5 * S.sigma[4] * Mf * Mf);
+    double ph = -GWH_PI / 4. + S.ieta * (3. / 128. * poly * (iv2 * iv2 * iv) +
+                                         (S.sigma[1] * Mf + 0.75 * S.sigma[2] * Mf43 + 0.6 * S.sigma[3] * Mf53 +
+                                          0.5 * S.sigma[4] * Mf * Mf));
     if (S.ppe_n > 0) ph += gwh_setup_ppe(S, f, nullptr);
     if (S.gimr) ph += gwh_setup_gimr(S, f, nullptr);
     return ph;
 }
-
-/* d/df of the inspiral phase (IMRPhenomD.cpp:1426-1460) */
-__device__ __forceinline__ double gwh_setup_dphase_ins(const SetupState &S, double f)
+__device__ __forceinline__ double gwh_setup_phase_ins(const SetupState &S, double f)
 {
-    double M = S.M;
-    double x = GWH_PI * M * f;
-    double lx = log(x);
+    const double Mf = S.M * f, u = cbrt(Mf), v = u * 1.4645918875615231, iv = 1.0 / v;
+    return gwh_setup_phase_ins_at(S, f, v, iv, log(GWH_PI * Mf), u, Mf);
+}
+
+/* d/df of the inspiral phase (IMRPhenomD.cpp:1426-1460) at f1p = 0.018 / M */
+__device__ __forceinline__ double gwh_setup_dphase_ins_f1p(const SetupState &S)
+{
+    const double M = S.M, v = GWH_MF1P_V, u = GWH_MF1P_U, lx = GWH_MF1P_LNPI;
     double c[8];
     for (int i = 0; i < 8; i++) c[i] = S.pp[i];
     c[5] = S.pp[8] + lx * S.pp[9];
     c[6] = S.pp[10] - S.pp[11] * lx;
-    double K = 3. / (128. * S.eta);
-    /* x^((i - 8) / 3) as powers of x^(-1/3) */
-    double v = cbrt(x), iv = 1.0 / v;
+    const double K = 3. / 128. * S.ieta, iv = 1.0 / v, inf = M * (1.0 / GWH_MF1P); /* 1 / f */
+    /* (pi M f)^((i - 8) / 3) as powers of v^-1 */
     double sum = 0, pw = iv;
 #pragma unroll
     for (int i = 7; i >= 0; i--) {
-        sum += c[i] * ((i - 5.) / 3.) * pw;
+        sum += c[i] * (((i - 5.) / 3.) * pw);
         pw *= iv;
     }
-    double d = K * (GWH_PI * M) * sum + K * (S.pp[9] - S.pp[11] * v) / f;
-    /* M^(4/3) f^(1/3) = M (Mf)^(1/3), M^(5/3) f^(2/3) = M (Mf)^(2/3) */
-    double u = cbrt(M * f);
-    double sg = S.sigma[1] * M + S.sigma[2] * M * u + S.sigma[3] * M * u * u + S.sigma[4] * M * M * f;
-    double r = d + sg / S.eta;
+    double r = K * ((GWH_PI * M) * sum + (S.pp[9] - S.pp[11] * v) * inf) +
+               S.ieta * (M * (S.sigma[1] + S.sigma[2] * u + S.sigma[3] * (u * u) + S.sigma[4] * GWH_MF1P));
     if (S.ppe_n > 0) {
         double dt;
-        gwh_setup_ppe(S, f, &dt);
+        gwh_setup_ppe(S, S.f1p, &dt);
         r += dt;
     }
     if (S.gimr) { /* the order-1 coefficient is already in the polynomial derivative above */
         double dt;
-        gwh_setup_gimr(S, f, &dt);
+        gwh_setup_gimr(S, S.f1p, &dt);
         const double iv4 = iv * iv * iv * iv;
-        r += dt - K * S.pp[1] * (-4. / 3.) * iv4 / f;
+        r += dt - K * S.pp[1] * (-4. / 3.) * iv4 * inf;
         /* The reference differentiates the log terms of c5 and c6 with their GR coefficients whatever gIMR did
          * to them (assign_nonstatic_pn_phase_coeff_deriv, IMRPhenomD.cpp:1068-1084, reached from gIMRPhenomD's
          * Dphase_ins through the GR class, gIMRPhenomD.cpp:167-184): with phi orders 8 and 9 set, the
          * connection slope at f1 is not the inspiral phase's own slope. */
         const double c9gr = gwh_pn_c8_gr(S.eta, S.delta, S.chi_a, S.chi_s), c11gr = 6848. / 63.;
-        r += K * ((c9gr - S.pp[9]) - (c11gr - S.pp[11]) * v) / f;
+        r += K * ((c9gr - S.pp[9]) - (c11gr - S.pp[11]) * v) * inf;
     }
     return r;
 }
@@ -524,127 +523,100 @@ __device__ __forceinline__ double gwh_setup_ppe_imr(const SetupState &S, double 
     return deriv ? d : t;
 }
 
-/* intermediate phase at f, given lMf = ln(M f) */
-__device__ __forceinline__ double gwh_setup_phase_int_l(const SetupState &S, double f, double lMf)
+/* intermediate phase at f and its derivative, given M f, 1 / (M f) and ln(M f) */
+__device__ __forceinline__ double gwh_setup_phase_int_l(const SetupState &S, double f, double Mf, double iMf, double lMf)
 {
-    double Mf = S.M * f;
-    return (1. / S.eta) * (S.beta[0] + S.beta[1] * Mf + S.beta[2] * lMf - S.beta[3] / 3. / (Mf * Mf * Mf)) +
+    return S.ieta * (S.beta[0] + S.beta[1] * Mf + S.beta[2] * lMf - S.beta[3] * (iMf * iMf * iMf) * (1. / 3.)) +
            gwh_setup_ppe_imr(S, f, false);
 }
-
-__device__ __forceinline__ double gwh_setup_phase_int(const SetupState &S, double f)
+__device__ __forceinline__ double gwh_setup_dphase_int(const SetupState &S, double f, double iMf)
 {
-    return gwh_setup_phase_int_l(S, f, log(S.M * f));
+    const double i2 = iMf * iMf;
+    return S.ieta * (S.M * (S.beta[1] + S.beta[2] * iMf + S.beta[3] * (i2 * i2))) + gwh_setup_ppe_imr(S, f, true);
 }
 
-__device__ __forceinline__ double gwh_setup_dphase_int(const SetupState &S, double f)
-{
-    double M = S.M;
-    return (1. / S.eta) * (S.beta[1] * M + S.beta[2] / f + S.beta[3] / (M * M * M * f * f * f * f)) +
-           gwh_setup_ppe_imr(S, f, true);
-}
-
+/* merger-ringdown phase at f and its derivative */
 __device__ __forceinline__ double gwh_setup_phase_mr(const SetupState &S, double f)
 {
-    double Mf = S.M * f;
-    return (1. / S.eta) * (S.alpha[0] + S.alpha[1] * Mf - S.alpha[2] / Mf + (4. / 3.) * S.alpha[3] * sqrt(sqrt(Mf * Mf * Mf)) +
-                           S.alpha[4] * atan((f - S.alpha[5] * S.fRD) / S.fdamp)) +
+    const double Mf = S.M * f;
+    return S.ieta * (S.alpha[0] + S.alpha[1] * Mf - S.alpha[2] / Mf + (4. / 3.) * S.alpha[3] * sqrt(sqrt(Mf * Mf * Mf)) +
+                     S.alpha[4] * atan((f - S.alpha[5] * S.fRD) / S.fdamp)) +
            gwh_setup_ppe_imr(S, f, false);
 }
-
 __device__ __forceinline__ double gwh_setup_dphase_mr(const SetupState &S, double f)
 {
-    double M = S.M;
-    double t = (f - S.alpha[5] * S.fRD) / S.fdamp;
-    return (S.alpha[4] / (S.fdamp * (1. + t * t)) + S.alpha[2] / (f * f * M) + M * (S.alpha[1] + S.alpha[3] / sqrt(sqrt(f * M)))) /
-               S.eta +
+    const double M = S.M, Mf = M * f, iMf = 1.0 / Mf;
+    const double w = S.fdamp, t = f - S.alpha[5] * S.fRD;
+    return S.ieta * (S.alpha[4] * w / (w * w + t * t) +
+                     M * (S.alpha[2] * (iMf * iMf) + S.alpha[1] + S.alpha[3] * (sqrt(sqrt(Mf * Mf * Mf)) * iMf))) +
            gwh_setup_ppe_imr(S, f, true);
 }
 
-__device__ __forceinline__ double gwh_setup_build_phase(const SetupState &S, double f)
+/* reduced inspiral amplitude and its frequency derivative (IMRPhenomD.cpp:1335-1420) at f1 = 0.014 / M */
+__device__ __forceinline__ void gwh_setup_amp_ins_f1(const SetupState &S, double *val, double *der)
 {
-    if (f < S.f1p) return gwh_setup_phase_ins(S, f);
-    if (f > S.f2p) return gwh_setup_phase_mr(S, f);
-    return gwh_setup_phase_int(S, f);
-}
-
-/* reduced inspiral amplitude and its frequency derivative (IMRPhenomD.cpp:1335-1420) */
-__device__ __forceinline__ void gwh_setup_amp_ins(const SetupState &S, double f, double *val, double *der)
-{
-    double M = S.M;
-    double x = GWH_PI * M * f, y = M * f;
-    double vx = cbrt(x), vy = cbrt(y);
     double v = 0, d = 0, p = 1.0;
+#pragma unroll
     for (int i = 0; i < 7; i++) {
         v += S.pa[i] * p;
-        if (i > 0) d += S.pa[i] * (i / 3.) * p / x * (GWH_PI * M);
-        p *= vx;
+        if (i > 0) d += S.pa[i] * ((i / 3.) * p);
+        p *= GWH_MF1_V;
     }
-    double y73 = y * y * vy, y83 = y73 * vy, y3 = y * y * y;
+    const double y = GWH_MF1, y73 = y * y * GWH_MF1_U, y83 = y73 * GWH_MF1_U, y3 = y * y * y;
     v += S.rho[0] * y73 + S.rho[1] * y83 + S.rho[2] * y3;
-    d += (S.rho[0] * (7. / 3.) * y73 + S.rho[1] * (8. / 3.) * y83 + S.rho[2] * 3. * y3) / y * M;
+    d += S.rho[0] * (7. / 3. * y73) + S.rho[1] * (8. / 3. * y83) + S.rho[2] * (3. * y3);
     *val = v;
-    *der = d;
+    *der = d * (S.M * (1. / GWH_MF1)); /* d ln f */
 }
 
-/* reduced merger-ringdown amplitude and its derivative (IMRPhenomD.cpp:1467-1532) */
-__device__ __forceinline__ void gwh_setup_amp_mr(const SetupState &S, double f, double *val, double *der)
+/* reduced merger-ringdown amplitude and its derivative (IMRPhenomD.cpp:1467-1532); iw = 1 / (gamma3 fdamp) */
+__device__ __forceinline__ void gwh_setup_amp_mr(const SetupState &S, double f, double iw, double *val, double *der)
 {
     double dl = f - S.fRD, w = S.g[2] * S.fdamp;
-    double L = dl * dl + w * w;
-    double a = S.g[0] * S.g[2] * S.fdamp * S.M * exp(-S.g[1] * dl / w) / (S.M * S.M * L);
+    double iL = 1.0 / (dl * dl + w * w);
+    double a = S.g[0] * w * S.iM * exp(-S.g[1] * dl * iw) * iL;
     *val = a;
-    *der = a * (-S.g[1] / w - 2.0 * dl / L);
+    *der = a * (-S.g[1] * iw - 2.0 * dl * iL);
 }
 
 /* ---- Pv2 precession helpers (IMRPhenomP.cpp) ---- */
-__device__ __forceinline__ double gwh_l2pn(double eta, double x)
+/* orbital angular momentum at v = (pi M f)^(1/3) */
+__device__ __forceinline__ double gwh_l2pn(double eta, double v)
 {
-    double eta2 = eta * eta;
-    return (eta * (1.0 + (1.5 + eta / 6.0) * x + (3.375 - (19.0 * eta) / 8. - eta2 / 24.0) * x * x)) / sqrt(x);
+    const double eta2 = eta * eta, x = v * v;
+    return eta * (1.0 + (1.5 + eta / 6.0) * x + (3.375 - (19.0 / 8.) * eta - eta2 / 24.0) * x * x) / v;
 }
 
 /* NNLO Euler-angle coefficients (IMRPhenomP.cpp:64-144) */
 __device__ inline void gwh_euler_coeffs(double q, double chil, double chip, double *a, double *e)
 {
-    double m2 = q / (1. + q), m1 = 1. / (1. + q);
-    double dm = m1 - m2;
-    double eta = m1 * m2, eta2 = eta * eta, eta3 = eta2 * eta, eta4 = eta3 * eta;
-    double chil2 = chil * chil, chip2 = chip * chip, chip4 = chip2 * chip2;
-    double dm2 = dm * dm, dm3 = dm2 * dm;
-    double m2_2 = m2 * m2, m2_3 = m2_2 * m2, m2_4 = m2_3 * m2, m2_5 = m2_4 * m2, m2_6 = m2_5 * m2, m2_7 = m2_6 * m2,
-           m2_8 = m2_7 * m2;
-    a[0] = (-0.18229166666666666 - (5 * dm) / (64. * m2));
-    a[1] = ((-15 * dm * m2 * chil) / (128. * eta) - (35 * m2_2 * chil) / (128. * eta));
-    a[2] = (-1.7952473958333333 - (4555 * dm) / (7168. * m2) - (15 * chip2 * dm * m2_3) / (128. * eta2) -
-            (35 * chip2 * m2_4) / (128. * eta2) - (515 * eta) / 384. - (15 * dm2 * eta) / (256. * m2_2) -
-            (175 * dm * eta) / (256. * m2));
-    a[3] = -(35 * GWH_PI) / 48. - (5 * dm * GWH_PI) / (16. * m2) + (5 * dm2 * chil) / 16. + (5 * dm * m2 * chil) / 3. +
-           (2545 * m2_2 * chil) / 1152. - (5 * chip2 * dm * m2_5 * chil) / (128. * eta3) -
-           (35 * chip2 * m2_6 * chil) / (384. * eta3) + (2035 * dm * m2 * chil) / (21504. * eta) +
-           (2995 * m2_2 * chil) / (9216. * eta);
-    a[4] = (4.318908476114694 + (27895885 * dm) / (2.1676032e7 * m2) - (15 * chip4 * dm * m2_7) / (512. * eta4) -
-            (35 * chip4 * m2_8) / (512. * eta4) - (485 * chip2 * dm * m2_3) / (14336. * eta2) +
-            (475 * chip2 * m2_4) / (6144. * eta2) + (15 * chip2 * dm2 * m2_2) / (256. * eta) +
-            (145 * chip2 * dm * m2_3) / (512. * eta) + (575 * chip2 * m2_4) / (1536. * eta) + (39695 * eta) / 86016. +
-            (1615 * dm2 * eta) / (28672. * m2_2) - (265 * dm * eta) / (14336. * m2) + (955 * eta2) / 576. +
-            (15 * dm3 * eta2) / (1024. * m2_3) + (35 * dm2 * eta2) / (256. * m2_2) + (2725 * dm * eta2) / (3072. * m2) -
-            (15 * dm * m2 * GWH_PI * chil) / (16. * eta) - (35 * m2_2 * GWH_PI * chil) / (16. * eta) +
-            (15 * chip2 * dm * m2_7 * chil2) / (128. * eta4) + (35 * chip2 * m2_8 * chil2) / (128. * eta4) +
-            (375 * dm2 * m2_2 * chil2) / (256. * eta) + (1815 * dm * m2_3 * chil2) / (256. * eta) +
-            (1645 * m2_4 * chil2) / (192. * eta));
+    const double s = 1. / (1. + q), m2 = q * s, m1 = s;
+    const double dm = m1 - m2;
+    const double eta = m1 * m2, eta2 = eta * eta, ie = 1.0 / eta, ie2 = ie * ie, im = 1.0 / m2;
+    const double r = dm * im, r2 = r * r, r3 = r2 * r; /* dm / m2 */
+    const double dm2 = dm * dm, c2 = chip * chip, m22 = m2 * m2, m24 = m22 * m22;
+    const double x = chil * m2, y = chil * m22, x2 = x * x, y2 = y * y; /* chi_L m2, chi_L m2^2 */
+    const double p = c2 * m22, p4 = p * m22;                              /* chi_p^2 m2^2, chi_p^2 m2^4 */
+    const double px = dm * m2 * p;                                        /* chi_p^2 dm m2^3 */
+    const double w = x * dm;                                              /* chi_L dm m2 */
+    a[0] = -0.18229166666666666 - (5. / 64.) * r;
+    a[1] = -ie * ((15. / 128.) * w + (35. / 128.) * y);
+    e[2] = -1.7952473958333333 - (4555. / 7168.) * r - eta * (515. / 384. + (15. / 256.) * r2 + (175. / 256.) * r);
+    a[2] = e[2] - ie2 * ((15. / 128.) * px + (35. / 128.) * p4);
+    e[3] = -(35. * GWH_PI / 48.) - (5. * GWH_PI / 16.) * r + (5. / 16.) * dm2 * chil + (5. / 3.) * w + (2545. / 1152.) * y +
+           ie * ((2035. / 21504.) * w + (2995. / 9216.) * y);
+    a[3] = e[3] - ie * ie2 * (x * ((5. / 128.) * px * m2 + (35. / 384.) * p4 * m2));
+    e[4] = 4.318908476114694 + (27895885. / 2.1676032e7) * r +
+           eta * (39695. / 86016. + (1615. / 28672.) * r2 - (265. / 14336.) * r) +
+           eta2 * (955. / 576. + (15. / 1024.) * r3 + (35. / 256.) * r2 + (2725. / 3072.) * r) +
+           ie * (-GWH_PI * ((15. / 16.) * w + (35. / 16.) * y) + (375. / 256.) * dm2 * x2 + (1815. / 256.) * dm * (x * y) +
+                 (1645. / 192.) * y2);
+    a[4] = e[4] - ie2 * ie2 * (p4 * ((15. / 512.) * px + (35. / 512.) * p4)) +
+           ie2 * (-(485. / 14336.) * px + (475. / 6144.) * p4) +
+           ie * ((15. / 256.) * dm2 * p + (145. / 512.) * px + (575. / 1536.) * p4) +
+           ie2 * ie2 * (y2 * ((15. / 128.) * px + (35. / 128.) * p4));
     e[0] = a[0];
     e[1] = a[1];
-    e[2] = (-1.7952473958333333 - (4555 * dm) / (7168. * m2) - (515 * eta) / 384. - (15 * dm2 * eta) / (256. * m2_2) -
-            (175 * dm * eta) / (256. * m2));
-    e[3] = -(35 * GWH_PI) / 48. - (5 * dm * GWH_PI) / (16. * m2) + (5 * dm2 * chil) / 16. + (5 * dm * m2 * chil) / 3. +
-           (2545 * m2_2 * chil) / 1152. + (2035 * dm * m2 * chil) / (21504. * eta) + (2995 * m2_2 * chil) / (9216. * eta);
-    e[4] = (4.318908476114694 + (27895885 * dm) / (2.1676032e7 * m2) + (39695 * eta) / 86016. +
-            (1615 * dm2 * eta) / (28672. * m2_2) - (265 * dm * eta) / (14336. * m2) + (955 * eta2) / 576. +
-            (15 * dm3 * eta2) / (1024. * m2_3) + (35 * dm2 * eta2) / (256. * m2_2) + (2725 * dm * eta2) / (3072. * m2) -
-            (15 * dm * m2 * GWH_PI * chil) / (16. * eta) - (35 * m2_2 * GWH_PI * chil) / (16. * eta) +
-            (375 * dm2 * m2_2 * chil2) / (256. * eta) + (1815 * dm * m2_3 * chil2) / (256. * eta) +
-            (1645 * m2_4 * chil2) / (192. * eta));
 }
 
 /* iv = 1 / v (a bin takes it from its tabulated f^{-1/3}).  The sum as explicit fused multiply-adds, so every kernel
@@ -669,9 +641,8 @@ __device__ __forceinline__ double gwh_euler_eval(const double *c, double v, doub
  *            role 1  PN coefficients, the inspiral amplitude and its derivative at f1
  *            role 2  IMRPhenomPv2 frame (thetaJN, alpha0, zeta), detector projections, tiles to visit
  *            role 3  chirp mass, amplitude scale, ppE coefficients, powers of M; Pv2 precession constants
- *   phase 2  role 0  inspiral phase at f1p                 role 1  its derivative at f1p
- *            role 2  merger-ringdown phase and derivative at f2p with alpha0 = alpha1 = 0, ln(M f1p),
- *                    ln(M f2p), amplitude connection
+ *   phase 2  role 0  inspiral phase and derivative at f1p  role 1  amplitude connection
+ *            role 2  merger-ringdown phase and derivative at f2p with alpha0 = alpha1 = 0, ln(M f2p)
  *            role 3  phase piece at f_ref, merger-ringdown derivative at f3 (alpha1 = 0); Pv2 Euler offsets
  *            Pv2 with shift_time: the ten knots of the t_c spline (merger-ringdown phase, alpha0 = alpha1 = 0)
  *   phase 3  role 0  the C1 phase connection (beta0, beta1, alpha0, alpha1), phase and time alignment
@@ -689,7 +660,7 @@ struct SetupShared {
     double alpha0, phi_aligned; /* Pv2 frame */
     double p_ins, d_ins;      /* inspiral phase and derivative at f1p */
     double q_mr, dq_mr;       /* merger-ringdown phase and derivative at f2p, alpha0 = alpha1 = 0 */
-    double l1, l2;            /* ln(M f1p), ln(M f2p) */
+    double l2;                /* ln(M f2p) */
     double ref;               /* at f_ref: inspiral phase, merger-ringdown phase (alpha0 = alpha1 = 0) or ln(M f_ref) */
     double dq_mr3;            /* merger-ringdown derivative at f3, alpha1 = 0 */
     double tq[10];            /* Pv2 t_c spline knots: merger-ringdown phase, alpha0 = alpha1 = 0 */
@@ -706,9 +677,11 @@ __device__ __forceinline__ void gwh_setup_base(const gwh_params &p, int ppe, Set
     S.eta = (S.m1 * S.m2) / (S.M * S.M);
     S.chi_s = 0.5 * (S.chi1 + S.chi2);
     S.chi_a = 0.5 * (S.chi1 - S.chi2);
+    S.ieta = 1.0 / S.eta;
+    S.iM = 1.0 / S.M;
     S.delta = sqrt(1. - 4. * S.eta);
-    S.chi_eff = (S.m1 * S.chi1 + S.m2 * S.chi2) / S.M;
-    S.chi_pn = S.chi_eff - (38. * S.eta / 113.) * (2. * S.chi_s);
+    S.chi_eff = (S.m1 * S.chi1 + S.m2 * S.chi2) * S.iM;
+    S.chi_pn = S.chi_eff - (38. / 113.) * S.eta * (2. * S.chi_s);
     /* ppE terms (waveform_generator.cpp:1296-1300 copies them for the ppE methods only) */
     S.ppe_n = 0;
     if (ppe == 1 || ppe == 2) {
@@ -727,7 +700,8 @@ __device__ __forceinline__ double gwh_setup_chip(const gwh_params &p, const Setu
     const double s1x = p.spin1[0], s1y = p.spin1[1], s2x = p.spin2[0], s2y = p.spin2[1];
     const double m1_2 = S.m1 * S.m1, m2_2 = S.m2 * S.m2;
     double S1p = m1_2 * sqrt(s1y * s1y + s1x * s1x), S2p = m2_2 * sqrt(s2y * s2y + s2x * s2x);
-    double A1 = 2 + (3 * S.m2) / (2 * S.m1), A2 = 2 + (3 * S.m1) / (2 * S.m2);
+    /* times 2 m1 m2: A1 = 2 + 3 m2 / (2 m1), A2 = 2 + 3 m1 / (2 m2) */
+    double A1 = S.m2 * (4 * S.m1 + 3 * S.m2), A2 = S.m1 * (4 * S.m2 + 3 * S.m1);
     double num = (A2 * S2p > A1 * S1p) ? A2 * S2p : A1 * S1p;
     double den = (S.m2 > S.m1) ? A2 * m2_2 : A1 * m1_2;
     return num / den;
@@ -764,20 +738,14 @@ __device__ __forceinline__ void gwh_setup_ringdown(const gwh_params &p, bool pv2
     for (int i = 0; i < 3; i++) S.g[i] = gwh_fit(fits, 4 + i, S.eta, xfit);
     double af;
     if (pv2) {
-        double Mt = S.m1 + S.m2;
-        double et = S.m1 * S.m2 / (Mt * Mt);
-        double qf, afp;
-        if (S.m1 >= S.m2) {
-            qf = S.m1 / Mt;
-            afp = gwh_final_spin0815(et, S.chi1, S.chi2);
-        } else {
-            qf = S.m2 / Mt;
-            afp = gwh_final_spin0815(et, S.chi2, S.chi1);
-        }
+        const bool first = S.m1 >= S.m2;
+        const double qf = (first ? S.m1 : S.m2) * S.iM;
+        const double afp = gwh_final_spin0815(S.eta, S.ieta, S.delta, first ? S.chi1 : S.chi2, first ? S.chi2 : S.chi1);
         double Sperp = chip * qf * qf;
-        af = sqrt(1.0 / (afp * afp)) * afp * sqrt(Sperp * Sperp + afp * afp);
+        const double a2 = sqrt(Sperp * Sperp + afp * afp);
+        af = afp == 0 ? __longlong_as_double(0x7ff8000000000000LL) : copysign(a2, afp); /* |afp|^-1 afp a2 */
     } else {
-        af = gwh_final_spin0815(S.eta, S.chi1, S.chi2);
+        af = gwh_final_spin0815(S.eta, S.ieta, S.delta, S.chi1, S.chi2);
     }
     if (p.dep_postmerger) {
         /* IMRPhenomD.cpp:1112-1179 */
@@ -792,19 +760,19 @@ __device__ __forceinline__ void gwh_setup_ringdown(const gwh_params &p, bool pv2
         S.fRD = (1. / GWH_2PI) * MWRD / (S.M * (1. - Er));
         S.fdamp = (1. / GWH_2PI) * MWd / (S.M * (1. - Er));
     } else {
-        double Er = gwh_erad0815(S.eta, S.chi1, S.chi2);
         double fr, fd;
-        gwh_qnm_eval(qnm, af, fr, fd);
-        S.fRD = fr / (1.0 - Er) / S.M;
-        S.fdamp = fd / (1.0 - Er) / S.M;
+        gwh_qnm_eval(qnm, af, fr, fd); /* its loads are in flight while the radiated energy is computed */
+        const double s = S.iM / (1.0 - gwh_erad0815(S.eta, S.delta, S.chi1, S.chi2));
+        S.fRD = fr * s;
+        S.fdamp = fd * s;
     }
-    S.f1p = 0.018 / S.M;
+    S.f1p = GWH_MF1P / S.M;
     S.f2p = S.fRD / 2.;
-    S.f1 = 0.014 / S.M;
+    S.f1 = GWH_MF1 / S.M;
     {
-        double g2 = S.g[1], g3 = S.g[2];
-        double v = (g2 > 1) ? S.fRD + (S.fdamp * (-1.) * g3) / g2 : S.fRD + S.fdamp * g3 * (sqrt(1 - g2 * g2) - 1) / g2;
-        S.f3 = fabs(v);
+        const double g2 = S.g[1], g3 = S.g[2];
+        const double v = (g2 > 1) ? -1.0 : sqrt(1 - g2 * g2) - 1;
+        S.f3 = fabs(S.fRD + S.fdamp * g3 * v / g2);
     }
 }
 
@@ -816,33 +784,32 @@ __device__ __forceinline__ void gwh_setup_pn(const gwh_params &p, SetupState &S)
     double eta2 = eta * eta, eta3 = eta2 * eta, cs2 = cs * cs, ca2 = ca * ca, pi2 = GWH_PI * GWH_PI;
     S.pa[0] = 1.;
     S.pa[1] = 0.;
-    S.pa[2] = (-323. / 224 + 451 * eta / 168);
-    S.pa[3] = (27. * dm * ca / 8 + (27. / 8 - 11. * eta / 6) * cs);
-    S.pa[4] = (-27312085. / 8128512 - 1975055 * eta / 338688 + 105271 * eta2 / 24192 + (-81. / 32 + 8 * eta) * ca2 -
-               81 * dm * ca * cs / 16 + (-81. / 32 + 17 * eta / 8) * cs2);
-    S.pa[5] = (-85 * GWH_PI / 64 + 85 * GWH_PI * eta / 16 + dm * (285197. / 16128 - 1579 * eta / 4032) * ca +
-               (285197. / 16128 - 15317 * eta / 672 - 2227 * eta2 / 1008) * cs);
-    S.pa[6] = (-177520268561. / 8583708672 + (545384828789. / 5007163392 - 205 * pi2 / 48) * eta -
-               3248849057 * eta2 / 178827264 + 34473079 * eta3 / 6386688 +
-               (1614569. / 64512 - 1873643. * eta / 16128 + 2167 * eta2 / 42) * ca2 +
-               (31 * GWH_PI / 12 - 7 * GWH_PI * eta / 3) * cs +
-               (1614569. / 64512 - 61391 * eta / 1344 + 57451 * eta2 / 4032) * cs2 +
-               dm * ca * (31 * GWH_PI / 12 + (1614569. / 32256 - 165961 * eta / 2688) * cs));
+    S.pa[2] = -323. / 224 + 451. / 168 * eta;
+    S.pa[3] = 27. / 8 * dm * ca + (27. / 8 - 11. / 6 * eta) * cs;
+    S.pa[4] = -27312085. / 8128512 - 1975055. / 338688 * eta + 105271. / 24192 * eta2 + (-81. / 32 + 8 * eta) * ca2 -
+              81. / 16 * dm * ca * cs + (-81. / 32 + 17. / 8 * eta) * cs2;
+    S.pa[5] = -85 * GWH_PI / 64 + 85 * GWH_PI / 16 * eta + dm * (285197. / 16128 - 1579. / 4032 * eta) * ca +
+              (285197. / 16128 - 15317. / 672 * eta - 2227. / 1008 * eta2) * cs;
+    S.pa[6] = -177520268561. / 8583708672 + (545384828789. / 5007163392 - 205 * pi2 / 48) * eta -
+              3248849057. / 178827264 * eta2 + 34473079. / 6386688 * eta3 +
+              (1614569. / 64512 - 1873643. / 16128 * eta + 2167. / 42 * eta2) * ca2 +
+              (31 * GWH_PI / 12 - 7 * GWH_PI / 3 * eta) * cs +
+              (1614569. / 64512 - 61391. / 1344 * eta + 57451. / 4032 * eta2) * cs2 +
+              dm * ca * (31 * GWH_PI / 12 + (1614569. / 32256 - 165961. / 2688 * eta) * cs);
     for (int i = 0; i < 12; i++) S.pp[i] = 0;
     S.pp[0] = 1.;
-    S.pp[2] = 3715. / 756 + 55. * eta / 9;
-    S.pp[3] = -16. * GWH_PI + 113. * dm * ca / 3 + (113. / 3 - 76. * eta / 3) * cs;
-    S.pp[4] = 15293365. / 508032 + 27145. * eta / 504 + 3085. * eta2 / 72 + (-405. / 8 + 200. * eta) * ca2 -
-              (405. / 4) * dm * ca * cs + (-405. / 8 + 5. * eta / 2) * cs2;
-    S.pp[7] = 77096675. * GWH_PI / 254016 + 378515. * GWH_PI * eta / 1512 - 74045. * GWH_PI * eta2 / 756 +
-              dm * (-25150083775. / 3048192 + 26804935. * eta / 6048 - 1985. * eta2 / 48) * ca +
-              (-25150083775. / 3048192 + 10566655595. * eta / 762048 - 1042165. * eta2 / 3024 + 5345. * eta3 / 36) * cs;
+    S.pp[2] = 3715. / 756 + 55. / 9 * eta;
+    S.pp[3] = -16. * GWH_PI + 113. / 3 * dm * ca + (113. / 3 - 76. / 3 * eta) * cs;
+    S.pp[4] = 15293365. / 508032 + 27145. / 504 * eta + 3085. / 72 * eta2 + (-405. / 8 + 200. * eta) * ca2 -
+              (405. / 4) * dm * ca * cs + (-405. / 8 + 5. / 2 * eta) * cs2;
+    S.pp[7] = 77096675. * GWH_PI / 254016 + 378515. * GWH_PI / 1512 * eta - 74045. * GWH_PI / 756 * eta2 +
+              dm * (-25150083775. / 3048192 + 26804935. / 6048 * eta - 1985. / 48 * eta2) * ca +
+              (-25150083775. / 3048192 + 10566655595. / 762048 * eta - 1042165. / 3024 * eta2 + 5345. / 36 * eta3) * cs;
     S.pp[8] = gwh_pn_c8_gr(eta, dm, ca, cs);
     S.pp[9] = S.pp[8];
-    S.pp[10] = 11583231236531. / 4694215680 - 6848. * GWH_GAMMA_E / 21 - 640. * pi2 / 3 +
-               (-15737765635. / 3048192 + 2255. * pi2 / 12) * eta + 76055. * eta2 / 1728 - 127825. * eta3 / 1296 +
-               2270. * dm * ca * GWH_PI / 3 + (2270. * GWH_PI / 3 - 520. * GWH_PI * eta) * cs -
-               6848. * (GWH_LOG_64) / 63;
+    S.pp[10] = 11583231236531. / 4694215680 - 6848. * GWH_GAMMA_E / 21 - 640. * pi2 / 3 - 6848. * (GWH_LOG_64) / 63 +
+               (-15737765635. / 3048192 + 2255. * pi2 / 12) * eta + 76055. / 1728 * eta2 - 127825. / 1296 * eta3 +
+               2270. * GWH_PI / 3 * dm * ca + (2270. * GWH_PI / 3 - 520. * GWH_PI * eta) * cs;
     S.pp[11] = 6848. / 63.;
     if (S.gimr) {
         const int direct[5] = {0, 2, 3, 4, 7};
@@ -860,10 +827,11 @@ __device__ __forceinline__ void gwh_setup_pn(const gwh_params &p, SetupState &S)
  * theory that cannot be mapped, give a NaN amplitude (and so a NaN likelihood). */
 __device__ __forceinline__ void gwh_setup_mass(const gwh_params &p, int ppe, SetupState &S)
 {
-    S.Mc = pow(S.m1 * S.m2, 0.6) / pow(S.M, 0.2);
+    S.Mc = S.M * exp(0.6 * log(S.eta)); /* (m1 m2)^(3/5) M^(-1/5) */
     double DL = p.DL * (GWH_MPC_SI / GWH_C_SI);
     double kA = p.sky_average ? sqrt(GWH_PI / 30.) : sqrt(GWH_PI * 40. / 192.);
-    S.A0 = kA * S.Mc * S.Mc / DL * pow(GWH_PI * S.Mc, -7. / 6.);
+    /* kA Mc^2 / DL (pi Mc)^(-7/6) */
+    S.A0 = kA * S.Mc * (1. / GWH_PI) / (DL * sqrt(cbrt(GWH_PI * S.Mc)));
     for (int i = 0; i < GWH_PPE_MAX; i++) S.ppe_e[i] = S.ppe_c[i] = 0.0;
     if (ppe == 1 || ppe == 2) {
         double b[GWH_PPE_MAX], beta[GWH_PPE_MAX];
@@ -882,13 +850,23 @@ __device__ __forceinline__ void gwh_setup_mass(const gwh_params &p, int ppe, Set
     }
 }
 
-/* role 2, phase 1: the Pv2 frame (IMRPhenomP.cpp:821-938, :1081-1211): thetaJN, alpha0, zeta and the
- * aligned-spin phase offset -phiJ */
+/* role 2, phase 1: the Pv2 frame (IMRPhenomP.cpp:821-938, :1081-1211): cosine and sine of thetaJN and of 2 zeta, alpha0
+ * and the aligned-spin phase offset -phiJ.  The reference turns every direction into an angle and back; here a rotation
+ * takes its cosine and sine from the direction's components, and only the two angles that enter a phase are formed. */
 struct Pv2Frame {
-    double thetaJN, alpha0, zeta, phi_aligned;
+    double cJN, sJN, c2z, s2z, alpha0, phi_aligned;
 };
-/* rotation by an angle given as its cosine and sine (the frame applies each of its three rotations several
- * times: one sincos per angle) */
+/* cosine and sine of atan2(y, x); atan2(0, 0) = 0.  Scaled by a power of 2, so that no square under- or overflows. */
+__device__ __forceinline__ void gwh_direction(double x, double y, double &c, double &s)
+{
+    const int e = -__builtin_amdgcn_frexp_exp(fmax(fabs(x), fabs(y)));
+    const bool none = (x == 0 && y == 0);
+    x = ldexp(x, e);
+    y = ldexp(y, e);
+    const double ih = none ? 0.0 : 1.0 / sqrt(x * x + y * y);
+    c = none ? 1.0 : x * ih;
+    s = y * ih;
+}
 __device__ __forceinline__ void gwh_rotz_cs(double c, double s, double &x, double &y)
 {
     double t1 = x * c - y * s, t2 = x * s + y * c;
@@ -907,12 +885,11 @@ __device__ __forceinline__ Pv2Frame gwh_setup_frame(const gwh_params &p, const S
     const double s1x = p.spin1[0], s1y = p.spin1[1], s2x = p.spin2[0], s2y = p.spin2[1];
     const bool reduced = (p.chip + 1) > 1e-10;
     const double m1_2 = S.m1 * S.m1, m2_2 = S.m2 * S.m2;
-    double xr = cbrt(GWH_PI * S.M * p.f_ref);
-    double L0 = S.M * S.M * gwh_l2pn(S.eta, xr * xr);
+    double L0 = S.M * S.M * gwh_l2pn(S.eta, cbrt(GWH_PI * S.M * p.f_ref));
     double J0x, J0y;
     if (reduced) {
         double sp, cp;
-        sincos(p.phip, &sp, &cp);
+        gwh_sincos_cw(p.phip, sp, cp);
         J0x = m1_2 * chip * cp;
         J0y = m1_2 * chip * sp;
     } else {
@@ -920,74 +897,66 @@ __device__ __forceinline__ Pv2Frame gwh_setup_frame(const gwh_params &p, const S
         J0y = m1_2 * s1y + m2_2 * s2y;
     }
     double J0z = L0 + m1_2 * S.chi1 + m2_2 * S.chi2;
-    double J0 = sqrt(J0x * J0x + J0y * J0y + J0z * J0z);
-    double thetaJ = acos(J0z / J0), phiJ = atan2(J0y, J0x);
-    double sJ, cJ, sP, cP; /* rotations by -thetaJ and -phiJ */
-    sincos(thetaJ, &sJ, &cJ);
-    sincos(phiJ, &sP, &cP);
-    sJ = -sJ;
+    /* rotation by -phiJ about z, then by -thetaJ about y */
+    double cP, sP, cJ, sJ, cK, sK;
+    gwh_direction(J0x, J0y, cP, sP);
+    gwh_direction(J0z, J0x * cP + J0y * sP, cJ, sJ);
     sP = -sP;
+    sJ = -sJ;
     Pv2Frame F;
-    F.phi_aligned = -phiJ;
-    double si, ci, sr, cr;
-    sincos(p.incl, &si, &ci);
-    sincos(GWH_PI / 2. - p.phiRef, &sr, &cr);
-    double Nx = si * cr, Ny = si * sr, Nz = ci;
-    double tx = Nx, ty = Ny, tz = Nz;
+    F.phi_aligned = -atan2(J0y, J0x);
+    double si, ci, sph, cph;
+    gwh_sincos_cw(p.incl, si, ci);
+    gwh_sincos_cw(p.phiRef, sph, cph);
+    /* line of sight N = (sin i cos(pi/2 - phi), sin i sin(pi/2 - phi), cos i), then rotated by kappa about z into the
+       x-z plane */
+    double tx = si * sph, ty = si * cph, tz = ci;
     gwh_rotz_cs(cP, sP, tx, ty);
     gwh_roty_cs(cJ, sJ, tx, tz);
-    double kappa = -atan2(ty, tx);
-    double sK, cK;
-    sincos(kappa, &sK, &cK);
-    tx = 0.;
+    gwh_direction(tx, -ty, cK, sK);
+    const double NxJ = tx * cK - ty * sK, NzJ = tz;
+    F.cJN = NzJ;
+    F.sJN = sqrt(tx * tx + ty * ty);
+    /* the orbital axis */
+    tx = sJ;
     ty = 0.;
-    tz = 1.;
-    gwh_rotz_cs(cP, sP, tx, ty);
-    gwh_roty_cs(cJ, sJ, tx, tz);
     gwh_rotz_cs(cK, sK, tx, ty);
     F.alpha0 = atan2(ty, tx);
-    tx = Nx;
-    ty = Ny;
-    tz = Nz;
-    gwh_rotz_cs(cP, sP, tx, ty);
-    gwh_roty_cs(cJ, sJ, tx, tz);
-    gwh_rotz_cs(cK, sK, tx, ty);
-    double NxJ = tx, NzJ = tz;
-    F.thetaJN = acos(NzJ);
-    double sph, cph;
-    sincos(p.phiRef, &sph, &cph);
     tx = -ci * sph;
     ty = -ci * cph;
     tz = si;
     gwh_rotz_cs(cP, sP, tx, ty);
     gwh_roty_cs(cJ, sJ, tx, tz);
     gwh_rotz_cs(cK, sK, tx, ty);
-    F.zeta = atan2(tx * NzJ - tz * NxJ, -ty);
+    double cz, sz;
+    gwh_direction(-ty, tx * NzJ - tz * NxJ, cz, sz);
+    F.c2z = cz * cz - sz * sz;
+    F.s2z = 2. * cz * sz;
     return F;
 }
 
 /* role 2, phase 1: polarisation constants and, per detector, the projection constants and the time-of-flight
  * phase slope (waveform_util.cpp:152-184, detector_util.cpp:768-790 and :900-1016) */
-__device__ __forceinline__ void gwh_setup_detectors(const gwh_params &p, bool pv2, double zeta, const DetGeom *geo,
-                                                    const int *dets, int ndet, InstCoef &C)
+__device__ __forceinline__ void gwh_setup_detectors(const gwh_params &p, bool pv2, double c2z, double s2z,
+                                                    const DetGeom *geo, const int *dets, int ndet, InstCoef &C)
 {
     /* the detectors' geometry is loaded before the trigonometry, which then covers the load latency */
     DetGeom gd[GWH_MAXDET];
 #pragma unroll
     for (int d = 0; d < GWH_MAXDET; d++)
         if (d < ndet) gd[d] = geo[dets[d]];
-    double ci = cos(p.incl);
+    double ci = 0, si = 0;
+    if (!pv2) gwh_sincos_cw(p.incl, si, ci);
     double kplus = .5 * (1. + ci * ci);
-    double c2z = cos(2. * zeta), s2z = sin(2. * zeta);
     const DetGeom &g0 = gd[0];
     C.wf_a = pv2 ? c2z : kplus;
     C.wf_b = pv2 ? s2z : ci;
     /* polarisation basis (shared by every detector) */
     const double gha = p.gmst - p.RA;
     double cg, sg, cd, sd, cp, sp;
-    sincos(gha, &sg, &cg);
-    sincos(p.DEC, &sd, &cd);
-    sincos(p.psi, &sp, &cp);
+    gwh_sincos_cw(gha, sg, cg);
+    gwh_sincos_cw(p.DEC, sd, cd);
+    gwh_sincos_cw(p.psi, sp, cp);
     const double X[3] = {-cp * sg - sp * cg * sd, -cp * cg + sp * sg * sd, sp * cd};
     const double Y[3] = {sp * sg - cp * cg * sd, sp * cg + cp * sg * sd, cp * cd};
     /* propagation direction for dt = (r0 - rd).n / c (hour angle gmst - RA) */
@@ -1007,7 +976,7 @@ __device__ __forceinline__ void gwh_setup_detectors(const gwh_params &p, bool pv
             fp *= g.gfac;
             fx *= g.gfac;
             double dt =
-                ((g0.loc[0] - g.loc[0]) * e0 + (g0.loc[1] - g.loc[1]) * e1 + (g0.loc[2] - g.loc[2]) * e2) / GWH_C_SI;
+                ((g0.loc[0] - g.loc[0]) * e0 + (g0.loc[1] - g.loc[1]) * e1 + (g0.loc[2] - g.loc[2]) * e2) * (1. / GWH_C_SI);
             if (!pv2) {
                 k0 = fp * kplus;
                 k1 = -fx * ci;
@@ -1027,14 +996,15 @@ __device__ __forceinline__ void gwh_setup_detectors(const gwh_params &p, bool pv
 
 /* role 2, phase 2: amplitude C1 connection, the Hermite quartic through (f1, v1, v1'), (f2, v2), (f3, v3, v3')
  * with f2 = (f1 + f3) / 2 (IMRPhenomD.cpp:1679-1702), as coefficients of powers of f */
-__device__ __forceinline__ void gwh_setup_amp_connection(double M, double f1, double f3, double v1, double d1,
+__device__ __forceinline__ void gwh_setup_amp_connection(double iM, double f1, double f3, double v1, double d1,
                                                          double v2, double v3, double d3, double *out)
 {
-    double f2 = (f1 + f3) / 2.;
-    double q12 = (v2 - v1) / (f2 - f1), q23 = (v3 - v2) / (f3 - f2);
-    double q012 = (q12 - d1) / (f2 - f1), q123 = (q23 - q12) / (f3 - f1), q234 = (d3 - q23) / (f3 - f2);
-    double q0123 = (q123 - q012) / (f3 - f1), q1234 = (q234 - q123) / (f3 - f1);
-    double q01234 = (q1234 - q0123) / (f3 - f1);
+    /* divided differences: f2 lies midway, so every difference is h = (f3 - f1) / 2 or 2 h */
+    const double f2 = (f1 + f3) / 2., ih = 2. / (f3 - f1), ih2 = 0.5 * ih;
+    const double q12 = (v2 - v1) * ih, q23 = (v3 - v2) * ih;
+    const double q012 = (q12 - d1) * ih, q123 = (q23 - q12) * ih2, q234 = (d3 - q23) * ih;
+    const double q0123 = (q123 - q012) * ih2, q1234 = (q234 - q123) * ih2;
+    const double q01234 = (q1234 - q0123) * ih2;
     double a[5] = {v1, d1, q012, q0123, q01234};
     double z[4] = {f1, f1, f2, f3};
     double poly[5] = {a[4], 0, 0, 0, 0};
@@ -1050,70 +1020,35 @@ __device__ __forceinline__ void gwh_setup_amp_connection(double M, double f1, do
 #pragma unroll
         for (int j = 0; j < 5; j++) poly[j] = nw[j];
     }
-    double Mk = 1.0;
+    double k = 1.0;
 #pragma unroll
-    for (int k = 0; k < 5; k++) {
-        out[k] = poly[k] / Mk;
-        Mk *= M;
+    for (int q = 0; q < 5; q++) {
+        out[q] = poly[q] * k;
+        k *= iM;
     }
 }
 
-/* phase 3: derivative at fRD of the natural cubic spline through the 10 knots (f_j, ph_j) on [0.8, 1.2] fRD
- * (IMRPhenomP.cpp:550-606), divided by 2 pi; 0 when the knots collapse */
-__device__ __forceinline__ double gwh_setup_tcorr(double fRD, const double *ph)
+/* phase 3: derivative at fRD of the natural cubic spline through the values q at the 10 knots on [0.8, 1.2] fRD
+ * (IMRPhenomP.cpp:550-606).  fRD lies midway between knots 4 and 5 and the knots are evenly spaced, so the spline's
+ * tridiagonal system has one solution for all instances: the derivative is a fixed combination of the differences of
+ * values on either side, +-{265/204, 5/34, 2/51, 1/102, 1/612} with alternating signs, over the spacing; 0 when the
+ * knots collapse. */
+__device__ __forceinline__ double gwh_setup_tcorr(double fRD, const double *q)
 {
-    const int n = 10;
-    double start = .8 * fRD, stop = 1.2 * fRD;
-    double df = (stop - start) / (n - 1);
+    const double df = 0.4 * fRD / 9;
     if (!(df > 0)) return 0;
-    double fs[10], c[10], dg[10], rh[10], of[10];
-#pragma unroll
-    for (int j = 0; j < n; j++) fs[j] = start + j * df;
-    const int m = n - 2;
-#pragma unroll
-    for (int i = 0; i < m; i++) {
-        double h0 = fs[i + 1] - fs[i], h1 = fs[i + 2] - fs[i + 1];
-        dg[i] = 2.0 * (h0 + h1);
-        of[i] = h1;
-        rh[i] = 3.0 * ((ph[i + 2] - ph[i + 1]) / h1 - (ph[i + 1] - ph[i]) / h0);
-    }
-#pragma unroll
-    for (int i = 1; i < m; i++) {
-        double w = of[i - 1] / dg[i - 1];
-        dg[i] -= w * of[i - 1];
-        rh[i] -= w * rh[i - 1];
-    }
-    c[0] = 0;
-    c[n - 1] = 0;
-    c[m] = rh[m - 1] / dg[m - 1];
-#pragma unroll
-    for (int i = m - 2; i >= 0; i--) c[i + 1] = (rh[i] - of[i] * c[i + 2]) / dg[i];
-    /* interval holding fRD (the bisection's answer, found by an unrolled scan so that every array index is a
-     * compile-time constant and the arrays stay in registers) */
-    double x0 = fs[0], x1 = fs[1], y0 = ph[0], y1 = ph[1], c0 = c[0], c1 = c[1];
-#pragma unroll
-    for (int j = 1; j < n - 1; j++)
-        if (fs[j] <= fRD) {
-            x0 = fs[j];
-            x1 = fs[j + 1];
-            y0 = ph[j];
-            y1 = ph[j + 1];
-            c0 = c[j];
-            c1 = c[j + 1];
-        }
-    double h = x1 - x0;
-    double b = (y1 - y0) / h - h * (c1 + 2.0 * c0) / 3.0;
-    double dd = (c1 - c0) / (3.0 * h);
-    double dx = fRD - x0;
-    return (b + dx * (2.0 * c0 + 3.0 * dd * dx)) / GWH_2PI;
+    const double s = (265. / 204.) * (q[5] - q[4]) - (5. / 34.) * (q[6] - q[3]) + (2. / 51.) * (q[7] - q[2]) -
+                     (1. / 102.) * (q[8] - q[1]) + (1. / 612.) * (q[9] - q[0]);
+    return s / df;
 }
 
 /* the t_c spline's knot j: 0.8 fRD + j (0.4 fRD / 9) */
 __device__ __forceinline__ double gwh_setup_knot(double fRD, int j)
 {
     double start = .8 * fRD, stop = 1.2 * fRD;
-    return start + j * ((stop - start) / 9);
+    return start + j * ((stop - start) * (1. / 9));
 }
+#pragma clang fp contract(fast)
 
 /* ------------------------------------------------------------------------- */
 /* per-bin FP64 evaluation                                                    */

@@ -2,12 +2,11 @@
  * gwh_trig.h -- sine and cosine of FP64 phases for the per-bin kernels.
  *
  * Phases of the hot path reach ~1e5-1e6 rad (2 pi f t_c plus the inspiral phase).  The library sincos of
- * FP64 carries a large-argument (Payne-Hanek) reduction for every call; here the argument is reduced by
- * Cody and Waite's method (W. J. Cody, W. Waite, Software Manual for the Elementary Functions, 1980):
+ * FP64 carries a large-argument (Payne-Hanek) reduction for every call; gwh_sincos_cw, for the per-instance setup,
+ * reduces by Cody and Waite's method (W. J. Cody, W. Waite, Software Manual for the Elementary Functions, 1980):
  * q = rint(x 2/pi), r = (x - q p1) - q p2 with pi/2 = p1 + p2 split into two doubles and each step one
- * fused multiply-add (x - q p1 is exact by Sterbenz's lemma, the neglected part of pi/2 is 1e-33, so r is
- * within half an ulp for |x| < 2^30), then sin r and cos r on [-pi/4, pi/4] by their Taylor series and the
- * quadrant by q mod 4.  Arguments beyond 2^30 rad take the library routine.
+ * fused multiply-add (x - q p1 is exact by Sterbenz's lemma, the neglected part of pi/2 is 1e-33), then sin r and
+ * cos r on [-pi/4, pi/4] by their Taylor series and the quadrant by q mod 4.
  *
  * gwh_sincos_table and gwh_exp_table trade the long series for a table lookup (gwh_trig_tables.h, 4.5 kB,
  * correctly rounded entries) and a short series on a tiny remainder: ~20 FP64 operations and one gather for
@@ -20,45 +19,53 @@
 
 #include "gwh_trig_tables.h"
 
-/* NT: highest odd power of the sine series (15: truncation below 5e-17 on [-pi/4, pi/4]; 11: below 7e-12) */
-template <int NT> __device__ __forceinline__ void gwh_sincos_cw(double x, double &s, double &c)
+/* sin and cos beyond gwh_sincos_cw's range (and of infinities and NaN): one copy of the library's long reduction */
+__device__ __noinline__ double2 gwh_sincos_huge(double x)
 {
-    static_assert(NT == 15 || NT == 11, "series length");
-    if (!(fabs(x) < 1073741824.0)) { /* |x| >= 2^30 or NaN */
-        sincos(x, &s, &c);
+    double s, c;
+    sincos(x, &s, &c);
+    return make_double2(s, c);
+}
+
+/* sin and cos for the setup (a handful of angles per instance), within an ulp: about 45 instructions inlined, where the
+ * library's sincos carries its second reduction, for huge arguments, at every call site. */
+#pragma clang fp contract(on)
+__device__ __forceinline__ void gwh_sincos_cw(double x, double &s, double &c)
+{
+    if (!(fabs(x) < 1099511627776.0)) { /* 2^40: up to there x - q p1 fits a double */
+        const double2 r = gwh_sincos_huge(x);
+        s = r.x;
+        c = r.y;
         return;
     }
     const double q = rint(x * 0.63661977236758134308);
     double r = fma(-q, 1.5707963267948966192, x);
     r = fma(-q, 6.123233995736766036e-17, r);
     const double r2 = r * r;
-    /* sin r = r + r^3 sum_k (-1)^k r^(2k) / (2k+3)!,  cos r = 1 - r^2/2 + r^4 sum_k (-1)^k r^(2k) / (2k+4)! */
+    /* sin r = r + r^3 sum_k (-1)^k r^(2k) / (2k+3)!,  cos r = 1 - r^2/2 + r^4 sum_k (-1)^k r^(2k) / (2k+4)!, to r^15 and
+       r^16: truncation below 5e-17 on [-pi/4, pi/4] */
     double ps, pc;
-    if (NT == 15) {
-        ps = fma(-7.6471637318198164759e-13, r2, 1.6059043836821614599e-10); /* -1/15!, 1/13! */
-        ps = fma(ps, r2, -2.5052108385441718775e-08);                        /* -1/11! */
-        ps = fma(ps, r2, 2.7557319223985890653e-06);                         /* 1/9! */
-        pc = fma(4.7794773323873852974e-14, r2, -1.1470745597729724714e-11); /* 1/16!, -1/14! */
-        pc = fma(pc, r2, 2.0876756987868098979e-09);                         /* 1/12! */
-        pc = fma(pc, r2, -2.7557319223985890653e-07);                        /* -1/10! */
-    } else {
-        ps = fma(-2.5052108385441718775e-08, r2, 2.7557319223985890653e-06); /* -1/11!, 1/9! */
-        pc = fma(2.0876756987868098979e-09, r2, -2.7557319223985890653e-07); /* 1/12!, -1/10! */
-    }
-    ps = fma(ps, r2, -1.9841269841269841270e-04); /* -1/7! */
-    ps = fma(ps, r2, 8.3333333333333333333e-03);  /* 1/5! */
-    ps = fma(ps, r2, -1.6666666666666666667e-01); /* -1/3! */
-    pc = fma(pc, r2, 2.4801587301587301587e-05);  /* 1/8! */
-    pc = fma(pc, r2, -1.3888888888888888889e-03); /* -1/6! */
-    pc = fma(pc, r2, 4.1666666666666666667e-02);  /* 1/4! */
+    ps = fma(-7.6471637318198164759e-13, r2, 1.6059043836821614599e-10); /* -1/15!, 1/13! */
+    ps = fma(ps, r2, -2.5052108385441718775e-08);                        /* -1/11! */
+    ps = fma(ps, r2, 2.7557319223985890653e-06);                         /* 1/9! */
+    ps = fma(ps, r2, -1.9841269841269841270e-04);                        /* -1/7! */
+    ps = fma(ps, r2, 8.3333333333333333333e-03);                         /* 1/5! */
+    ps = fma(ps, r2, -1.6666666666666666667e-01);                        /* -1/3! */
+    pc = fma(4.7794773323873852974e-14, r2, -1.1470745597729724714e-11); /* 1/16!, -1/14! */
+    pc = fma(pc, r2, 2.0876756987868098979e-09);                         /* 1/12! */
+    pc = fma(pc, r2, -2.7557319223985890653e-07);                        /* -1/10! */
+    pc = fma(pc, r2, 2.4801587301587301587e-05);                         /* 1/8! */
+    pc = fma(pc, r2, -1.3888888888888888889e-03);                        /* -1/6! */
+    pc = fma(pc, r2, 4.1666666666666666667e-02);                         /* 1/4! */
     pc = fma(pc, r2, -0.5);
     const double sr = fma(ps * r2, r, r);
     const double cr = fma(pc, r2, 1.0);
-    const int iq = (int)q;
+    const int iq = (int)(long long)q;
     const double ss = (iq & 1) ? cr : sr, cc = (iq & 1) ? sr : cr;
     s = (iq & 2) ? -ss : ss;
     c = ((iq + 1) & 2) ? -cc : cc;
 }
+#pragma clang fp contract(fast)
 
 /* sin and cos of an FP64 phase through the table: the phase in turns r = n / 256 + y with n the nearest integer
  * to 256 r (rounded by the 1.5 * 2^52 addition, whose low mantissa bits then hold n mod 256) and y = r - n / 256
