@@ -944,7 +944,7 @@ static int fisher_run(int event, int model, int basis, int precision, const gwh_
             double fcut = 0;
             for (const gwh_params &p : inst) {
                 const double c = .2 / (p.mass1 * GWH_MSOL_SEC + p.mass2 * GWH_MSOL_SEC);
-                fcut = (c <= fcut) ? fcut : c; /* NaN: every chunk */
+                if (!(c <= fcut || fcut != fcut)) fcut = c; /* NaN stays: every chunk */
             }
             const std::vector<double> &cf = *ev.chunk_fmin;
             while (nb > 1 && cf[nb - 1] > fcut * (1 + 1e-9)) nb--;

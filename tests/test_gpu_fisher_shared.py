@@ -95,3 +95,18 @@ def test_points_of_very_different_mass_share_a_pass():
         s = sum(G.fisher_numerical(f, psd, G.BASIS_PHENOMD_MCMC, d, 0, 11, p, epsilon=-1e-7) for d in range(3))
         assert _norm_err(F[i], s) <= TOL
     ev.close()
+
+
+def test_a_point_without_masses_leaves_the_others_alone():
+    """the batch's chunks end at the highest cutoff 0.2 / M of its points; one without a cutoff does not hide the
+    light point before it behind the heavy point after it"""
+    f = W.uniform_grid(20., 2048., 0.5)
+    psd = W.analytic_psd(f)
+    ev = G.Event(f, [np.zeros(len(f), complex)], [psd], [0])
+    P = W.perturbed_params(W.injection_params(1)[0], 3, step=1)
+    P["mass1"], P["mass2"] = [8., np.nan, 90.], [6., 20., 70.]
+    a = G.fisher_batch(ev, P, G.IMRPHENOMD, G.BASIS_PHENOMD_FULL, 11, epsilon=1e-6)
+    for i in (0, 2):
+        alone = G.fisher_batch(ev, P[i:i + 1], G.IMRPHENOMD, G.BASIS_PHENOMD_FULL, 11, epsilon=1e-6)[0]
+        assert np.linalg.norm(a[i] - alone) <= 1e-12 * np.linalg.norm(alone)
+    ev.close()
