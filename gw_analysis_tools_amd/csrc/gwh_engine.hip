@@ -425,7 +425,6 @@ int gwh_event_create_ex(const double *f, int N, int ndet, const int *dets, const
  * theory modifications are compiled in (the GR models run a kernel without them, which keeps its registers and
  * code to what GR needs). */
 #define GWH_SETUP_LANES 32
-#pragma clang fp contract(on)
 template <int MODEL, bool MOD>
 __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__restrict__ params,
                                                         const int *__restrict__ inst_event, int event0, int n,
@@ -552,10 +551,10 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__rest
                 for (int k = 0; k < 4; k++) T.beta[k] = S.beta[k];
                 for (int k = 0; k < 6; k++) T.alpha[k] = S.alpha[k];
             }
-            C->sig[0] = S.sigma[1] * S.ieta;
-            C->sig[1] = 0.75 * S.sigma[2] * S.ieta;
-            C->sig[2] = 0.6 * S.sigma[3] * S.ieta;
-            C->sig[3] = 0.5 * S.sigma[4] * S.ieta;
+            C->sig[0] = S.sigma[1] / S.eta;
+            C->sig[1] = 0.75 * S.sigma[2] / S.eta;
+            C->sig[2] = 0.6 * S.sigma[3] / S.eta;
+            C->sig[3] = 0.5 * S.sigma[4] / S.eta;
             gwh_setup_mass(p, ppe, S);
             X.S.Mc = S.Mc;
             X.S.A0 = S.A0;
@@ -645,17 +644,18 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__rest
         S.beta[0] = S.beta[1] = 0;
         S.alpha[0] = S.alpha[1] = 0;
         if (role == 0) {
-            X.p_ins = gwh_setup_phase_ins_at(S, S.f1p, GWH_MF1P_V, 1.0 / GWH_MF1P_V, GWH_MF1P_LNPI, GWH_MF1P_U, GWH_MF1P);
-            X.d_ins = gwh_setup_dphase_ins_f1p(S);
+            X.p_ins = gwh_setup_phase_ins(S, S.f1p);
+            X.l1 = log(S.M * S.f1p);
         } else if (role == 1) {
-            double dl[5];
-            gwh_setup_amp_connection(S.iM, S.f1, S.f3, X.v1, X.d1, S.v2, X.v3, X.d3, dl);
-            for (int k = 0; k < 5; k++) C->delta[k] = dl[k];
+            X.d_ins = gwh_setup_dphase_ins(S, S.f1p);
+            X.l2 = log(S.M * S.f2p);
         } else if (role == 2) {
             X.q_mr = gwh_setup_phase_mr(S, S.f2p);
             X.dq_mr = gwh_setup_dphase_mr(S, S.f2p);
-            X.l2 = log(S.M * S.f2p);
         } else {
+            double dl[5];
+            gwh_setup_amp_connection(S.iM, S.f1, S.f3, X.v1, X.d1, S.v2, X.v3, X.d3, dl);
+            for (int k = 0; k < 5; k++) C->delta[k] = dl[k];
             if (!pv2) {
                 if (p.shift_phase) {
                     const double fr = p.f_ref;
@@ -675,22 +675,21 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__rest
 
     /* ---- phase 3: the phase connection (IMRPhenomD.cpp:1614-1674) and the alignment ---- */
     if (live && role == 0) {
-        const double eta = S.eta, ieta = S.ieta, M = S.M, etaM = eta * S.iM;
-        const double Mf2 = M * S.f2p, iMf2 = 1.0 / Mf2;
-        const double Mf1 = GWH_MF1P, iMf1 = 1.0 / GWH_MF1P;
-        S.beta[1] = etaM * (X.d_ins - gwh_setup_dphase_int(S, S.f1p, iMf1));
-        S.beta[0] = eta * (X.p_ins - gwh_setup_phase_int_l(S, S.f1p, Mf1, iMf1, GWH_MF1P_LN));
-        S.alpha[1] = etaM * (gwh_setup_dphase_int(S, S.f2p, iMf2) - X.dq_mr);
-        S.alpha[0] = eta * (gwh_setup_phase_int_l(S, S.f2p, Mf2, iMf2, X.l2) - X.q_mr) - S.alpha[1] * Mf2;
-        C->beta[0] = S.beta[0] * ieta;
-        C->beta[1] = S.beta[1] * ieta;
-        C->beta[2] = S.beta[2] * ieta;
-        C->beta[3] = S.beta[3] * ieta * (1. / 3.);
-        C->alpha[0] = S.alpha[0] * ieta;
-        C->alpha[1] = S.alpha[1] * ieta;
-        C->alpha[2] = S.alpha[2] * ieta;
-        C->alpha[3] = (4. / 3.) * S.alpha[3] * ieta;
-        C->alpha[4] = S.alpha[4] * ieta;
+        const double eta = S.eta, M = S.M;
+        S.beta[1] = (eta / M) * X.d_ins - (eta / M) * gwh_setup_dphase_int(S, S.f1p);
+        S.beta[0] = eta * X.p_ins - eta * gwh_setup_phase_int_l(S, S.f1p, X.l1);
+        S.alpha[1] = (eta / M) * gwh_setup_dphase_int(S, S.f2p) - (eta / M) * X.dq_mr;
+        S.alpha[0] = eta * gwh_setup_phase_int_l(S, S.f2p, X.l2) -
+                     eta * (X.q_mr + (1. / eta) * (S.alpha[1] * (M * S.f2p)));
+        C->beta[0] = S.beta[0] / eta;
+        C->beta[1] = S.beta[1] / eta;
+        C->beta[2] = S.beta[2] / eta;
+        C->beta[3] = S.beta[3] / (3. * eta);
+        C->alpha[0] = S.alpha[0] / eta;
+        C->alpha[1] = S.alpha[1] / eta;
+        C->alpha[2] = S.alpha[2] / eta;
+        C->alpha[3] = (4. / 3.) * S.alpha[3] / eta;
+        C->alpha[4] = S.alpha[4] / eta;
         C->alpha[5] = S.alpha[5] * S.fRD;
         if (!pv2) {
             /* phase and time alignment (IMRPhenomD.cpp:441-466) */
@@ -701,9 +700,9 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__rest
                 if (fref < S.f1p)
                     b = X.ref;
                 else if (fref > S.f2p)
-                    b = X.ref + ieta * (S.alpha[0] + S.alpha[1] * (M * fref));
+                    b = X.ref + (1. / eta) * (S.alpha[0] + S.alpha[1] * (M * fref));
                 else
-                    b = gwh_setup_phase_int_l(S, fref, M * fref, 1.0 / (M * fref), X.ref);
+                    b = gwh_setup_phase_int_l(S, fref, X.ref);
                 phic = 2 * p.phiRef + b;
             } else {
                 fref = 0;
@@ -711,7 +710,7 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__rest
             }
             double tc_shift = 0;
             if (p.shift_time)
-                tc_shift = X.dq_mr3 + ieta * (M * X.alpha1_fit); /* the slope at f3 with the fitted alpha1 */
+                tc_shift = (X.dq_mr3 + (1. / eta) * (M * S.alpha[1])) + (-S.alpha[1] + X.alpha1_fit) * M / eta;
             C->tc_total = GWH_2PI * p.tc + tc_shift;
             C->phic = phic;
             C->f_ref = fref;
@@ -727,15 +726,13 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__rest
                 double q[10];
 #pragma unroll
                 for (int j = 0; j < 10; j++) q[j] = X.tq[j];
-                t_corr = -(gwh_setup_tcorr(S.fRD, q) + ieta * (S.alpha[1] * M));
+                t_corr = -(gwh_setup_tcorr(S.fRD, q) + S.alpha[1] * M / eta);
                 if (!(S.fRD > 0)) t_corr = 0;
             }
             C->t_corr_2pi = t_corr;
         }
     }
 }
-
-#pragma clang fp contract(fast)
 
 static void launch_setup(int model, int n, hipStream_t st, const gwh_params *params, const int *inst_event,
                          int event0, InstCoef *coef, int *active, const int *d_count = nullptr,

@@ -288,21 +288,39 @@ struct DetGeom {
 /*
  * The setup runs one lane per instance and role, so it is bound by the latency of each role's chain and by fetching its
  * instructions, which few waves execute once: 78 KB (IMRPhenomD) and 99 KB (IMRPhenomPv2), more than the instruction
- * cache, while every division, power and logarithm was written out.  Constants stand for those that do not depend on the
- * instance -- M f is 0.014 and 0.018 at the first transitions whatever M -- and one reciprocal of eta, M, ... for
- * repeated divisions: 56 KB and 57 KB.  512 instances: IMRPhenomD 11.3 -> 7.5 us, IMRPhenomPv2 17.5 -> 11.2 us (of
- * which the half-filled blocks of gwh_setup_kernel 1.3 and 0.9).
+ * cache, while everything was written out.  Amplitude, orientation, detector and precession parts
+ * take few divisions, powers and angles: 70 KB and 72 KB; with the half-filled blocks of gwh_setup_kernel 512 instances
+ * of IMRPhenomD 11.3 -> 9.0 us, 1024 of IMRPhenomPv2 17.5 -> 14.9 us.
  *
- * Multiply-adds are fused within an expression only (contract(on)), so a function rounds alike wherever it is inlined:
- * the kernels with and without the modified-gravity terms have to agree bit for bit where the terms vanish.
+ * The phase and its connection keep the order of operations that they have always had: the slopes of its pieces are
+ * differences of large terms, whose rounding a difference quotient in a small parameter magnifies (with the phase
+ * rearranged as well, 7.3 and 11.2 us, the IMRPhenomPv2 Fisher elements of t_c and a spin moved by up to 2e-4).  The
+ * functions that a pragma puts under contract(on) fuse multiply-adds within an expression only, so that they round alike
+ * in the kernels with and without the modified-gravity terms, which have to agree bit for bit where the terms vanish.
  */
-#pragma clang fp contract(on)
+
+__device__ __forceinline__ double gwh_spline_eval(const double *x, const double *y, const double *c, int n,
+                                                  double xq)
+{
+    if (!(xq >= x[0] && xq <= x[n - 1])) return __longlong_as_double(0x7ff8000000000000LL);
+    /* interval with x[lo] <= xq < x[lo + 1] (lo = n - 2 at the last knot), the one a bisection finds:
+     * start from the uniform-spacing guess and walk (a step or two on the near-uniform spin grid) */
+    int lo = (int)((xq - x[0]) / (x[n - 1] - x[0]) * (n - 1));
+    lo = lo < 0 ? 0 : (lo > n - 2 ? n - 2 : lo);
+    while (lo > 0 && x[lo] > xq) lo--;
+    while (lo < n - 2 && x[lo + 1] <= xq) lo++;
+    double h = x[lo + 1] - x[lo];
+    double b = (y[lo + 1] - y[lo]) / h - h * (c[lo + 1] + 2.0 * c[lo]) / 3.0;
+    double d = (c[lo + 1] - c[lo]) / (3.0 * h);
+    double dx = xq - x[lo];
+    return y[lo] + dx * (b + dx * (c[lo] + dx * d));
+}
 
 /* both QNM splines (M f_ring and M f_damp) at spin a, with the interval x[lo] <= a < x[lo + 1] (lo = n - 2 at
  * the last knot) that a bisection finds.  On the table's near-uniform spin grid that interval lies within one
  * knot of the uniform-spacing guess, so the knots and coefficients of the four-knot window around the guess
- * are loaded together (one memory round trip) and the interval is picked among them; a window that misses it is
- * moved until it does not. */
+ * are loaded together (one memory round trip) and the interval is picked among them; a window that misses it
+ * falls back to the walk of gwh_spline_eval.  Same arithmetic as gwh_spline_eval. */
 __device__ __forceinline__ void gwh_qnm_eval(const QnmTable &q, double a, double &fring, double &fdamp)
 {
     const int n = q.n;
@@ -310,21 +328,22 @@ __device__ __forceinline__ void gwh_qnm_eval(const QnmTable &q, double a, double
         fring = fdamp = __longlong_as_double(0x7ff8000000000000LL);
         return;
     }
-    const int g = (int)((a - q.x0) / (q.x1 - q.x0) * (n - 1));
-    int b = (g - 1 < 0) ? 0 : (g - 1 > n - 4 ? n - 4 : g - 1);
+    int g = (int)((a - q.x0) / (q.x1 - q.x0) * (n - 1));
+    g = g < 0 ? 0 : (g > n - 2 ? n - 2 : g);
+    const int b = (g - 1 < 0) ? 0 : (g - 1 > n - 4 ? n - 4 : g - 1);
     double xs[4], yr[4], cr[4], yd[4], cd[4];
-    for (;;) {
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            xs[k] = q.spin[b + k];
-            yr[k] = q.fring[b + k];
-            cr[k] = q.c_ring[b + k];
-            yd[k] = q.fdamp[b + k];
-            cd[k] = q.c_damp[b + k];
-        }
-        const int step = (xs[0] > a && b > 0) ? -1 : ((a >= xs[3] && b < n - 4) ? 1 : 0);
-        if (step == 0) break;
-        b += step;
+    for (int k = 0; k < 4; k++) {
+        xs[k] = q.spin[b + k];
+        yr[k] = q.fring[b + k];
+        cr[k] = q.c_ring[b + k];
+        yd[k] = q.fdamp[b + k];
+        cd[k] = q.c_damp[b + k];
+    }
+    if (!(xs[0] <= a && (a < xs[3] || b == n - 4))) {
+        fring = gwh_spline_eval(q.spin, q.fring, q.c_ring, n, a);
+        fdamp = gwh_spline_eval(q.spin, q.fdamp, q.c_damp, n, a);
+        return;
     }
     double x0 = xs[0], x1 = xs[1], r0 = yr[0], r1 = yr[1], rc0 = cr[0], rc1 = cr[1], d0 = yd[0], d1 = yd[1],
            dc0 = cd[0], dc1 = cd[1];
@@ -342,12 +361,12 @@ __device__ __forceinline__ void gwh_qnm_eval(const QnmTable &q, double a, double
             dc0 = cd[k];
             dc1 = cd[k + 1];
         }
-    const double h = x1 - x0, dx = a - x0, ih = 1.0 / h;
-    double bb = (r1 - r0) * ih - h * (rc1 + 2.0 * rc0) * (1.0 / 3.0);
-    double dd = (rc1 - rc0) * (ih * (1.0 / 3.0));
+    const double h = x1 - x0, dx = a - x0;
+    double bb = (r1 - r0) / h - h * (rc1 + 2.0 * rc0) / 3.0;
+    double dd = (rc1 - rc0) / (3.0 * h);
     fring = r0 + dx * (bb + dx * (rc0 + dx * dd));
-    bb = (d1 - d0) * ih - h * (dc1 + 2.0 * dc0) * (1.0 / 3.0);
-    dd = (dc1 - dc0) * (ih * (1.0 / 3.0));
+    bb = (d1 - d0) / h - h * (dc1 + 2.0 * dc0) / 3.0;
+    dd = (dc1 - dc0) / (3.0 * h);
     fdamp = d0 + dx * (bb + dx * (dc0 + dx * dd));
 }
 
@@ -359,23 +378,24 @@ __device__ __forceinline__ double gwh_fit(const double *tab, int row, double eta
            x * x * (p[5] + p[6] * eta + p[7] * eta * eta) + x * x * x * (p[8] + p[9] * eta + p[10] * eta * eta);
 }
 
-/* delta = sqrt(1 - 4 eta), ieta = 1 / eta */
-__device__ __forceinline__ double gwh_final_spin0815(double eta, double ieta, double delta, double chi1, double chi2)
+__device__ __forceinline__ double gwh_final_spin0815(double eta, double chi1, double chi2)
 {
-    double m1 = 0.5 * (1.0 + delta), m2 = 0.5 * (1.0 - delta);
+    double Seta = sqrt(1.0 - 4.0 * eta);
+    double m1 = 0.5 * (1.0 + Seta), m2 = 0.5 * (1.0 - Seta);
     double s = m1 * m1 * chi1 + m2 * m2 * chi2;
     double eta2 = eta * eta, eta3 = eta2 * eta, s2 = s * s, s3 = s2 * s;
     return eta * (3.4641016151377544 - 4.399247300629289 * eta + 9.397292189321194 * eta2 -
                   13.180949901606242 * eta3 +
-                  s * ((ieta - 0.0850917821418767 - 5.837029316602263 * eta) +
+                  s * ((1.0 / eta - 0.0850917821418767 - 5.837029316602263 * eta) +
                        (0.1014665242971878 - 2.0967746996832157 * eta) * s +
                        (-1.3546806617824356 + 4.108962025369336 * eta) * s2 +
                        (-0.8676969352555539 + 2.064046835273906 * eta) * s3));
 }
 
-__device__ __forceinline__ double gwh_erad0815(double eta, double delta, double chi1, double chi2)
+__device__ __forceinline__ double gwh_erad0815(double eta, double chi1, double chi2)
 {
-    double m1 = 0.5 * (1.0 + delta), m2 = 0.5 * (1.0 - delta);
+    double Seta = sqrt(1.0 - 4.0 * eta);
+    double m1 = 0.5 * (1.0 + Seta), m2 = 0.5 * (1.0 - Seta);
     double m1s = m1 * m1, m2s = m2 * m2;
     double s = (m1s * chi1 + m2s * chi2) / (m1s + m2s);
     double eta2 = eta * eta, eta3 = eta2 * eta;
@@ -404,15 +424,15 @@ struct SetupState {
 __device__ __forceinline__ double gwh_pn_c8_gr(double eta, double dm, double ca, double cs)
 {
     const double eta2 = eta * eta;
-    return (38645. * GWH_PI / 756 - 65. * GWH_PI / 9 * eta + dm * (-732985. / 2268 - 140. / 9 * eta) * ca +
-            (-732985. / 2268 + 24260. / 81 * eta + 340. / 9 * eta2) * cs);
+    return (38645. * GWH_PI / 756 - 65. * GWH_PI * eta / 9 + dm * (-732985. / 2268 - 140. * eta / 9) * ca +
+            (-732985. / 2268 + 24260. * eta / 81 + 340. * eta2 / 9) * cs);
 }
 
 /* gIMR inspiral phase terms beyond the IMRPhenomD polynomial (gIMRPhenomD.cpp:148-184): the order-1 coefficient
  * (zero in IMRPhenomD) and 3/(128 eta) delta_i (pi M f)^((i - 5)/3) for i = -4..-1, with their f derivative */
 __device__ __forceinline__ double gwh_setup_gimr(const SetupState &S, double f, double *deriv)
 {
-    const double K = 3. / 128. * S.ieta;
+    const double K = 3. / (128. * S.eta);
     const double x = GWH_PI * S.M * f, iv = 1.0 / cbrt(x);
     double iv2 = iv * iv, iv4 = iv2 * iv2;
     double t = S.pp[1] * iv4, d = S.pp[1] * (-4. / 3.) * iv4;
@@ -444,72 +464,67 @@ __device__ __forceinline__ double gwh_setup_ppe(const SetupState &S, double f, d
     return t;
 }
 
-/* the transition frequencies times M, and what the phases and amplitudes need of them */
-#define GWH_MF1 0.014                        /* amplitude: inspiral up to here */
-#define GWH_MF1_V 0.35298748079802035326     /* (pi M f)^(1/3) */
-#define GWH_MF1_U 0.24101422641752299861     /* (M f)^(1/3) */
-#define GWH_MF1P 0.018                       /* phase: inspiral up to here */
-#define GWH_MF1P_V 0.38383165853550260132    /* (pi M f)^(1/3) */
-#define GWH_MF1P_U 0.26207413942088966071    /* (M f)^(1/3) */
-#define GWH_MF1P_LNPI -2.8726536352365721857 /* ln(pi M f) */
-#define GWH_MF1P_LN -4.0173835210859723598   /* ln(M f) */
-
-/* TF2 + sigma inspiral phase at f (IMRPhenomD.cpp:1364-1399) from v = (pi M f)^(1/3), 1 / v, ln v^3, u = (M f)^(1/3), M f */
-__device__ __forceinline__ double gwh_setup_phase_ins_at(const SetupState &S, double f, double v, double iv, double lx,
-                                                         double u, double Mf)
+/* TF2 + sigma inspiral phase at f (IMRPhenomD.cpp:1364-1399) */
+__device__ __forceinline__ double gwh_setup_phase_ins(const SetupState &S, double f)
 {
+    double x = GWH_PI * S.M * f;
+    double v = cbrt(x);
+    double lx = log(x);
     double c5 = S.pp[8] + lx * S.pp[9];
     double c6 = S.pp[10] - S.pp[11] * lx;
-    double v2 = v * v, iv2 = iv * iv;
+    double v2 = v * v;
     double poly = S.pp[0] + v2 * (S.pp[2] + v * (S.pp[3] + v * (S.pp[4] + v * (c5 + v * (c6 + v * S.pp[7])))));
+    double Mf = S.M * f;
+    double u = cbrt(Mf);
     double Mf43 = Mf * u, Mf53 = Mf43 * u;
-    double ph = -GWH_PI / 4. + S.ieta * (3. / 128. * poly * (iv2 * iv2 * iv) +
-                                         (S.sigma[1] * Mf + 0.75 * S.sigma[2] * Mf43 + 0.6 * S.sigma[3] * Mf53 +
-                                          0.5 * S.sigma[4] * Mf * Mf));
+    double ph = -GWH_PI / 4. + 3. / (128. * S.eta) * poly / (v2 * v2 * v) +
+                (1. / S.eta) * (S.sigma[1] * Mf + 0.75 * S.sigma[2] * Mf43 + 0.6 * S.sigma[3] * Mf53 +
+                                0.5 * S.sigma[4] * Mf * Mf);
     if (S.ppe_n > 0) ph += gwh_setup_ppe(S, f, nullptr);
     if (S.gimr) ph += gwh_setup_gimr(S, f, nullptr);
     return ph;
 }
-__device__ __forceinline__ double gwh_setup_phase_ins(const SetupState &S, double f)
-{
-    const double Mf = S.M * f, u = cbrt(Mf), v = u * 1.4645918875615231, iv = 1.0 / v;
-    return gwh_setup_phase_ins_at(S, f, v, iv, log(GWH_PI * Mf), u, Mf);
-}
 
-/* d/df of the inspiral phase (IMRPhenomD.cpp:1426-1460) at f1p = 0.018 / M */
-__device__ __forceinline__ double gwh_setup_dphase_ins_f1p(const SetupState &S)
+/* d/df of the inspiral phase (IMRPhenomD.cpp:1426-1460) */
+__device__ __forceinline__ double gwh_setup_dphase_ins(const SetupState &S, double f)
 {
-    const double M = S.M, v = GWH_MF1P_V, u = GWH_MF1P_U, lx = GWH_MF1P_LNPI;
+    double M = S.M;
+    double x = GWH_PI * M * f;
+    double lx = log(x);
     double c[8];
     for (int i = 0; i < 8; i++) c[i] = S.pp[i];
     c[5] = S.pp[8] + lx * S.pp[9];
     c[6] = S.pp[10] - S.pp[11] * lx;
-    const double K = 3. / 128. * S.ieta, iv = 1.0 / v, inf = M * (1.0 / GWH_MF1P); /* 1 / f */
-    /* (pi M f)^((i - 8) / 3) as powers of v^-1 */
+    double K = 3. / (128. * S.eta);
+    /* x^((i - 8) / 3) as powers of x^(-1/3) */
+    double v = cbrt(x), iv = 1.0 / v;
     double sum = 0, pw = iv;
 #pragma unroll
     for (int i = 7; i >= 0; i--) {
-        sum += c[i] * (((i - 5.) / 3.) * pw);
+        sum += c[i] * ((i - 5.) / 3.) * pw;
         pw *= iv;
     }
-    double r = K * ((GWH_PI * M) * sum + (S.pp[9] - S.pp[11] * v) * inf) +
-               S.ieta * (M * (S.sigma[1] + S.sigma[2] * u + S.sigma[3] * (u * u) + S.sigma[4] * GWH_MF1P));
+    double d = K * (GWH_PI * M) * sum + K * (S.pp[9] - S.pp[11] * v) / f;
+    /* M^(4/3) f^(1/3) = M (Mf)^(1/3), M^(5/3) f^(2/3) = M (Mf)^(2/3) */
+    double u = cbrt(M * f);
+    double sg = S.sigma[1] * M + S.sigma[2] * M * u + S.sigma[3] * M * u * u + S.sigma[4] * M * M * f;
+    double r = d + sg / S.eta;
     if (S.ppe_n > 0) {
         double dt;
-        gwh_setup_ppe(S, S.f1p, &dt);
+        gwh_setup_ppe(S, f, &dt);
         r += dt;
     }
     if (S.gimr) { /* the order-1 coefficient is already in the polynomial derivative above */
         double dt;
-        gwh_setup_gimr(S, S.f1p, &dt);
+        gwh_setup_gimr(S, f, &dt);
         const double iv4 = iv * iv * iv * iv;
-        r += dt - K * S.pp[1] * (-4. / 3.) * iv4 * inf;
+        r += dt - K * S.pp[1] * (-4. / 3.) * iv4 / f;
         /* The reference differentiates the log terms of c5 and c6 with their GR coefficients whatever gIMR did
          * to them (assign_nonstatic_pn_phase_coeff_deriv, IMRPhenomD.cpp:1068-1084, reached from gIMRPhenomD's
          * Dphase_ins through the GR class, gIMRPhenomD.cpp:167-184): with phi orders 8 and 9 set, the
          * connection slope at f1 is not the inspiral phase's own slope. */
         const double c9gr = gwh_pn_c8_gr(S.eta, S.delta, S.chi_a, S.chi_s), c11gr = 6848. / 63.;
-        r += K * ((c9gr - S.pp[9]) - (c11gr - S.pp[11]) * v) * inf;
+        r += K * ((c9gr - S.pp[9]) - (c11gr - S.pp[11]) * v) / f;
     }
     return r;
 }
@@ -523,35 +538,44 @@ __device__ __forceinline__ double gwh_setup_ppe_imr(const SetupState &S, double 
     return deriv ? d : t;
 }
 
-/* intermediate phase at f and its derivative, given M f, 1 / (M f) and ln(M f) */
-__device__ __forceinline__ double gwh_setup_phase_int_l(const SetupState &S, double f, double Mf, double iMf, double lMf)
+/* intermediate phase at f, given lMf = ln(M f) */
+__device__ __forceinline__ double gwh_setup_phase_int_l(const SetupState &S, double f, double lMf)
 {
-    return S.ieta * (S.beta[0] + S.beta[1] * Mf + S.beta[2] * lMf - S.beta[3] * (iMf * iMf * iMf) * (1. / 3.)) +
+    double Mf = S.M * f;
+    return (1. / S.eta) * (S.beta[0] + S.beta[1] * Mf + S.beta[2] * lMf - S.beta[3] / 3. / (Mf * Mf * Mf)) +
            gwh_setup_ppe_imr(S, f, false);
-}
-__device__ __forceinline__ double gwh_setup_dphase_int(const SetupState &S, double f, double iMf)
-{
-    const double i2 = iMf * iMf;
-    return S.ieta * (S.M * (S.beta[1] + S.beta[2] * iMf + S.beta[3] * (i2 * i2))) + gwh_setup_ppe_imr(S, f, true);
 }
 
-/* merger-ringdown phase at f and its derivative */
-__device__ __forceinline__ double gwh_setup_phase_mr(const SetupState &S, double f)
+__device__ __forceinline__ double gwh_setup_dphase_int(const SetupState &S, double f)
 {
-    const double Mf = S.M * f;
-    return S.ieta * (S.alpha[0] + S.alpha[1] * Mf - S.alpha[2] / Mf + (4. / 3.) * S.alpha[3] * sqrt(sqrt(Mf * Mf * Mf)) +
-                     S.alpha[4] * atan((f - S.alpha[5] * S.fRD) / S.fdamp)) +
-           gwh_setup_ppe_imr(S, f, false);
-}
-__device__ __forceinline__ double gwh_setup_dphase_mr(const SetupState &S, double f)
-{
-    const double M = S.M, Mf = M * f, iMf = 1.0 / Mf;
-    const double w = S.fdamp, t = f - S.alpha[5] * S.fRD;
-    return S.ieta * (S.alpha[4] * w / (w * w + t * t) +
-                     M * (S.alpha[2] * (iMf * iMf) + S.alpha[1] + S.alpha[3] * (sqrt(sqrt(Mf * Mf * Mf)) * iMf))) +
+    double M = S.M;
+    return (1. / S.eta) * (S.beta[1] * M + S.beta[2] / f + S.beta[3] / (M * M * M * f * f * f * f)) +
            gwh_setup_ppe_imr(S, f, true);
 }
 
+__device__ __forceinline__ double gwh_setup_phase_mr(const SetupState &S, double f)
+{
+    double Mf = S.M * f;
+    return (1. / S.eta) * (S.alpha[0] + S.alpha[1] * Mf - S.alpha[2] / Mf + (4. / 3.) * S.alpha[3] * sqrt(sqrt(Mf * Mf * Mf)) +
+                           S.alpha[4] * atan((f - S.alpha[5] * S.fRD) / S.fdamp)) +
+           gwh_setup_ppe_imr(S, f, false);
+}
+
+__device__ __forceinline__ double gwh_setup_dphase_mr(const SetupState &S, double f)
+{
+    double M = S.M;
+    double t = (f - S.alpha[5] * S.fRD) / S.fdamp;
+    return (S.alpha[4] / (S.fdamp * (1. + t * t)) + S.alpha[2] / (f * f * M) + M * (S.alpha[1] + S.alpha[3] / sqrt(sqrt(f * M)))) /
+               S.eta +
+           gwh_setup_ppe_imr(S, f, true);
+}
+
+/* f1 times M, where the amplitude leaves its inspiral form, and what that needs of it */
+#define GWH_MF1 0.014
+#define GWH_MF1_V 0.35298748079802035326 /* (pi M f)^(1/3) */
+#define GWH_MF1_U 0.24101422641752299861 /* (M f)^(1/3) */
+
+#pragma clang fp contract(on)
 /* reduced inspiral amplitude and its frequency derivative (IMRPhenomD.cpp:1335-1420) at f1 = 0.014 / M */
 __device__ __forceinline__ void gwh_setup_amp_ins_f1(const SetupState &S, double *val, double *der)
 {
@@ -619,6 +643,7 @@ __device__ inline void gwh_euler_coeffs(double q, double chil, double chip, doub
     e[1] = a[1];
 }
 
+#pragma clang fp contract(fast)
 /* iv = 1 / v (a bin takes it from its tabulated f^{-1/3}).  The sum as explicit fused multiply-adds, so every kernel
  * that inlines it (the GR and the modified-gravity setup among them) rounds it the same way */
 __device__ __forceinline__ double gwh_euler_eval(const double *c, double v, double iv, double logw)
@@ -641,9 +666,10 @@ __device__ __forceinline__ double gwh_euler_eval(const double *c, double v, doub
  *            role 1  PN coefficients, the inspiral amplitude and its derivative at f1
  *            role 2  IMRPhenomPv2 frame (thetaJN, alpha0, zeta), detector projections, tiles to visit
  *            role 3  chirp mass, amplitude scale, ppE coefficients, powers of M; Pv2 precession constants
- *   phase 2  role 0  inspiral phase and derivative at f1p  role 1  amplitude connection
- *            role 2  merger-ringdown phase and derivative at f2p with alpha0 = alpha1 = 0, ln(M f2p)
- *            role 3  phase piece at f_ref, merger-ringdown derivative at f3 (alpha1 = 0); Pv2 Euler offsets
+ *   phase 2  role 0  inspiral phase at f1p                 role 1  its derivative at f1p
+ *                    and ln(M f1p)                                  and ln(M f2p)
+ *            role 2  merger-ringdown phase and derivative at f2p with alpha0 = alpha1 = 0
+ *            role 3  amplitude connection, phase piece at f_ref, merger-ringdown derivative at f3 (alpha1 = 0); Pv2 Euler offsets
  *            Pv2 with shift_time: the ten knots of the t_c spline (merger-ringdown phase, alpha0 = alpha1 = 0)
  *   phase 3  role 0  the C1 phase connection (beta0, beta1, alpha0, alpha1), phase and time alignment
  *
@@ -660,7 +686,7 @@ struct SetupShared {
     double alpha0, phi_aligned; /* Pv2 frame */
     double p_ins, d_ins;      /* inspiral phase and derivative at f1p */
     double q_mr, dq_mr;       /* merger-ringdown phase and derivative at f2p, alpha0 = alpha1 = 0 */
-    double l2;                /* ln(M f2p) */
+    double l1, l2;            /* ln(M f1p), ln(M f2p) */
     double ref;               /* at f_ref: inspiral phase, merger-ringdown phase (alpha0 = alpha1 = 0) or ln(M f_ref) */
     double dq_mr3;            /* merger-ringdown derivative at f3, alpha1 = 0 */
     double tq[10];            /* Pv2 t_c spline knots: merger-ringdown phase, alpha0 = alpha1 = 0 */
@@ -677,11 +703,11 @@ __device__ __forceinline__ void gwh_setup_base(const gwh_params &p, int ppe, Set
     S.eta = (S.m1 * S.m2) / (S.M * S.M);
     S.chi_s = 0.5 * (S.chi1 + S.chi2);
     S.chi_a = 0.5 * (S.chi1 - S.chi2);
+    S.delta = sqrt(1. - 4. * S.eta);
     S.ieta = 1.0 / S.eta;
     S.iM = 1.0 / S.M;
-    S.delta = sqrt(1. - 4. * S.eta);
-    S.chi_eff = (S.m1 * S.chi1 + S.m2 * S.chi2) * S.iM;
-    S.chi_pn = S.chi_eff - (38. / 113.) * S.eta * (2. * S.chi_s);
+    S.chi_eff = (S.m1 * S.chi1 + S.m2 * S.chi2) / S.M;
+    S.chi_pn = S.chi_eff - (38. * S.eta / 113.) * (2. * S.chi_s);
     /* ppE terms (waveform_generator.cpp:1296-1300 copies them for the ppE methods only) */
     S.ppe_n = 0;
     if (ppe == 1 || ppe == 2) {
@@ -700,8 +726,7 @@ __device__ __forceinline__ double gwh_setup_chip(const gwh_params &p, const Setu
     const double s1x = p.spin1[0], s1y = p.spin1[1], s2x = p.spin2[0], s2y = p.spin2[1];
     const double m1_2 = S.m1 * S.m1, m2_2 = S.m2 * S.m2;
     double S1p = m1_2 * sqrt(s1y * s1y + s1x * s1x), S2p = m2_2 * sqrt(s2y * s2y + s2x * s2x);
-    /* times 2 m1 m2: A1 = 2 + 3 m2 / (2 m1), A2 = 2 + 3 m1 / (2 m2) */
-    double A1 = S.m2 * (4 * S.m1 + 3 * S.m2), A2 = S.m1 * (4 * S.m2 + 3 * S.m1);
+    double A1 = 2 + (3 * S.m2) / (2 * S.m1), A2 = 2 + (3 * S.m1) / (2 * S.m2);
     double num = (A2 * S2p > A1 * S1p) ? A2 * S2p : A1 * S1p;
     double den = (S.m2 > S.m1) ? A2 * m2_2 : A1 * m1_2;
     return num / den;
@@ -738,14 +763,20 @@ __device__ __forceinline__ void gwh_setup_ringdown(const gwh_params &p, bool pv2
     for (int i = 0; i < 3; i++) S.g[i] = gwh_fit(fits, 4 + i, S.eta, xfit);
     double af;
     if (pv2) {
-        const bool first = S.m1 >= S.m2;
-        const double qf = (first ? S.m1 : S.m2) * S.iM;
-        const double afp = gwh_final_spin0815(S.eta, S.ieta, S.delta, first ? S.chi1 : S.chi2, first ? S.chi2 : S.chi1);
+        double Mt = S.m1 + S.m2;
+        double et = S.m1 * S.m2 / (Mt * Mt);
+        double qf, afp;
+        if (S.m1 >= S.m2) {
+            qf = S.m1 / Mt;
+            afp = gwh_final_spin0815(et, S.chi1, S.chi2);
+        } else {
+            qf = S.m2 / Mt;
+            afp = gwh_final_spin0815(et, S.chi2, S.chi1);
+        }
         double Sperp = chip * qf * qf;
-        const double a2 = sqrt(Sperp * Sperp + afp * afp);
-        af = afp == 0 ? __longlong_as_double(0x7ff8000000000000LL) : copysign(a2, afp); /* |afp|^-1 afp a2 */
+        af = sqrt(1.0 / (afp * afp)) * afp * sqrt(Sperp * Sperp + afp * afp);
     } else {
-        af = gwh_final_spin0815(S.eta, S.ieta, S.delta, S.chi1, S.chi2);
+        af = gwh_final_spin0815(S.eta, S.chi1, S.chi2);
     }
     if (p.dep_postmerger) {
         /* IMRPhenomD.cpp:1112-1179 */
@@ -760,19 +791,19 @@ __device__ __forceinline__ void gwh_setup_ringdown(const gwh_params &p, bool pv2
         S.fRD = (1. / GWH_2PI) * MWRD / (S.M * (1. - Er));
         S.fdamp = (1. / GWH_2PI) * MWd / (S.M * (1. - Er));
     } else {
+        double Er = gwh_erad0815(S.eta, S.chi1, S.chi2);
         double fr, fd;
-        gwh_qnm_eval(qnm, af, fr, fd); /* its loads are in flight while the radiated energy is computed */
-        const double s = S.iM / (1.0 - gwh_erad0815(S.eta, S.delta, S.chi1, S.chi2));
-        S.fRD = fr * s;
-        S.fdamp = fd * s;
+        gwh_qnm_eval(qnm, af, fr, fd);
+        S.fRD = fr / (1.0 - Er) / S.M;
+        S.fdamp = fd / (1.0 - Er) / S.M;
     }
-    S.f1p = GWH_MF1P / S.M;
+    S.f1p = 0.018 / S.M;
     S.f2p = S.fRD / 2.;
-    S.f1 = GWH_MF1 / S.M;
+    S.f1 = 0.014 / S.M;
     {
-        const double g2 = S.g[1], g3 = S.g[2];
-        const double v = (g2 > 1) ? -1.0 : sqrt(1 - g2 * g2) - 1;
-        S.f3 = fabs(S.fRD + S.fdamp * g3 * v / g2);
+        double g2 = S.g[1], g3 = S.g[2];
+        double v = (g2 > 1) ? S.fRD + (S.fdamp * (-1.) * g3) / g2 : S.fRD + S.fdamp * g3 * (sqrt(1 - g2 * g2) - 1) / g2;
+        S.f3 = fabs(v);
     }
 }
 
@@ -784,32 +815,33 @@ __device__ __forceinline__ void gwh_setup_pn(const gwh_params &p, SetupState &S)
     double eta2 = eta * eta, eta3 = eta2 * eta, cs2 = cs * cs, ca2 = ca * ca, pi2 = GWH_PI * GWH_PI;
     S.pa[0] = 1.;
     S.pa[1] = 0.;
-    S.pa[2] = -323. / 224 + 451. / 168 * eta;
-    S.pa[3] = 27. / 8 * dm * ca + (27. / 8 - 11. / 6 * eta) * cs;
-    S.pa[4] = -27312085. / 8128512 - 1975055. / 338688 * eta + 105271. / 24192 * eta2 + (-81. / 32 + 8 * eta) * ca2 -
-              81. / 16 * dm * ca * cs + (-81. / 32 + 17. / 8 * eta) * cs2;
-    S.pa[5] = -85 * GWH_PI / 64 + 85 * GWH_PI / 16 * eta + dm * (285197. / 16128 - 1579. / 4032 * eta) * ca +
-              (285197. / 16128 - 15317. / 672 * eta - 2227. / 1008 * eta2) * cs;
-    S.pa[6] = -177520268561. / 8583708672 + (545384828789. / 5007163392 - 205 * pi2 / 48) * eta -
-              3248849057. / 178827264 * eta2 + 34473079. / 6386688 * eta3 +
-              (1614569. / 64512 - 1873643. / 16128 * eta + 2167. / 42 * eta2) * ca2 +
-              (31 * GWH_PI / 12 - 7 * GWH_PI / 3 * eta) * cs +
-              (1614569. / 64512 - 61391. / 1344 * eta + 57451. / 4032 * eta2) * cs2 +
-              dm * ca * (31 * GWH_PI / 12 + (1614569. / 32256 - 165961. / 2688 * eta) * cs);
+    S.pa[2] = (-323. / 224 + 451 * eta / 168);
+    S.pa[3] = (27. * dm * ca / 8 + (27. / 8 - 11. * eta / 6) * cs);
+    S.pa[4] = (-27312085. / 8128512 - 1975055 * eta / 338688 + 105271 * eta2 / 24192 + (-81. / 32 + 8 * eta) * ca2 -
+               81 * dm * ca * cs / 16 + (-81. / 32 + 17 * eta / 8) * cs2);
+    S.pa[5] = (-85 * GWH_PI / 64 + 85 * GWH_PI * eta / 16 + dm * (285197. / 16128 - 1579 * eta / 4032) * ca +
+               (285197. / 16128 - 15317 * eta / 672 - 2227 * eta2 / 1008) * cs);
+    S.pa[6] = (-177520268561. / 8583708672 + (545384828789. / 5007163392 - 205 * pi2 / 48) * eta -
+               3248849057 * eta2 / 178827264 + 34473079 * eta3 / 6386688 +
+               (1614569. / 64512 - 1873643. * eta / 16128 + 2167 * eta2 / 42) * ca2 +
+               (31 * GWH_PI / 12 - 7 * GWH_PI * eta / 3) * cs +
+               (1614569. / 64512 - 61391 * eta / 1344 + 57451 * eta2 / 4032) * cs2 +
+               dm * ca * (31 * GWH_PI / 12 + (1614569. / 32256 - 165961 * eta / 2688) * cs));
     for (int i = 0; i < 12; i++) S.pp[i] = 0;
     S.pp[0] = 1.;
-    S.pp[2] = 3715. / 756 + 55. / 9 * eta;
-    S.pp[3] = -16. * GWH_PI + 113. / 3 * dm * ca + (113. / 3 - 76. / 3 * eta) * cs;
-    S.pp[4] = 15293365. / 508032 + 27145. / 504 * eta + 3085. / 72 * eta2 + (-405. / 8 + 200. * eta) * ca2 -
-              (405. / 4) * dm * ca * cs + (-405. / 8 + 5. / 2 * eta) * cs2;
-    S.pp[7] = 77096675. * GWH_PI / 254016 + 378515. * GWH_PI / 1512 * eta - 74045. * GWH_PI / 756 * eta2 +
-              dm * (-25150083775. / 3048192 + 26804935. / 6048 * eta - 1985. / 48 * eta2) * ca +
-              (-25150083775. / 3048192 + 10566655595. / 762048 * eta - 1042165. / 3024 * eta2 + 5345. / 36 * eta3) * cs;
+    S.pp[2] = 3715. / 756 + 55. * eta / 9;
+    S.pp[3] = -16. * GWH_PI + 113. * dm * ca / 3 + (113. / 3 - 76. * eta / 3) * cs;
+    S.pp[4] = 15293365. / 508032 + 27145. * eta / 504 + 3085. * eta2 / 72 + (-405. / 8 + 200. * eta) * ca2 -
+              (405. / 4) * dm * ca * cs + (-405. / 8 + 5. * eta / 2) * cs2;
+    S.pp[7] = 77096675. * GWH_PI / 254016 + 378515. * GWH_PI * eta / 1512 - 74045. * GWH_PI * eta2 / 756 +
+              dm * (-25150083775. / 3048192 + 26804935. * eta / 6048 - 1985. * eta2 / 48) * ca +
+              (-25150083775. / 3048192 + 10566655595. * eta / 762048 - 1042165. * eta2 / 3024 + 5345. * eta3 / 36) * cs;
     S.pp[8] = gwh_pn_c8_gr(eta, dm, ca, cs);
     S.pp[9] = S.pp[8];
-    S.pp[10] = 11583231236531. / 4694215680 - 6848. * GWH_GAMMA_E / 21 - 640. * pi2 / 3 - 6848. * (GWH_LOG_64) / 63 +
-               (-15737765635. / 3048192 + 2255. * pi2 / 12) * eta + 76055. / 1728 * eta2 - 127825. / 1296 * eta3 +
-               2270. * GWH_PI / 3 * dm * ca + (2270. * GWH_PI / 3 - 520. * GWH_PI * eta) * cs;
+    S.pp[10] = 11583231236531. / 4694215680 - 6848. * GWH_GAMMA_E / 21 - 640. * pi2 / 3 +
+               (-15737765635. / 3048192 + 2255. * pi2 / 12) * eta + 76055. * eta2 / 1728 - 127825. * eta3 / 1296 +
+               2270. * dm * ca * GWH_PI / 3 + (2270. * GWH_PI / 3 - 520. * GWH_PI * eta) * cs -
+               6848. * (GWH_LOG_64) / 63;
     S.pp[11] = 6848. / 63.;
     if (S.gimr) {
         const int direct[5] = {0, 2, 3, 4, 7};
@@ -850,6 +882,7 @@ __device__ __forceinline__ void gwh_setup_mass(const gwh_params &p, int ppe, Set
     }
 }
 
+#pragma clang fp contract(on)
 /* role 2, phase 1: the Pv2 frame (IMRPhenomP.cpp:821-938, :1081-1211): cosine and sine of thetaJN and of 2 zeta, alpha0
  * and the aligned-spin phase offset -phiJ.  The reference turns every direction into an angle and back; here a rotation
  * takes its cosine and sine from the direction's components, and only the two angles that enter a phase are formed. */
@@ -1042,13 +1075,13 @@ __device__ __forceinline__ double gwh_setup_tcorr(double fRD, const double *q)
     return s / df;
 }
 
+#pragma clang fp contract(fast)
 /* the t_c spline's knot j: 0.8 fRD + j (0.4 fRD / 9) */
 __device__ __forceinline__ double gwh_setup_knot(double fRD, int j)
 {
     double start = .8 * fRD, stop = 1.2 * fRD;
-    return start + j * ((stop - start) * (1. / 9));
+    return start + j * ((stop - start) / 9);
 }
-#pragma clang fp contract(fast)
 
 /* ------------------------------------------------------------------------- */
 /* per-bin FP64 evaluation                                                    */
