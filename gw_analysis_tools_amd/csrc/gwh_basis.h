@@ -116,6 +116,17 @@ GWH_HD static void unpack(const gwh_params &p, int basis, double *v, int *lf)
 /* parts of a basis vector's record that do not depend on each other (a kernel gives each its own wave) */
 #define GWH_REPACK_PARTS 3
 
+/* the spins of the bases that hold them as they are */
+GWH_HD static void repack_spins(const double *v, int basis, gwh_params &a)
+{
+    a.spin1[2] = v[9];
+    a.spin2[2] = v[10];
+    if (basis == GWH_BASIS_PV2_FULL) {
+        a.chip = v[11];
+        a.phip = v[12];
+    }
+}
+
 /* a: a gen_params carrying only the non-parameter options (fisher.cpp:2513-2572).  Part 0: sky position, orientation,
  * phase, time; 1: distance and (cosine of) inclination, IMRPhenomPv2's first spin; 2: masses and spins */
 GWH_HD static void repack_part(const double *v, int basis, int part, gwh_params &a)
@@ -159,17 +170,23 @@ GWH_HD static void repack_part(const double *v, int basis, int part, gwh_params 
             sph_to_cart(s2, a.spin2);
         }
     } else if (part == 2) {
-        a.spin1[2] = v[9];
-        a.spin2[2] = v[10];
-        if (basis == GWH_BASIS_PV2_FULL) {
-            a.chip = v[11];
-            a.phip = v[12];
-        }
+        repack_spins(v, basis, a);
     }
 }
 GWH_HD static void repack(const double *v, int basis, gwh_params &a)
 {
     for (int part = 0; part < GWH_REPACK_PARTS; part++) repack_part(v, basis, part, a);
+}
+
+/* the fields of a repacked vector that depend on its element i */
+GWH_HD static void repack_element(const double *v, int basis, int i, gwh_params &a)
+{
+    if (basis == GWH_BASIS_PHENOMD_SKYAVG)
+        repack_part(v, basis, 2, a);
+    else if (basis != GWH_BASIS_PV2_MCMC && i >= 9)
+        repack_spins(v, basis, a);
+    else
+        repack_part(v, basis, (i == 3 || i == 6 || i == 9 || i == 11 || i == 13) ? 1 : (i >= 7 ? 2 : 0), a);
 }
 
 #endif

@@ -231,6 +231,32 @@ struct DevBuf {
     template <class T> T *as() { return (T *)p; }
 };
 
+/* n 8-byte words that the setup's launch also copies to the device, from host memory that it reads directly, for the
+ * kernels behind it */
+struct StageCopy {
+    const double *src = nullptr;
+    double *dst = nullptr;
+    int n = 0;
+};
+/* pinned host memory and its device address */
+int gwh_pinned_alloc(void **host, void **dev, size_t bytes);
+
+/* Pinned host memory that kernels read and write directly (coherent, at g on the device), grown as needed up to
+ * GWH_STAGE_MAX: what exceeds that goes through the runtime's own staging. */
+#define GWH_STAGE_MAX (4u << 20)
+struct HostStage {
+    char *h = nullptr, *g = nullptr;
+    size_t cap = 0;
+    int ensure(size_t bytes); /* only with no work in flight that uses it */
+};
+
+/* Bytes of a parameter record that a model's setup reads: the GR models none of the modified-gravity terms, which are
+ * the last two thirds of it.  Records of a batch may lie that far apart. */
+inline int gwh_record_bytes(int model)
+{
+    return gwh_ppe_variant(model) ? (int)sizeof(gwh_params) : (int)offsetof(gwh_params, ppe_nmod);
+}
+
 /* Device scratch of one batched-likelihood launch sequence (setup, tiles, finalize).  The engine owns one;
  * the serving broker owns one per stream so batches can be in flight together. */
 struct Scratch {
@@ -243,6 +269,9 @@ struct Scratch {
  *   d_mask        device ints, n: only instances with d_mask[i] != 0 are evaluated
  *   reserve_only  size the scratch buffers for this launch and return without launching
  *   capturing     the stream is being captured into a graph: no timing events are recorded
+ *   record_bytes  distance of the parameter records
+ *   setup_events  instance events as the setup reads them (d_events: as the kernels after it do)
+ *   copy          words copied by the setup's launch
  *   finalize_later  the last kernel (partial sums -> log-likelihoods) is left to the caller, with these arguments
  * Instances that are not evaluated get a NaN result. */
 struct LaunchExtra {
@@ -250,28 +279,32 @@ struct LaunchExtra {
     const int *d_mask = nullptr;
     bool reserve_only = false;
     bool capturing = false;
+    int record_bytes = sizeof(gwh_params);
+    const int *setup_events = nullptr;
+    StageCopy copy;
     FinalizeArgs *finalize_later = nullptr;
 };
 
 /* Device scratch and stream of one Fisher computation (the engine's own, or a broker worker's). */
 struct FisherScratch {
     hipStream_t stream = nullptr;
-    DevBuf params, coef, misc, deriv, gram, out, sig, raw;
+    DevBuf coef, misc, deriv, gram, out, sig, raw;
     size_t max_operand = (size_t)1 << 30; /* operand rows of one pass: points per pass follow from it */
-    /* pinned host staging of a pass's stencil records, weights and flags; two alternate, so the host builds the
-     * next pass while the device runs the current one (stage_done: the copy out of each has run) */
-    void *stage[2] = {nullptr, nullptr};
+    /* pinned host staging of a pass's stencil records, weights and flags, and of its matrices on the way back; two
+     * alternate, so the host builds the next pass while the device runs the current one (stage_done: the pass whose
+     * data each holds has ended) */
+    void *stage[2] = {nullptr, nullptr}, *stage_dev[2] = {nullptr, nullptr}; /* on the host, on the device */
     size_t stage_cap[2] = {0, 0};
     hipEvent_t stage_done[2] = {nullptr, nullptr};
     size_t bytes() const /* device bytes */
     {
-        return params.cap + coef.cap + misc.cap + deriv.cap + gram.cap + out.cap + sig.cap + raw.cap;
+        return coef.cap + misc.cap + deriv.cap + gram.cap + out.cap + sig.cap + raw.cap;
     }
     /* give back the device buffers (the stream's work finished first); all_host: the host staging too */
     void release(bool all_host = false)
     {
         if (stream) (void)hipStreamSynchronize(stream);
-        for (DevBuf *d : {&params, &coef, &misc, &deriv, &gram, &out, &sig, &raw}) d->release();
+        for (DevBuf *d : {&coef, &misc, &deriv, &gram, &out, &sig, &raw}) d->release();
         if (!all_host) return;
         for (int i = 0; i < 2; i++) {
             if (stage[i]) (void)hipHostFree(stage[i]);
@@ -304,6 +337,7 @@ struct Engine {
     DevBuf work, wcount; /* flattened (instance, tile) lists of multi-event batches */
     FisherScratch fisher; /* stream = the engine stream */
     DevBuf fft, fftwork, mxpart, mxres, mxin; /* FFT-maximised likelihoods */
+    HostStage stage; /* inputs and results of the call that holds the lock; its work has ended when that returns */
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     /* live timing of the per-bin kernel inside a caller's timed region: event pairs around each launch */
     std::vector<hipEvent_t> kt_ev;
@@ -358,7 +392,7 @@ size_t gwh_fisher_batch_bytes(int event, int model, int basis, int precision, co
 
 /* per-instance setup on device buffers */
 int gwh_setup_launch(const int *d_events, int events0, int model, const gwh_params *d_params, int n, InstCoef *d_coef,
-                     hipStream_t stream);
+                     hipStream_t stream, int record_bytes = sizeof(gwh_params), StageCopy copy = StageCopy());
 
 uint64_t gwh_hash_bytes(const void *p, size_t n, uint64_t seed);
 

@@ -69,6 +69,36 @@ Engine &gwh_engine()
     return *e;
 }
 
+int gwh_pinned_alloc(void **host, void **dev, size_t bytes)
+{
+    if (hipHostMalloc(host, bytes, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+        *host = nullptr;
+        return gwh_set_error(GWH_ERR_NOMEM, "pinned staging allocation failed");
+    }
+    if (hipHostGetDevicePointer(dev, *host, 0) != hipSuccess)
+        return gwh_set_error(GWH_ERR_HIP, "no device address for pinned staging");
+    return GWH_OK;
+}
+
+int HostStage::ensure(size_t bytes)
+{
+    if (bytes <= cap) return GWH_OK;
+    if (h) (void)hipHostFree(h);
+    h = g = nullptr;
+    cap = 0;
+    const size_t c = std::min<size_t>(std::max<size_t>(bytes + bytes / 4, 1u << 16), GWH_STAGE_MAX);
+    void *dev = nullptr, *host = nullptr;
+    const int rc = gwh_pinned_alloc(&host, &dev, c);
+    if (rc != GWH_OK) {
+        if (host) (void)hipHostFree(host);
+        return rc;
+    }
+    h = (char *)host;
+    g = (char *)dev;
+    cap = c;
+    return GWH_OK;
+}
+
 int DevBuf::ensure(size_t bytes)
 {
     if (bytes <= cap) return GWH_OK;
@@ -423,19 +453,49 @@ int gwh_event_create_ex(const double *f, int N, int ndet, const int *dets, const
  * 119 of 8 bytes 952 bytes apart per lane, go through twice as many CUs (512 instances 11.3 -> 10.0 us; with a quarter of
  * the lanes the fetch of the code by ever more CUs costs more than that saves: 11.0, an eighth 15.4).  MOD: the ppE / gIMR /
  * theory modifications are compiled in (the GR models run a kernel without them, which keeps its registers and
- * code to what GR needs). */
+ * code to what GR needs).
+ *
+ * The records come in through LDS, each byte once, in order and all in flight together: they may lie in host memory (one
+ * load after another there: 6 us more for the 448 bytes that MOD reads of a record), where a copy to the device would
+ * stand between the launches (384 IMRPhenomPv2 Fisher points in five passes 1241 -> 1065 us). */
 #define GWH_SETUP_LANES 32
+#define GWH_SETUP_COPY 1024 /* words of StageCopy per block */
 template <int MODEL, bool MOD>
-__global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__restrict__ params,
+__global__ __launch_bounds__(256) void gwh_setup_kernel(const char *__restrict__ params, int record_bytes,
                                                         const int *__restrict__ inst_event, int event0, int n,
                                                         QnmTable qnm,
                                                         const DetGeom *__restrict__ geo,
                                                         const EventDesc *__restrict__ events,
                                                         InstCoef *__restrict__ coef, int *__restrict__ active,
                                                         const int *__restrict__ d_count, const int *__restrict__ d_mask,
-                                                        int ppe_variant)
+                                                        int ppe_variant, StageCopy copy)
 {
     const int ppe = MOD ? ppe_variant : 0;
+    constexpr int words = (int)(MOD ? sizeof(gwh_params) : offsetof(gwh_params, ppe_nmod)) / 8;
+    typedef double __attribute__((may_alias)) word;
+    __shared__ __align__(8) char records[GWH_SETUP_LANES * words * 8];
+    const int blocks = (n + GWH_SETUP_LANES - 1) / GWH_SETUP_LANES;
+    if ((int)blockIdx.x >= blocks) { /* the blocks behind the instances */
+        const int k0 = ((int)blockIdx.x - blocks) * GWH_SETUP_COPY;
+        for (int k = k0 + threadIdx.x; k < k0 + GWH_SETUP_COPY && k < copy.n; k += 256) copy.dst[k] = copy.src[k];
+        return;
+    }
+    {
+        constexpr int rounds = (GWH_SETUP_LANES * words + 255) / 256;
+        word w[rounds]; /* all loads in flight together */
+#pragma unroll
+        for (int q = 0; q < rounds; q++) {
+            const int k = q * 256 + threadIdx.x, r = blockIdx.x * GWH_SETUP_LANES + k / words;
+            if (k < GWH_SETUP_LANES * words && r < n)
+                w[q] = *(const word *)(params + (size_t)r * record_bytes + (k % words) * 8);
+        }
+#pragma unroll
+        for (int q = 0; q < rounds; q++) {
+            const int k = q * 256 + threadIdx.x;
+            if (k < GWH_SETUP_LANES * words) *(word *)(records + k * 8) = w[q];
+        }
+    }
+    __syncthreads();
     __shared__ SetupShared sh[GWH_SETUP_LANES];
     constexpr bool pv2 = (MODEL == GWH_IMRPHENOMPV2);
     const int lane = threadIdx.x & 63;
@@ -448,7 +508,7 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__rest
     }
     SetupShared &X = sh[lane & (GWH_SETUP_LANES - 1)];
     InstCoef *C = coef + (live ? i : 0);
-    gwh_params p;
+    const gwh_params &p = *(const gwh_params *)(records + (lane & (GWH_SETUP_LANES - 1)) * (words * 8));
     SetupState S;
     int ev = event0;
     double eul_a = 0, eul_e = 0; /* Pv2: Euler angles at f_ref (role 3) */
@@ -456,7 +516,6 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__rest
     /* ---- phase 1 ---- */
     if (live) {
         if (inst_event) ev = inst_event[i];
-        p = params[i];
         gwh_setup_base(p, ppe, S);
         if (role == 0) {
             const double chip = pv2 ? gwh_setup_chip(p, S) : -1;
@@ -736,22 +795,23 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const gwh_params *__rest
 
 static void launch_setup(int model, int n, hipStream_t st, const gwh_params *params, const int *inst_event,
                          int event0, InstCoef *coef, int *active, const int *d_count = nullptr,
-                         const int *d_mask = nullptr)
+                         const int *d_mask = nullptr, int record_bytes = sizeof(gwh_params),
+                         const EventDesc *d_events = nullptr, StageCopy copy = StageCopy())
 {
     Engine &E = gwh_engine();
-    dim3 g((n + GWH_SETUP_LANES - 1) / GWH_SETUP_LANES), b(256);
+    dim3 g((n + GWH_SETUP_LANES - 1) / GWH_SETUP_LANES + (copy.n + GWH_SETUP_COPY - 1) / GWH_SETUP_COPY), b(256);
     const int var = gwh_ppe_variant(model);
     auto k = gwh_is_pv2(model) ? (var ? gwh_setup_kernel<GWH_IMRPHENOMPV2, true> : gwh_setup_kernel<GWH_IMRPHENOMPV2, false>)
                                : (var ? gwh_setup_kernel<GWH_IMRPHENOMD, true> : gwh_setup_kernel<GWH_IMRPHENOMD, false>);
-    hipLaunchKernelGGL(k, g, b, 0, st, params, inst_event, event0, n, E.qnm, (const DetGeom *)E.d_geo,
-                       (const EventDesc *)E.d_events, coef, active, d_count, d_mask, var);
+    hipLaunchKernelGGL(k, g, b, 0, st, (const char *)params, record_bytes, inst_event, event0, n, E.qnm,
+                       (const DetGeom *)E.d_geo, d_events ? d_events : (const EventDesc *)E.d_events, coef, active, d_count, d_mask, var, copy);
 }
 
 int gwh_setup_launch(const int *d_events, int events0, int model, const gwh_params *d_params, int n, InstCoef *d_coef,
-                     hipStream_t stream)
+                     hipStream_t stream, int record_bytes, StageCopy copy)
 {
-    Engine &E = gwh_engine();
-    launch_setup(model, n, stream, d_params, d_events, events0, d_coef, nullptr);
+    launch_setup(model, n, stream, d_params, d_events, events0, d_coef, nullptr, nullptr, nullptr, record_bytes, nullptr,
+                 copy);
     GWH_HIP(hipGetLastError());
     return GWH_OK;
 }
@@ -956,8 +1016,8 @@ int gwh_loglike_launch(const int *d_events, int events0, int model, int precisio
     W.event0 = events0;
     W.n = n;
     W.tiles0 = maxtiles;
-    launch_setup(model, n, stream, d_params, d_events, events0, s_coef.as<InstCoef>(), s_active.as<int>(), X.d_count,
-                 X.d_mask);
+    launch_setup(model, n, stream, d_params, X.setup_events ? X.setup_events : d_events, events0, s_coef.as<InstCoef>(),
+                 s_active.as<int>(), X.d_count, X.d_mask, X.record_bytes, nullptr, X.copy);
     GWH_HIP(hipGetLastError());
     if (X.capturing) timed = false;
     if (timed) GWH_HIP(hipEventRecord(E.ev0, stream));
@@ -1369,35 +1429,67 @@ int gwh_loglike_batch_device_noalloc(const int *d_events, int events0, int model
                               nullptr, nullptr, 0, &S, nullptr);
 }
 
-int gwh_loglike_batch(const int *events, int events0, int model, int precision, const gwh_params *params, int n,
-                      double *logl)
+/* Log-likelihoods (what 0) or SNRs (1) of host records.  The kernels read records and event ids from pinned memory, of
+ * each record only the bytes that the model has a use for, and write the results to it: pageable copies cost a staging
+ * pass and a wait each (1024 IMRPhenomPv2 instances 118 -> 94 us, 384 IMRPhenomD instances of 48 events 240 -> 220 us).
+ * Batches beyond GWH_STAGE_MAX go through pageable copies. */
+static int batch_from_host(const int *events, int events0, int model, int precision, const gwh_params *params, int n,
+                           double *out, int what)
 {
     Engine &E = gwh_engine();
     std::lock_guard<std::recursive_mutex> lk(E.mu);
-    int st = gwh_ensure_init();
-    if (st != GWH_OK) return st;
+    int rc = gwh_ensure_init();
+    if (rc != GWH_OK) return rc;
     if (n <= 0) return GWH_OK;
-    if (!params || !logl) return gwh_set_error(GWH_ERR_INVALID, "null argument");
-    int rc;
-    if ((rc = E.params.ensure((size_t)n * sizeof(gwh_params))) != GWH_OK) return rc;
-    if ((rc = E.logl.ensure((size_t)n * sizeof(double))) != GWH_OK) return rc;
-    GWH_HIP(hipMemcpyAsync(E.params.p, params, (size_t)n * sizeof(gwh_params), hipMemcpyHostToDevice, E.stream));
-    const int *dev = nullptr;
-    if (events) {
+    if (!params || !out) return gwh_set_error(GWH_ERR_INVALID, "null argument");
+    if (events)
         for (int i = 0; i < n; i++)
             if (events[i] < 0 || events[i] >= GWH_MAX_EVENTS || !E.events[events[i]].live)
                 return gwh_set_error(GWH_ERR_INVALID, "unknown event in batch");
-        if ((rc = E.inst_event.ensure((size_t)n * sizeof(int))) != GWH_OK) return rc;
-        GWH_HIP(hipMemcpyAsync(E.inst_event.p, events, (size_t)n * sizeof(int), hipMemcpyHostToDevice, E.stream));
-        dev = E.inst_event.as<const int>();
-        events0 = events[0];
+    LaunchExtra X;
+    X.record_bytes = gwh_model_valid(model) ? gwh_record_bytes(model) : (int)sizeof(gwh_params);
+    const size_t ids = events ? ((size_t)n * sizeof(int) + 7) / 8 * 8 : 0, res = (size_t)n * sizeof(double);
+    size_t rec = (size_t)n * X.record_bytes;
+    const bool staged = rec + ids + res <= GWH_STAGE_MAX;
+    if (events && (rc = E.inst_event.ensure(ids)) != GWH_OK) return rc;
+    const gwh_params *d_params;
+    double *d_out;
+    if (staged) {
+        if ((rc = E.stage.ensure(rec + ids + res)) != GWH_OK) return rc;
+        for (int i = 0; i < n; i++) memcpy(E.stage.h + (size_t)i * X.record_bytes, params + i, X.record_bytes);
+        if (events) {
+            memcpy(E.stage.h + rec, events, (size_t)n * sizeof(int));
+            X.setup_events = (const int *)(E.stage.g + rec);
+            X.copy = {(const double *)(E.stage.g + rec), E.inst_event.as<double>(), (int)(ids / 8)};
+        }
+        d_params = (const gwh_params *)E.stage.g;
+        d_out = (double *)(E.stage.g + rec + ids);
+    } else {
+        X.record_bytes = sizeof(gwh_params);
+        if ((rc = E.params.ensure((size_t)n * sizeof(gwh_params))) != GWH_OK) return rc;
+        if ((rc = E.logl.ensure(res)) != GWH_OK) return rc;
+        GWH_HIP(hipMemcpyAsync(E.params.p, params, (size_t)n * sizeof(gwh_params), hipMemcpyHostToDevice, E.stream));
+        if (events)
+            GWH_HIP(hipMemcpyAsync(E.inst_event.p, events, (size_t)n * sizeof(int), hipMemcpyHostToDevice, E.stream));
+        d_params = E.params.as<const gwh_params>();
+        d_out = E.logl.as<double>();
     }
-    rc = gwh_loglike_launch(dev, events0, model, precision, E.params.as<const gwh_params>(), n, E.logl.as<double>(),
-                            E.stream, false, nullptr, events);
-    if (rc != GWH_OK) return rc;
-    GWH_HIP(hipMemcpyAsync(logl, E.logl.p, (size_t)n * sizeof(double), hipMemcpyDeviceToHost, E.stream));
+    rc = gwh_loglike_launch(events ? E.inst_event.as<const int>() : nullptr, events ? events[0] : events0, model,
+                            precision, d_params, n, d_out, E.stream, false, nullptr, events, what, nullptr, &X);
+    if (rc != GWH_OK) {
+        (void)hipStreamSynchronize(E.stream); /* nothing in flight when the staging is used next */
+        return rc;
+    }
+    if (!staged) GWH_HIP(hipMemcpyAsync(out, d_out, res, hipMemcpyDeviceToHost, E.stream));
     GWH_HIP(hipStreamSynchronize(E.stream));
+    if (staged) memcpy(out, E.stage.h + rec + ids, res);
     return GWH_OK;
+}
+
+int gwh_loglike_batch(const int *events, int events0, int model, int precision, const gwh_params *params, int n,
+                      double *logl)
+{
+    return batch_from_host(events, events0, model, precision, params, n, logl, 0);
 }
 
 int gwh_time_loglike_batch_device(int events0, int model, int precision, const void *d_params, int n, double *d_logl,
@@ -1631,19 +1723,21 @@ int gwh_device_copy(void *dst, const void *src, size_t bytes)
 
 /* ---- single-call drop-in entry points ---- */
 
-static int upload_single(const double *f, int n, const gwh_params *p, int model, int det, const int *dets = nullptr,
-                         int ndet = 1)
+/* A call on one parameter set's waveform: where its kernels read the frequencies and write up to two arrays of n complex
+ * numbers each.  Up to GWH_STAGE_MAX bytes they do so in pinned host memory and nothing is copied by the runtime, whose
+ * pageable copies (three in, two out) cost more than the kernels (8129 bins, both polarisations: 72 -> 47 us). */
+struct SingleIO {
+    const double *f;
+    double2 *out1, *out2;
+    char *host; /* staged: out1 and then out2 on the host */
+};
+
+static int upload_single(const double *f, int n, const gwh_params *p, int model, int det, int nout, SingleIO &io,
+                         const int *dets = nullptr, int ndet = 1)
 {
     Engine &E = gwh_engine();
     int rc;
-    if ((rc = E.f.ensure((size_t)n * 8)) != GWH_OK) return rc;
-    if ((rc = E.params.ensure(sizeof(gwh_params))) != GWH_OK) return rc;
     if ((rc = E.coef.ensure(sizeof(InstCoef))) != GWH_OK) return rc;
-    if ((rc = E.out1.ensure((size_t)n * 16)) != GWH_OK) return rc;
-    if ((rc = E.out2.ensure((size_t)n * 16)) != GWH_OK) return rc;
-    if ((rc = E.misc.ensure(256)) != GWH_OK) return rc;
-    GWH_HIP(hipMemcpyAsync(E.f.p, f, (size_t)n * 8, hipMemcpyHostToDevice, E.stream));
-    GWH_HIP(hipMemcpyAsync(E.params.p, p, sizeof(gwh_params), hipMemcpyHostToDevice, E.stream));
     /* a one-detector descriptor for the setup (only the detector ids are read) */
     EventDesc ds;
     memset(&ds, 0, sizeof(ds));
@@ -1652,10 +1746,63 @@ static int upload_single(const double *f, int n, const gwh_params *p, int model,
     ds.bpl = 1;
     ds.lanes = GWH_TPB;
     for (int d = 0; d < GWH_MAXDET; d++) ds.det[d] = (dets && d < ndet) ? dets[d] : det;
+    const size_t arr = (size_t)n * 16, rec = (sizeof(gwh_params) + 15) / 16 * 16, desc = (sizeof(ds) + 15) / 16 * 16;
+    const size_t all = rec + desc + nout * arr + (size_t)n * 8;
+    if (all <= GWH_STAGE_MAX) {
+        if ((rc = E.stage.ensure(all)) != GWH_OK) return rc;
+        char *h = E.stage.h, *g = E.stage.g;
+        memcpy(h, p, sizeof(gwh_params));
+        memcpy(h + rec, &ds, sizeof(ds));
+        memcpy(h + rec + desc + nout * arr, f, (size_t)n * 8);
+        io.host = h + rec + desc;
+        io.out1 = (double2 *)(g + rec + desc);
+        io.out2 = io.out1 + (nout > 1 ? n : 0);
+        io.f = (const double *)(g + rec + desc + nout * arr);
+        launch_setup(model, 1, E.stream, (const gwh_params *)g, nullptr, 0, E.coef.as<InstCoef>(), nullptr, nullptr,
+                     nullptr, sizeof(gwh_params), (const EventDesc *)(g + rec));
+        GWH_HIP(hipGetLastError());
+        return GWH_OK;
+    }
+    if ((rc = E.f.ensure((size_t)n * 8)) != GWH_OK) return rc;
+    if ((rc = E.params.ensure(sizeof(gwh_params))) != GWH_OK) return rc;
+    if ((rc = E.out1.ensure(arr)) != GWH_OK) return rc;
+    if (nout > 1 && (rc = E.out2.ensure(arr)) != GWH_OK) return rc;
+    GWH_HIP(hipMemcpyAsync(E.f.p, f, (size_t)n * 8, hipMemcpyHostToDevice, E.stream));
+    GWH_HIP(hipMemcpyAsync(E.params.p, p, sizeof(gwh_params), hipMemcpyHostToDevice, E.stream));
     GWH_HIP(hipMemcpyAsync(E.d_events + (GWH_MAX_EVENTS - 1), &ds, sizeof(ds), hipMemcpyHostToDevice, E.stream));
     launch_setup(model, 1, E.stream, E.params.as<const gwh_params>(), nullptr, GWH_MAX_EVENTS - 1,
                  E.coef.as<InstCoef>(), nullptr);
     GWH_HIP(hipGetLastError());
+    io.f = E.f.as<const double>();
+    io.out1 = E.out1.as<double2>();
+    io.out2 = nout > 1 ? E.out2.as<double2>() : io.out1;
+    io.host = nullptr;
+    return GWH_OK;
+}
+
+/* what: 0 the polarisations, 1 and 2 a detector's response (gwh_waveform_kernel) */
+static void launch_waveform(int model, int n, const SingleIO &io, int what, int d = 0)
+{
+    Engine &E = gwh_engine();
+    auto k = gwh_is_pv2(model) ? gwh_waveform_kernel<GWH_IMRPHENOMPV2> : gwh_waveform_kernel<GWH_IMRPHENOMD>;
+    hipLaunchKernelGGL(k, dim3((n + 255) / 256), dim3(256), 0, E.stream, io.f, n, E.coef.as<const InstCoef>(), what,
+                       io.out1, io.out2, d);
+}
+
+/* the arrays to the caller, with the call's last wait */
+static int download_single(const SingleIO &io, int n, double *a, double *b)
+{
+    Engine &E = gwh_engine();
+    const size_t arr = (size_t)n * 16;
+    if (!io.host) {
+        GWH_HIP(hipMemcpyAsync(a, io.out1, arr, hipMemcpyDeviceToHost, E.stream));
+        if (b) GWH_HIP(hipMemcpyAsync(b, io.out2, arr, hipMemcpyDeviceToHost, E.stream));
+    }
+    GWH_HIP(hipStreamSynchronize(E.stream));
+    if (io.host) {
+        memcpy(a, io.host, arr);
+        if (b) memcpy(b, io.host + arr, arr);
+    }
     return GWH_OK;
 }
 
@@ -1677,19 +1824,11 @@ int gwh_fourier_waveform(const double *frequencies, int length, double *hplus, d
     if (rc != GWH_OK) return rc;
     if ((rc = check_common(frequencies, length, params, model)) != GWH_OK) return rc;
     if (!hplus || !hcross) return gwh_set_error(GWH_ERR_INVALID, "null output");
-    if ((rc = upload_single(frequencies, length, params, model, 0)) != GWH_OK) return rc;
-    dim3 g((length + 255) / 256);
-    if (!gwh_is_pv2(model))
-        hipLaunchKernelGGL(gwh_waveform_kernel<GWH_IMRPHENOMD>, g, dim3(256), 0, E.stream, E.f.as<const double>(),
-                           length, E.coef.as<const InstCoef>(), 0, E.out1.as<double2>(), E.out2.as<double2>());
-    else
-        hipLaunchKernelGGL(gwh_waveform_kernel<GWH_IMRPHENOMPV2>, g, dim3(256), 0, E.stream, E.f.as<const double>(),
-                           length, E.coef.as<const InstCoef>(), 0, E.out1.as<double2>(), E.out2.as<double2>());
+    SingleIO io;
+    if ((rc = upload_single(frequencies, length, params, model, 0, 2, io)) != GWH_OK) return rc;
+    launch_waveform(model, length, io, 0);
     GWH_HIP(hipGetLastError());
-    GWH_HIP(hipMemcpyAsync(hplus, E.out1.p, (size_t)length * 16, hipMemcpyDeviceToHost, E.stream));
-    GWH_HIP(hipMemcpyAsync(hcross, E.out2.p, (size_t)length * 16, hipMemcpyDeviceToHost, E.stream));
-    GWH_HIP(hipStreamSynchronize(E.stream));
-    return GWH_OK;
+    return download_single(io, length, hplus, hcross);
 }
 
 int gwh_fourier_detector_response(const double *frequencies, int length, double *response, int detector, int model,
@@ -1703,18 +1842,11 @@ int gwh_fourier_detector_response(const double *frequencies, int length, double 
     if (!response) return gwh_set_error(GWH_ERR_INVALID, "null output");
     if (detector < 0 || detector >= GWH_NDET_TABLE)
         return gwh_set_error(GWH_ERR_UNSUPPORTED, "unsupported detector (the reference exits here)");
-    if ((rc = upload_single(frequencies, length, params, model, detector)) != GWH_OK) return rc;
-    dim3 g((length + 255) / 256);
-    if (!gwh_is_pv2(model))
-        hipLaunchKernelGGL(gwh_waveform_kernel<GWH_IMRPHENOMD>, g, dim3(256), 0, E.stream, E.f.as<const double>(),
-                           length, E.coef.as<const InstCoef>(), 1, E.out1.as<double2>(), E.out2.as<double2>());
-    else
-        hipLaunchKernelGGL(gwh_waveform_kernel<GWH_IMRPHENOMPV2>, g, dim3(256), 0, E.stream, E.f.as<const double>(),
-                           length, E.coef.as<const InstCoef>(), 1, E.out1.as<double2>(), E.out2.as<double2>());
+    SingleIO io;
+    if ((rc = upload_single(frequencies, length, params, model, detector, 1, io)) != GWH_OK) return rc;
+    launch_waveform(model, length, io, 1);
     GWH_HIP(hipGetLastError());
-    GWH_HIP(hipMemcpyAsync(response, E.out1.p, (size_t)length * 16, hipMemcpyDeviceToHost, E.stream));
-    GWH_HIP(hipStreamSynchronize(E.stream));
-    return GWH_OK;
+    return download_single(io, length, response, nullptr);
 }
 
 /* the host arrays of a call, all registered (gwh_host_data_register)? */
@@ -1898,17 +2030,6 @@ struct SingleCalls {
 };
 SingleCalls g_single;
 
-int pinned_alloc(void **host, void **dev, size_t bytes)
-{
-    if (hipHostMalloc(host, bytes, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
-        *host = nullptr;
-        return gwh_set_error(GWH_ERR_NOMEM, "pinned staging allocation failed");
-    }
-    if (hipHostGetDevicePointer(dev, *host, 0) != hipSuccess)
-        return gwh_set_error(GWH_ERR_HIP, "no device address for pinned staging");
-    return GWH_OK;
-}
-
 uint64_t pointer_tuple_hash(const CallArrays &A)
 {
     std::vector<const void *> ptrs;
@@ -1993,10 +2114,10 @@ void run_single_batch(SingleLane &L, std::vector<gwh::CoalesceItem *> &items)
             L.h_logl = L.g_logl = nullptr;
             L.cap = 0;
             const int cap = std::max(n, 256);
-            if ((rc = pinned_alloc((void **)&L.h_params, (void **)&L.g_params, (size_t)cap * sizeof(gwh_params))) ==
+            if ((rc = gwh_pinned_alloc((void **)&L.h_params, (void **)&L.g_params, (size_t)cap * sizeof(gwh_params))) ==
                     GWH_OK &&
-                (rc = pinned_alloc((void **)&L.h_events, (void **)&L.g_events, (size_t)cap * sizeof(int))) == GWH_OK &&
-                (rc = pinned_alloc((void **)&L.h_logl, (void **)&L.g_logl, (size_t)cap * sizeof(double))) == GWH_OK)
+                (rc = gwh_pinned_alloc((void **)&L.h_events, (void **)&L.g_events, (size_t)cap * sizeof(int))) == GWH_OK &&
+                (rc = gwh_pinned_alloc((void **)&L.h_logl, (void **)&L.g_logl, (size_t)cap * sizeof(double))) == GWH_OK)
                 L.cap = cap;
         }
         bool multi = false;
@@ -2256,32 +2377,7 @@ double gwh_data_snr(const double *frequencies, int length, const double *data, c
 int gwh_snr_batch(const int *events, int events0, int model, int precision, const gwh_params *params, int n,
                   double *snr)
 {
-    Engine &E = gwh_engine();
-    std::lock_guard<std::recursive_mutex> lk(E.mu);
-    int st = gwh_ensure_init();
-    if (st != GWH_OK) return st;
-    if (n <= 0) return GWH_OK;
-    if (!params || !snr) return gwh_set_error(GWH_ERR_INVALID, "null argument");
-    int rc;
-    if ((rc = E.params.ensure((size_t)n * sizeof(gwh_params))) != GWH_OK) return rc;
-    if ((rc = E.logl.ensure((size_t)n * sizeof(double))) != GWH_OK) return rc;
-    GWH_HIP(hipMemcpyAsync(E.params.p, params, (size_t)n * sizeof(gwh_params), hipMemcpyHostToDevice, E.stream));
-    const int *dev = nullptr;
-    if (events) {
-        for (int i = 0; i < n; i++)
-            if (events[i] < 0 || events[i] >= GWH_MAX_EVENTS || !E.events[events[i]].live)
-                return gwh_set_error(GWH_ERR_INVALID, "unknown event in batch");
-        if ((rc = E.inst_event.ensure((size_t)n * sizeof(int))) != GWH_OK) return rc;
-        GWH_HIP(hipMemcpyAsync(E.inst_event.p, events, (size_t)n * sizeof(int), hipMemcpyHostToDevice, E.stream));
-        dev = E.inst_event.as<const int>();
-        events0 = events[0];
-    }
-    rc = gwh_loglike_launch(dev, events0, model, precision, E.params.as<const gwh_params>(), n, E.logl.as<double>(),
-                            E.stream, false, nullptr, events, 1);
-    if (rc != GWH_OK) return rc;
-    GWH_HIP(hipMemcpyAsync(snr, E.logl.p, (size_t)n * sizeof(double), hipMemcpyDeviceToHost, E.stream));
-    GWH_HIP(hipStreamSynchronize(E.stream));
-    return GWH_OK;
+    return batch_from_host(events, events0, model, precision, params, n, snr, 1);
 }
 
 int gwh_work_counts(int event, int model, const gwh_params *params, int n, int *counts)
@@ -2321,22 +2417,14 @@ int gwh_create_coherent_GW_detection(const int *detectors, int num_detectors, co
     for (int d = 0; d < num_detectors; d++)
         if (detectors[d] < 0 || detectors[d] >= GWH_NDET_TABLE)
             return gwh_set_error(GWH_ERR_UNSUPPORTED, "unsupported detector");
-    if ((rc = upload_single(frequencies, length, params, model, detectors[0], detectors, num_detectors)) != GWH_OK)
+    SingleIO io;
+    if ((rc = upload_single(frequencies, length, params, model, detectors[0], 1, io, detectors, num_detectors)) != GWH_OK)
         return rc;
-    dim3 g((length + 255) / 256);
     for (int d = 0; d < num_detectors; d++) {
-        if (!gwh_is_pv2(model))
-            hipLaunchKernelGGL(gwh_waveform_kernel<GWH_IMRPHENOMD>, g, dim3(256), 0, E.stream, E.f.as<const double>(),
-                               length, E.coef.as<const InstCoef>(), 2, E.out1.as<double2>(), E.out2.as<double2>(), d);
-        else
-            hipLaunchKernelGGL(gwh_waveform_kernel<GWH_IMRPHENOMPV2>, g, dim3(256), 0, E.stream,
-                               E.f.as<const double>(), length, E.coef.as<const InstCoef>(), 2, E.out1.as<double2>(),
-                               E.out2.as<double2>(), d);
+        launch_waveform(model, length, io, 2, d);
         GWH_HIP(hipGetLastError());
-        GWH_HIP(hipMemcpyAsync(responses + (size_t)2 * length * d, E.out1.p, (size_t)length * 16,
-                               hipMemcpyDeviceToHost, E.stream));
+        if ((rc = download_single(io, length, responses + (size_t)2 * length * d, nullptr)) != GWH_OK) return rc;
     }
-    GWH_HIP(hipStreamSynchronize(E.stream));
     return GWH_OK;
 }
 

@@ -34,6 +34,7 @@ typedef float gwh_f4 __attribute__((ext_vector_type(4)));
 #define GWH_GRAM_ROWS 4096 /* operand rows per Gram block */
 #define GWH_FUSED_BINS 64  /* bins per block of the fused stencil + Gram kernel: one per lane of each wave */
 #define GWH_FUSED_MAX_POINTS 128 /* points per pass of the fused path (passes pipeline with the host staging) */
+#define GWH_FUSED_MIN_POINTS 16  /* fewer than these are not left for a last pass of their own */
 #ifndef GWH_FUSED_WAVES
 #define GWH_FUSED_WAVES 8 /* waves per block of the fused kernel: GWH_FROWS / GWH_FUSED_WAVES operand rows each */
 #endif
@@ -95,10 +96,16 @@ static void unpack_mod(const gwh_params &p, int basis, int var, int nmod, double
         lf[base + i] = 0;
     }
 }
-static void repack_mod(const double *v, int basis, int var, int nmod, gwh_params &q)
+/* the fields of a record that depend on its vector's element i (-1: on any).  q may hold only the bytes of a record that
+ * its model reads (gwh_record_bytes). */
+static void repack_mod(const double *v, int basis, int var, int nmod, int element, gwh_params &q)
 {
-    repack(v, basis, q);
     const int base = basis_dim(basis);
+    if (element < 0)
+        repack(v, basis, q);
+    else if (element < base)
+        repack_element(v, basis, element, q);
+    if (element >= 0 && element < base) return;
     for (int i = 0; i < nmod; i++) {
         if (var != 3) {
             q.ppe_beta[i] = v[base + i];
@@ -154,8 +161,8 @@ static double host_dtoa(double ra, double dec, double gmst, int d1, int d2)
 #define GWH_EV_SAME_PHASE 8 /* core, time and phase shift: the phase at the first detector */
 
 /* Stencil of one point: for every parameter i, S evaluations with weights c[i][s] (the difference
- * quotient including 1/eps and the log factor theta_i); instance parameter sets are appended to
- * `inst`, their GWH_EV_* bits to `flags`: GWH_EV_NO_TOF marks the order-4 +-2 eps evaluations that shift tc instead
+ * quotient including 1/eps and the log factor theta_i); the dim * S parameter sets go to `inst`, record_bytes apart,
+ * their GWH_EV_* bits to `flags`: GWH_EV_NO_TOF marks the order-4 +-2 eps evaluations that shift tc instead
  * of using the time-of-flight phase (fisher.cpp:433-453). */
 struct PointStencil {
     int S;
@@ -171,14 +178,14 @@ static double coordinate_step(double step, double v)
 }
 
 static int build_stencil(const gwh_params &p, int basis, int var, int nmod, int order, double step, int det,
-                         int ref_det, std::vector<gwh_params> &inst, std::vector<int> &flags,
-                         PointStencil &ps)
+                         int ref_det, char *inst, int record_bytes, int *flags, PointStencil &ps)
 {
     int dim = basis_dim(basis) + nmod;
     double v[GWH_FROWS];
     int lf[GWH_FROWS];
     unpack_mod(p, basis, var, nmod, v, lf);
     gwh_params base = non_parameter_options(p);
+    repack_mod(v, basis, var, nmod, -1, base); /* a stencil record differs from it where its one element enters */
     ps.S = (order >= 4) ? 4 : 2;
     for (int i = 0; i < GWH_FROWS; i++)
         for (int s = 0; s < GWH_MAXSTEN; s++) ps.c[i][s] = 0;
@@ -209,12 +216,13 @@ static int build_stencil(const gwh_params &p, int basis, int var, int nmod, int 
             double w[GWH_FROWS];
             for (int j = 0; j < dim; j++) w[j] = v[j];
             w[i] = v[i] + off[s];
-            gwh_params q = base;
-            repack_mod(w, basis, var, nmod, q);
+            gwh_params &q = *(gwh_params *)inst;
+            memcpy(inst, &base, record_bytes);
+            repack_mod(w, basis, var, nmod, i, q);
             bool two = (S == 4) && (s == 0 || s == 3);
             if (two && det != ref_det) q.tc -= host_dtoa(q.RA, q.DEC, q.gmst, ref_det, det);
-            inst.push_back(q);
-            flags.push_back(two ? GWH_EV_NO_TOF : 0);
+            *flags++ = two ? GWH_EV_NO_TOF : 0;
+            inst += record_bytes;
         }
     }
     return dim;
@@ -224,15 +232,18 @@ static int build_stencil(const gwh_params &p, int basis, int var, int nmod, int 
  * follow from fields with equal bits.  Core: masses, spins, the chi_p given, the ringdown option, the ppE / gIMR terms
  * (and for a theory's terms the distance, through its redshift).  IMRPhenomPv2 frame: core, phi_p, f_ref, inclination
  * and phase.  Phase: core, t_c and the reference: for IMRPhenomD the phase and f_ref, for IMRPhenomPv2 phi_p and f_ref
- * (its phase offset is the azimuth of J, in which inclination and phase do not enter). */
-static int shared_parts(const gwh_params &a, const gwh_params &b, bool pv2)
+ * (its phase offset is the azimuth of J, in which inclination and phase do not enter).  mod: the model has ppE / gIMR
+ * terms (the records of the others end before them). */
+static int shared_parts(const gwh_params &a, const gwh_params &b, bool pv2, bool mod)
 {
     auto eq = [](const void *x, const void *y, size_t n) { return memcmp(x, y, n) == 0; };
 #define GWH_SAME(F) eq(&a.F, &b.F, sizeof(a.F))
     if (!(GWH_SAME(mass1) && GWH_SAME(mass2) && GWH_SAME(spin1) && GWH_SAME(spin2) && GWH_SAME(chip) &&
-          GWH_SAME(dep_postmerger) && GWH_SAME(ppe_nmod) && GWH_SAME(ppe_theory) && GWH_SAME(cosmology) &&
-          GWH_SAME(ppe_b) && GWH_SAME(ppe_beta) && GWH_SAME(gimr_dphi) && GWH_SAME(gimr_dsigma) &&
-          GWH_SAME(gimr_dbeta) && GWH_SAME(gimr_dalpha) && (!a.ppe_theory || GWH_SAME(DL))))
+          GWH_SAME(dep_postmerger)))
+        return 0;
+    if (mod && !(GWH_SAME(ppe_nmod) && GWH_SAME(ppe_theory) && GWH_SAME(cosmology) && GWH_SAME(ppe_b) &&
+                 GWH_SAME(ppe_beta) && GWH_SAME(gimr_dphi) && GWH_SAME(gimr_dsigma) && GWH_SAME(gimr_dbeta) &&
+                 GWH_SAME(gimr_dalpha) && (!a.ppe_theory || GWH_SAME(DL))))
         return 0;
     int bits = GWH_EV_SAME_CORE;
     const bool ref = GWH_SAME(f_ref) && GWH_SAME(phip);
@@ -244,9 +255,9 @@ static int shared_parts(const gwh_params &a, const gwh_params &b, bool pv2)
 
 /* vector operations of one evaluation after another (the fused kernel's code, counted by hand; only the proportions
  * matter): the projections always, the rest where it is not shared */
-static int evaluation_cost(const gwh_params *prev, const gwh_params &p, bool pv2, int ndet)
+static int evaluation_cost(const gwh_params *prev, const gwh_params &p, bool pv2, bool mod, int ndet)
 {
-    const int same = prev ? shared_parts(*prev, p, pv2) : 0;
+    const int same = prev ? shared_parts(*prev, p, pv2, mod) : 0;
     int c = 20 + 14 * ndet;
     if (!(same & GWH_EV_SAME_CORE)) c += pv2 ? 330 : 150;
     if (pv2 && !(same & GWH_EV_SAME_TWIST)) c += 130;
@@ -260,15 +271,16 @@ static int evaluation_cost(const gwh_params *prev, const gwh_params &p, bool pv2
 /* Rows of the waves of the fused kernel: rows in decreasing order of their cost alone, each to the wave that ends
  * earliest with it, where what it shares with the wave's last row costs nothing.  inst: the dim * S parameter sets of
  * one point.  The choice changes only the time: an operand's value does not depend on its wave. */
-static void assign_rows(const gwh_params *inst, int dim, int S, bool pv2, int ndet, int slots,
+static void assign_rows(const char *inst, int record_bytes, int dim, int S, bool pv2, bool mod, int ndet, int slots,
                         int (*row)[GWH_FUSED_SLOTS])
 {
     int load[GWH_FUSED_WAVES] = {0}, used[GWH_FUSED_WAVES] = {0}, order[GWH_FROWS], alone[GWH_FROWS];
     auto cost = [&](int last, int i) { /* row i after row `last` (-1: first of its wave) */
         int c = 0;
         for (int s = 0; s < S; s++) {
-            const gwh_params *prev = s ? &inst[i * S + s - 1] : (last >= 0 ? &inst[last * S + S - 1] : nullptr);
-            c += evaluation_cost(prev, inst[i * S + s], pv2, ndet);
+            const int e = i * S + s, b = s ? e - 1 : (last >= 0 ? last * S + S - 1 : -1);
+            const gwh_params *prev = b >= 0 ? (const gwh_params *)(inst + (size_t)b * record_bytes) : nullptr;
+            c += evaluation_cost(prev, *(const gwh_params *)(inst + (size_t)e * record_bytes), pv2, mod, ndet);
         }
         return c;
     };
@@ -682,7 +694,8 @@ static void launch_fused(bool pv2, bool sky, dim3 g, hipStream_t st, const Stenc
  * the blocks are spread over 64 threads per element and not over four: 12 points of 1025 blocks 68 -> 8.5 us, 128
  * points of 254 blocks 18.7 -> 7.3 us. */
 __global__ __launch_bounds__(1024) void gwh_gram_reduce_kernel(const double *__restrict__ partial, int nblk, int dim,
-                                                               double scale, double *__restrict__ out)
+                                                               double scale, double *__restrict__ out,
+                                                               double *__restrict__ host)
 {
     __shared__ double red[64][17];
     const int pt = blockIdx.x, tri = gram_tri(dim);
@@ -703,6 +716,9 @@ __global__ __launch_bounds__(1024) void gwh_gram_reduce_kernel(const double *__r
         const int j = e - gram_tri(i);
         const double v = red[0][threadIdx.x] * scale;
         double *o = out + (size_t)pt * dim * dim;
+        o[i * dim + j] = v;
+        o[j * dim + i] = v;
+        o = host + (size_t)pt * dim * dim;
         o[i * dim + j] = v;
         o[j * dim + i] = v;
     }
@@ -851,69 +867,92 @@ static int fisher_run(int event, int model, int basis, int precision, const gwh_
     if (!fused && (rc = F.deriv.ensure((size_t)chunk * per_pt_bytes)) != GWH_OK) return rc;
     if ((rc = F.gram.ensure((size_t)chunk * part_bytes)) != GWH_OK) return rc;
     if ((rc = F.out.ensure((size_t)n * dim * dim * 8)) != GWH_OK) return rc;
-    std::vector<gwh_params> inst;
-    std::vector<int> flags; /* GWH_EV_* bits of every record */
-    std::vector<double> cw;
+    const bool mod = gwh_ppe_variant(model) != 0;
+    const int record_bytes = gwh_record_bytes(model);
     StencilArgs a;
     const int slots = (S == 4 || sky) ? 2 : GWH_FUSED_SLOTS; /* as launch_fused */
-    int slot = 0;
-    for (int p0 = 0; p0 < n; p0 += chunk, slot ^= 1) {
-        int np = std::min(chunk, n - p0);
-        inst.clear();
-        flags.clear();
-        cw.assign((size_t)np * GWH_FROWS * GWH_MAXSTEN, 0.0);
-        inst.reserve((size_t)np * per_point);
+    const size_t out_bytes = (size_t)dim * dim * 8; /* a point's matrix */
+    /* the pass that each staging holds, whose matrices the caller does not have yet */
+    struct Pending {
+        int p0, np;
+        const char *m;
+    } pending[2] = {{0, 0, nullptr}, {0, 0, nullptr}};
+    auto collect = [&](int sl) {
+        if (!pending[sl].np) return GWH_OK;
+        GWH_HIP(hipEventSynchronize(F.stage_done[sl]));
+        memcpy(out + (size_t)pending[sl].p0 * dim * dim, pending[sl].m, pending[sl].np * out_bytes);
+        pending[sl].np = 0;
+        return GWH_OK;
+    };
+    /* buffers of the largest pass */
+    const size_t ni_max = (size_t)chunk * per_point,
+                 misc_max = (size_t)chunk * GWH_FROWS * GWH_MAXSTEN * 8 + (ni_max * 4 + 7) / 8 * 8,
+                 stage_max = ni_max * record_bytes + misc_max + chunk * out_bytes;
+    if ((rc = F.coef.ensure(ni_max * sizeof(InstCoef))) != GWH_OK) return rc;
+    if ((rc = F.misc.ensure(misc_max + 256)) != GWH_OK) return rc;
+    /* the device waits for the host to build the first pass: of several, the first two are a quarter and a half of the
+       others */
+    int slot = 0, pass = (fused && n > chunk) ? std::max(1, chunk / 4) : chunk;
+    for (int p0 = 0, np; p0 < n; p0 += np, slot ^= 1, pass = std::min(2 * pass, chunk)) {
+        np = std::min(pass, n - p0);
+        if (fused && n - p0 - np < GWH_FUSED_MIN_POINTS && n - p0 <= chunk) np = n - p0;
+        const int ni = np * per_point;
+        const size_t ncw = (size_t)np * GWH_FROWS * GWH_MAXSTEN;
+        /* a pass in pinned memory, which the kernels read and write: records, weights and flags (these two copied by the
+           setup's launch), then the matrices.  As copies on the stream these took 50 us between two passes (384 points:
+           1241 -> 1065 us; building whole records anew for every stencil point, and the first pass no shorter than the
+           others: 1348 us). */
+        const size_t rec_bytes = (size_t)ni * record_bytes, flag_bytes = ((size_t)ni * 4 + 7) / 8 * 8,
+                     misc_bytes = ncw * 8 + flag_bytes;
+        if (F.stage_done[slot]) GWH_HIP(hipEventSynchronize(F.stage_done[slot])); /* its last pass has ended */
+        else GWH_HIP(hipEventCreateWithFlags(&F.stage_done[slot], hipEventDisableTiming));
+        if ((rc = collect(slot)) != GWH_OK) return rc;
+        if (F.stage_cap[slot] < stage_max) {
+            if (F.stage[slot]) GWH_HIP(hipHostFree(F.stage[slot]));
+            F.stage[slot] = nullptr;
+            F.stage_cap[slot] = 0;
+            if ((rc = gwh_pinned_alloc(&F.stage[slot], &F.stage_dev[slot], stage_max + stage_max / 4)) != GWH_OK) return rc;
+            F.stage_cap[slot] = stage_max + stage_max / 4;
+        }
+        char *st = (char *)F.stage[slot];
+        double *cw = (double *)(st + rec_bytes);
+        int *flags = (int *)(cw + ncw); /* GWH_EV_* bits of every record */
+        double fcut = 0;                /* highest cutoff of a record */
         for (int q = 0; q < np; q++) {
             PointStencil ps;
-            build_stencil(params[p0 + q], basis, gwh_ppe_variant(model), nmod, order, eps, det_for_tof, ref_det,
-                          inst, flags, ps);
-            if (sky) {
-                inst.push_back(params[p0 + q]); /* central amplitude: the caller's parameters */
-                flags.push_back(0);
+            char *rec = st + (size_t)q * per_point * record_bytes;
+            int *fl = flags + (size_t)q * per_point;
+            build_stencil(params[p0 + q], basis, gwh_ppe_variant(model), nmod, order, eps, det_for_tof, ref_det, rec,
+                          record_bytes, fl, ps);
+            if (sky) { /* central amplitude: the caller's parameters */
+                memcpy(rec + (size_t)(per_point - 1) * record_bytes, &params[p0 + q], record_bytes);
+                fl[per_point - 1] = 0;
             }
+            auto at = [&](int e) -> const gwh_params & { return *(const gwh_params *)(rec + (size_t)e * record_bytes); };
             if (fused) {
-                const gwh_params *rec = &inst[(size_t)q * per_point];
-                if (p0 == 0 && q == 0) assign_rows(rec, dim, S, pv2, sky ? 1 : d_count, slots, a.row);
+                if (p0 == 0 && q == 0)
+                    assign_rows(rec, record_bytes, dim, S, pv2, mod, sky ? 1 : d_count, slots, a.row);
                 for (int w = 0; w < GWH_FUSED_WAVES; w++) {
                     int prev = -1;
                     for (int h = 0; h < slots && a.row[w][h] >= 0; h++)
                         for (int e = a.row[w][h] * S; e < (a.row[w][h] + 1) * S; prev = e++)
-                            if (prev >= 0) flags[(size_t)q * per_point + e] |= shared_parts(rec[prev], rec[e], pv2);
+                            if (prev >= 0) fl[e] |= shared_parts(at(prev), at(e), pv2, mod);
                 }
             }
-            for (int i = 0; i < GWH_FROWS; i++)
-                for (int s = 0; s < GWH_MAXSTEN; s++) cw[((size_t)q * GWH_FROWS + i) * GWH_MAXSTEN + s] = ps.c[i][s];
+            for (int e = 0; e < per_point; e++) {
+                const double c = .2 / (at(e).mass1 * GWH_MSOL_SEC + at(e).mass2 * GWH_MSOL_SEC);
+                if (!(c <= fcut || fcut != fcut)) fcut = c; /* NaN stays: every chunk */
+            }
+            memcpy(cw + (size_t)q * GWH_FROWS * GWH_MAXSTEN, ps.c, sizeof(ps.c));
         }
-        int ni = (int)inst.size();
-        if ((rc = F.params.ensure((size_t)ni * sizeof(gwh_params))) != GWH_OK) return rc;
-        if ((rc = F.coef.ensure((size_t)ni * sizeof(InstCoef))) != GWH_OK) return rc;
-        if ((rc = F.misc.ensure(cw.size() * 8 + flags.size() * 4 + 256)) != GWH_OK) return rc;
-        /* stage the pass in pinned memory (asynchronous copies; the device buffers are reused in stream order) */
-        const size_t rec_bytes = (size_t)ni * sizeof(gwh_params), misc_bytes = cw.size() * 8 + flags.size() * 4,
-                     stage_bytes = rec_bytes + misc_bytes;
-        if (F.stage_done[slot]) GWH_HIP(hipEventSynchronize(F.stage_done[slot])); /* its last copy has run */
-        else GWH_HIP(hipEventCreateWithFlags(&F.stage_done[slot], hipEventDisableTiming));
-        if (F.stage_cap[slot] < stage_bytes) {
-            if (F.stage[slot]) GWH_HIP(hipHostFree(F.stage[slot]));
-            F.stage[slot] = nullptr;
-            F.stage_cap[slot] = 0;
-            GWH_HIP(hipHostMalloc(&F.stage[slot], stage_bytes + stage_bytes / 4, hipHostMallocDefault));
-            F.stage_cap[slot] = stage_bytes + stage_bytes / 4;
-        }
-        char *st = (char *)F.stage[slot];
-        memcpy(st, inst.data(), rec_bytes);
-        memcpy(st + rec_bytes, cw.data(), cw.size() * 8);
-        memcpy(st + rec_bytes + cw.size() * 8, flags.data(), flags.size() * 4);
-        GWH_HIP(hipMemcpyAsync(F.params.p, st, rec_bytes, hipMemcpyHostToDevice, F.stream));
-        char *misc = (char *)F.misc.p;
-        GWH_HIP(hipMemcpyAsync(misc, st + rec_bytes, misc_bytes, hipMemcpyHostToDevice, F.stream));
-        GWH_HIP(hipEventRecord(F.stage_done[slot], F.stream));
-        if ((rc = gwh_setup_launch(nullptr, event, model, F.params.as<const gwh_params>(), ni, F.coef.as<InstCoef>(),
-                                   F.stream)) != GWH_OK)
+        char *misc = (char *)F.misc.p, *dev = (char *)F.stage_dev[slot];
+        if ((rc = gwh_setup_launch(nullptr, event, model, (const gwh_params *)dev, ni, F.coef.as<InstCoef>(), F.stream,
+                                   record_bytes, {(const double *)(dev + rec_bytes), (double *)misc,
+                                                  (int)(misc_bytes / 8)})) != GWH_OK)
             return rc;
         a.coef = F.coef.as<const InstCoef>();
         a.cw = (const double *)misc;
-        a.flags = (const int *)(misc + cw.size() * 8);
+        a.flags = (const int *)(misc + ncw * 8);
         a.dim = dim;
         a.S = S;
         a.per_point = per_point;
@@ -941,11 +980,6 @@ static int fisher_run(int event, int model, int basis, int precision, const gwh_
             /* only the 64-bin chunks that begin at or below some record's cutoff 0.2/M hold anything (a margin covers
                the rounding of the device's own cutoff, which decides bin by bin): 77 of 254 chunks for 65 solar masses
                on 20-2048 Hz */
-            double fcut = 0;
-            for (const gwh_params &p : inst) {
-                const double c = .2 / (p.mass1 * GWH_MSOL_SEC + p.mass2 * GWH_MSOL_SEC);
-                if (!(c <= fcut || fcut != fcut)) fcut = c; /* NaN stays: every chunk */
-            }
             const std::vector<double> &cf = *ev.chunk_fmin;
             while (nb > 1 && cf[nb - 1] > fcut * (1 + 1e-9)) nb--;
             launch_fused(pv2, sky, dim3(nb, np), F.stream, a, evp, event, F.gram.as<double>());
@@ -957,8 +991,11 @@ static int fisher_run(int event, int model, int basis, int precision, const gwh_
         }
         GWH_HIP(hipGetLastError());
         hipLaunchKernelGGL(gwh_gram_reduce_kernel, dim3(np, (gram_tri(dim) + 15) / 16), dim3(1024), 0, F.stream, F.gram.as<const double>(),
-                           nb, dim, scale, F.out.as<double>() + (size_t)p0 * dim * dim);
+                           nb, dim, scale, F.out.as<double>() + (size_t)p0 * dim * dim,
+                           (double *)(dev + rec_bytes + misc_bytes));
         GWH_HIP(hipGetLastError());
+        GWH_HIP(hipEventRecord(F.stage_done[slot], F.stream));
+        pending[slot] = {p0, np, st + rec_bytes + misc_bytes};
     }
     if (sigma) {
         if ((rc = F.sig.ensure((size_t)n * dim * 8)) != GWH_OK) return rc;
@@ -967,8 +1004,9 @@ static int fisher_run(int event, int model, int basis, int precision, const gwh_
         GWH_HIP(hipGetLastError());
         GWH_HIP(hipMemcpyAsync(sigma, F.sig.p, (size_t)n * dim * 8, hipMemcpyDeviceToHost, F.stream));
     }
-    GWH_HIP(hipMemcpyAsync(out, F.out.p, (size_t)n * dim * dim * 8, hipMemcpyDeviceToHost, F.stream));
-    GWH_HIP(hipStreamSynchronize(F.stream));
+    for (int k = 0; k < 2; k++, slot ^= 1)
+        if ((rc = collect(slot)) != GWH_OK) return rc;
+    if (sigma) GWH_HIP(hipStreamSynchronize(F.stream));
     return GWH_OK;
 }
 
@@ -1031,9 +1069,8 @@ size_t gwh_fisher_batch_bytes(int event, int model, int basis, int precision, co
            gwh_grown_capacity(chunk * part_bytes, F.gram.cap) +
            gwh_grown_capacity((size_t)n * dim * dim * 8, F.out.cap) +
            (want_sigma ? gwh_grown_capacity((size_t)n * dim * 8, F.sig.cap) : F.sig.cap) +
-           gwh_grown_capacity(ni * sizeof(gwh_params), F.params.cap) +
            gwh_grown_capacity(ni * sizeof(InstCoef), F.coef.cap) +
-           gwh_grown_capacity(chunk * GWH_FROWS * GWH_MAXSTEN * 8 + ni * 4 + 256, F.misc.cap) + F.raw.cap;
+           gwh_grown_capacity(chunk * GWH_FROWS * GWH_MAXSTEN * 8 + (ni * 4 + 7) / 8 * 8 + 256, F.misc.cap) + F.raw.cap;
 }
 
 extern "C" {

@@ -414,8 +414,16 @@ int gwh_maximized_loglike_batch(int event, int model, const gwh_params *params, 
     if (chunk > 65535) chunk = 65535;
     /* the extrinsic values the intrinsic likelihood fixes (mcmc_gw.cpp:2611-2617 IMRPhenomD, :2660-2666 Pv2);
      * the statistics are invariant under the IMRPhenomD ones (amplitude, phase, time), not under Pv2's */
-    std::vector<gwh_params> q(params, params + n);
-    for (auto &p : q) {
+    /* a batch of one pass goes through pinned memory as the likelihood batches do, results included */
+    int record_bytes = gwh_record_bytes(model);
+    const size_t rec = (size_t)n * record_bytes;
+    const bool staged = n <= chunk && rec + (size_t)n * 8 <= GWH_STAGE_MAX;
+    if (!staged) record_bytes = sizeof(gwh_params);
+    std::vector<gwh_params> q(staged ? 0 : n);
+    if (staged && (rc = E.stage.ensure(rec + (size_t)n * 8)) != GWH_OK) return rc;
+    for (int i = 0; i < n; i++) {
+        gwh_params &p = staged ? *(gwh_params *)(E.stage.h + (size_t)i * record_bytes) : q[i];
+        memcpy((void *)&p, params + i, record_bytes);
         p.psi = 0;
         p.phiRef = 1;
         p.incl = 0;
@@ -434,9 +442,11 @@ int gwh_maximized_loglike_batch(int event, int model, const gwh_params *params, 
     const double hh_scale = ev.df_fisher / ev.df_like;  /* the stored Simpson step -> f[1] - f[0] */
     for (int i0 = 0; i0 < n; i0 += chunk) {
         const int m = std::min(chunk, n - i0);
-        GWH_HIP(hipMemcpyAsync(E.params.p, q.data() + i0, (size_t)m * sizeof(gwh_params), hipMemcpyHostToDevice, st));
-        if ((rc = gwh_setup_launch(nullptr, event, model, E.params.as<const gwh_params>(), m, E.coef.as<InstCoef>(),
-                                   st)) != GWH_OK)
+        const gwh_params *d_params = staged ? (const gwh_params *)E.stage.g : E.params.as<const gwh_params>();
+        if (!staged)
+            GWH_HIP(hipMemcpyAsync(E.params.p, q.data() + i0, (size_t)m * sizeof(gwh_params), hipMemcpyHostToDevice, st));
+        if ((rc = gwh_setup_launch(nullptr, event, model, d_params, m, E.coef.as<InstCoef>(), st, record_bytes)) !=
+            GWH_OK)
             return rc;
         dim3 g(nblk, m);
         if (pv2)
@@ -454,11 +464,12 @@ int gwh_maximized_loglike_batch(int event, int model, const gwh_params *params, 
                            E.fft.as<const double2>(), E.mxpart.as<const double>(), hh_scale, df, stat);
         GWH_HIP(hipGetLastError());
         hipLaunchKernelGGL(gwh_maxll_network_kernel, dim3((m + GWH_MX_TPB - 1) / GWH_MX_TPB), dim3(GWH_MX_TPB), 0, st, m,
-                           D, (const double *)stat, E.mxres.as<double>());
+                           D, (const double *)stat, staged ? (double *)(E.stage.g + rec) : E.mxres.as<double>());
         GWH_HIP(hipGetLastError());
-        GWH_HIP(hipMemcpyAsync(out + i0, E.mxres.p, (size_t)m * 8, hipMemcpyDeviceToHost, st));
+        if (!staged) GWH_HIP(hipMemcpyAsync(out + i0, E.mxres.p, (size_t)m * 8, hipMemcpyDeviceToHost, st));
     }
     GWH_HIP(hipStreamSynchronize(st));
+    if (staged) memcpy(out, E.stage.h + rec, (size_t)n * 8);
     return GWH_OK;
 }
 
