@@ -12,7 +12,7 @@ step), so per-step latencies give p50/p99.
 of the detector phases through the FP64 tables), on the tiling the autotuner picks for the event before the
 warm-up.  Reported beside it: the FP64 batched engine, the
 plain FP64 one-instance-per-launch path, max |delta logL| mixed vs FP64 over every timed evaluation, the same for
-IMRPhenomPv2 on the same grid (1024 chains; its mixed mode keeps FP64 table-driven sin/cos and exponentials),
+IMRPhenomPv2 on the same grid (1024 chains; its mixed mode runs the FP64 kernels),
 kernel-level roofline from HIP events, the single-detector workload with its sky-averaged Fisher, batched
 13-parameter IMRPhenomPv2 Fisher matrices, the tempering step on the device, the FFT-maximised likelihood, the
 uneven multi-event batch, the serving broker, the reference-signature C++ layer called from many host threads,
