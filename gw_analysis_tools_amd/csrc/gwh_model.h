@@ -290,7 +290,7 @@ struct DetGeom {
  * instructions, which few waves execute once: 78 KB (IMRPhenomD) and 99 KB (IMRPhenomPv2), more than the instruction
  * cache, while everything was written out.  Amplitude, orientation, detector and precession parts
  * take few divisions, powers and angles: 70 KB and 72 KB; with the half-filled blocks of gwh_setup_kernel 512 instances
- * of IMRPhenomD 11.3 -> 9.0 us, 1024 of IMRPhenomPv2 17.5 -> 14.9 us.
+ * of IMRPhenomD 11.3 -> 9.6 us (10.2 -> 8.9 in a tempering step), 1024 of IMRPhenomPv2 17.5 -> 14.9 us.
  *
  * The phase and its connection keep the order of operations that they have always had: the slopes of its pieces are
  * differences of large terms, whose rounding a difference quotient in a small parameter magnifies (with the phase
