@@ -4,7 +4,7 @@
  *
  * Hot path (one MCMC step):
  *   1. gwh_setup_kernel      FP64 InstCoef record of every instance: four waves per
- *                            64 instances compute independent parts, joined in LDS
+ *                            32 instances compute independent parts, joined in LDS
  *   2. loglike kernel        (instance, bin-tile) work items, one block each
  *                            (gwh_tiles.h): in tile-major order for one event
  *                            (or events whose sizes are known only on the
