@@ -889,7 +889,8 @@ __device__ __forceinline__ void gwh_setup_mass(const gwh_params &p, int ppe, Set
 struct Pv2Frame {
     double cJN, sJN, c2z, s2z, alpha0, phi_aligned;
 };
-/* cosine and sine of atan2(y, x); atan2(0, 0) = 0.  Scaled by a power of 2, so that no square under- or overflows. */
+/* cosine and sine of atan2(y, x), which is 0 or pi where x and y are zeros, by the sign of x.  Scaled by a power of 2, so
+ * that no square under- or overflows. */
 __device__ __forceinline__ void gwh_direction(double x, double y, double &c, double &s)
 {
     const int e = -__builtin_amdgcn_frexp_exp(fmax(fabs(x), fabs(y)));
@@ -897,7 +898,7 @@ __device__ __forceinline__ void gwh_direction(double x, double y, double &c, dou
     x = ldexp(x, e);
     y = ldexp(y, e);
     const double ih = none ? 0.0 : 1.0 / sqrt(x * x + y * y);
-    c = none ? 1.0 : x * ih;
+    c = none ? copysign(1.0, x) : x * ih;
     s = y * ih;
 }
 __device__ __forceinline__ void gwh_rotz_cs(double c, double s, double &x, double &y)
@@ -919,21 +920,31 @@ __device__ __forceinline__ Pv2Frame gwh_setup_frame(const gwh_params &p, const S
     const bool reduced = (p.chip + 1) > 1e-10;
     const double m1_2 = S.m1 * S.m1, m2_2 = S.m2 * S.m2;
     double L0 = S.M * S.M * gwh_l2pn(S.eta, cbrt(GWH_PI * S.M * p.f_ref));
-    double J0x, J0y;
-    if (reduced) {
-        double sp, cp;
-        gwh_sincos_cw(p.phip, sp, cp);
-        J0x = m1_2 * chip * cp;
-        J0y = m1_2 * chip * sp;
-    } else {
-        J0x = m1_2 * s1x + m2_2 * s2x;
-        J0y = m1_2 * s1y + m2_2 * s2y;
+    /* total angular momentum; no fused products, so that in-plane spins that cancel leave what they leave in the reference
+       and not the rounding error of one of the products, whose direction would become the frame's */
+    double J0x, J0y, J0z, J0;
+    {
+#pragma clang fp contract(off)
+        if (reduced) {
+            double sp, cp;
+            gwh_sincos_cw(p.phip, sp, cp);
+            J0x = m1_2 * chip * cp;
+            J0y = m1_2 * chip * sp;
+        } else {
+            J0x = m1_2 * s1x + m2_2 * s2x;
+            J0y = m1_2 * s1y + m2_2 * s2y;
+        }
+        J0z = L0 + m1_2 * S.chi1 + m2_2 * S.chi2;
+        J0 = sqrt(J0x * J0x + J0y * J0y + J0z * J0z);
     }
-    double J0z = L0 + m1_2 * S.chi1 + m2_2 * S.chi2;
     /* rotation by -phiJ about z, then by -thetaJ about y */
     double cP, sP, cJ, sJ, cK, sK;
     gwh_direction(J0x, J0y, cP, sP);
     gwh_direction(J0z, J0x * cP + J0y * sP, cJ, sJ);
+    if (fabs(J0z) == J0 && J0 < HUGE_VAL) { /* a tilt that the reference's acos(J0z / J0) rounds to 0 or pi */
+        cJ = copysign(1.0, J0z);
+        sJ = J0z < 0 ? 1.2246467991473532e-16 : 0.0; /* sin of the double next to pi */
+    }
     sP = -sP;
     sJ = -sJ;
     Pv2Frame F;
@@ -950,9 +961,12 @@ __device__ __forceinline__ Pv2Frame gwh_setup_frame(const gwh_params &p, const S
     const double NxJ = tx * cK - ty * sK, NzJ = tz;
     F.cJN = NzJ;
     F.sJN = sqrt(tx * tx + ty * ty);
-    /* the orbital axis */
-    tx = sJ;
+    /* the orbital axis, turned in full: where J lies along it alpha0 is 0 or pi by the signs of zeros */
+    tx = 0.;
     ty = 0.;
+    tz = 1.;
+    gwh_rotz_cs(cP, sP, tx, ty);
+    gwh_roty_cs(cJ, sJ, tx, tz);
     gwh_rotz_cs(cK, sK, tx, ty);
     F.alpha0 = atan2(ty, tx);
     tx = -ci * sph;

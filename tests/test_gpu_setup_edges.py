@@ -42,6 +42,21 @@ def _edges(kind):
             add(mass1=m[0], mass2=m[1])
         for c in (0., .3, 1.):
             add(chip=c, phip=2.)
+    elif kind == "cancelling":
+        # J along the orbital axis with chi_p > 0: exactly, to rounding, within a tilt that acos(J_z / J) cannot resolve,
+        # with zeros of either sign, and against the axis; the line of sight in all four quadrants
+        for phi in (0.2, 1.9, 3.5, 5.5):
+            for s in (.5, .25, .3, .7):
+                for a in (s, -s):
+                    add(mass1=30., mass2=30., spin1=[a, 0, .2], spin2=[-a, 0, .2], incl=1.2, phiRef=phi)
+                    add(mass1=30., mass2=30., spin1=[0, a, .2], spin2=[0, -a, -.1], incl=2.3, phiRef=phi)
+                    add(mass1=30., mass2=30., spin1=[a, -.1, .2], spin2=[-a, .1, .2], incl=1.2, phiRef=phi)
+                    add(mass1=30., mass2=15., spin1=[a / 4, 0, .2], spin2=[-a, 0, .2], incl=.8, phiRef=phi)
+                    add(mass1=80., mass2=10., spin1=[a / 64, 0, -.95], spin2=[-a, 0, 0], incl=1.2, phiRef=phi)
+            for x in (1e-12, -1e-12):
+                add(mass1=30., mass2=30., spin1=[.5, x, .2], spin2=[-.5, 0, .2], incl=1.2, phiRef=phi)
+                add(mass1=30., mass2=30., spin1=[x, .5, .2], spin2=[0, -.5, .2], incl=1.2, phiRef=phi)
+            add(mass1=30., mass2=30., spin1=[-0., .5, .2], spin2=[-0., -.5, .2], incl=1.2, phiRef=phi)
     elif kind == "reference":
         for fr in (5., 20., 60., 100., 200., 300., 500., 1000.):
             for st in (0, 1):
@@ -54,7 +69,8 @@ def _edges(kind):
     return np.array(out, dtype=base.dtype)
 
 
-@pytest.mark.parametrize("kind,model", [("geometry", G.IMRPHENOMPV2), ("reference", G.IMRPHENOMD),
+@pytest.mark.parametrize("kind,model", [("geometry", G.IMRPHENOMPV2), ("cancelling", G.IMRPHENOMPV2),
+                                        ("reference", G.IMRPHENOMD),
                                         ("reference", G.IMRPHENOMPV2), ("angles", G.IMRPHENOMD)])
 def test_degenerate_setups_match_oracle(net, kind, model):
     f, psd, data, ev = net
