@@ -209,7 +209,8 @@ struct Event {
     uint64_t last_use = 0;
     int pins = 0;          /* step graphs holding this event's buffers: no destroy, eviction or re-tiling */
     int method = 0, log10F = 0; /* integration rule of the stored weights */
-    std::shared_ptr<const std::vector<double>> chunk_fmin; /* host: smallest frequency of every chunk of 64 bins */
+    /* host: smallest frequency of every chunk of 64 bins; -infinity where a weight may not be finite */
+    std::shared_ptr<const std::vector<double>> chunk_fmin;
 };
 
 /* grow-only device buffer; a fixed one is a view of memory the buffer does not own (never grown or freed:

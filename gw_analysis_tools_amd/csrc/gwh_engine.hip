@@ -424,7 +424,15 @@ int gwh_event_create_ex(const double *f, int N, int ndet, const int *dets, const
     /* Gauss-Legendre weights carry no step: nothing to rescale */
     ds.snr_scale = (method == GWH_GAUSSLEG) ? 1.0 : df_f / ev.df_like;
     auto chunk_fmin = std::make_shared<std::vector<double>>((N + 63) / 64, HUGE_VAL);
-    for (int k = 0; k < N; k++) (*chunk_fmin)[k / 64] = std::fmin((*chunk_fmin)[k / 64], f[k]);
+    for (int k = 0; k < N; k++) {
+        double &m = (*chunk_fmin)[k / 64];
+        m = std::fmin(m, f[k]);
+        /* a bin whose weight may not be a number once rooted (gwh_event_prep_kernel) spoils every matrix that it enters,
+           above the cutoff too: 0 times that is none, with or without lighter points in the pass */
+        const double w = (weights ? weights[k] : dfac) * (log10_jac ? f[k] : 1.0);
+        for (int d = 0; d < ndet; d++)
+            if (!(w >= 0 && w < HUGE_VAL && psd[(size_t)d * N + k] > w * 1e-300)) m = -HUGE_VAL;
+    }
     ev.chunk_fmin = chunk_fmin;
     ds.sorted = 1;
     for (int k = 1; k < N; k++)

@@ -110,3 +110,22 @@ def test_a_point_without_masses_leaves_the_others_alone():
         alone = G.fisher_batch(ev, P[i:i + 1], G.IMRPHENOMD, G.BASIS_PHENOMD_FULL, 11, epsilon=1e-6)[0]
         assert np.linalg.norm(a[i] - alone) <= 1e-12 * np.linalg.norm(alone)
     ev.close()
+
+
+@pytest.mark.parametrize("psd_bin", [0., -1e-46, np.nan])
+@pytest.mark.parametrize("at", [0.6, 0.95])
+def test_a_weight_without_a_value_does_not_depend_on_the_neighbours(psd_bin, at):
+    """a bin whose noise is zero, negative or not a number leaves no matrix of the event a value, above a point's cutoff
+    too (0 times such a weight), whether or not a lighter point in the pass reaches the bin's chunk"""
+    f = W.uniform_grid(20., 2000., 0.5)
+    psd = W.analytic_psd(f)
+    psd[int(at * len(f))] = psd_bin
+    ev = G.Event(f, [np.zeros(len(f), complex)] * 2, [W.analytic_psd(f), psd], [0, 1])
+    P = np.concatenate([W.injection_params(1, mass1=m, mass2=0.6 * m) for m in (90., 4., 60.)])
+    for model, basis, dim in ((G.IMRPHENOMD, G.BASIS_PHENOMD_MCMC, 11), (G.IMRPHENOMPV2, G.BASIS_PV2_FULL, 13)):
+        P["chip"], P["phip"] = 0.3, 0.7
+        F = G.fisher_batch(ev, P, model, basis, dim, epsilon=-1e-7)
+        for i in range(len(P)):
+            one = G.fisher_batch(ev, P[i:i + 1], model, basis, dim, epsilon=-1e-7)
+            assert not np.any(np.isfinite(F[i])) and np.array_equal(F[i], one[0], equal_nan=True)
+    ev.close()
