@@ -129,3 +129,17 @@ def test_a_weight_without_a_value_does_not_depend_on_the_neighbours(psd_bin, at)
             one = G.fisher_batch(ev, P[i:i + 1], model, basis, dim, epsilon=-1e-7)
             assert not np.any(np.isfinite(F[i])) and np.array_equal(F[i], one[0], equal_nan=True)
     ev.close()
+
+
+@pytest.mark.parametrize("tail", [np.inf, np.nan])
+def test_bins_without_a_frequency_count_nothing(tail):
+    """a grid padded with infinities or NaN, below and above the cutoff inside one chunk of 64: such bins are above every cutoff"""
+    f = np.linspace(20., 800., 100)
+    psd = W.analytic_psd(f)
+    f[-3:] = tail
+    for model, basis, dim, kw in CASES[1:5]:
+        p = _params(kw)
+        d = G.fisher_derivatives(f, basis, 1, 0, dim, p, model=model)
+        assert np.all(d[:, -3:] == 0)
+        F = G.fisher_numerical(f, psd, basis, 1, 0, dim, p, model=model)
+        assert _norm_err(F, _gram(f, psd, d)) <= TOL
