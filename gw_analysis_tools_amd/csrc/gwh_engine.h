@@ -251,6 +251,25 @@ struct HostStage {
     int ensure(size_t bytes); /* only with no work in flight that uses it */
 };
 
+/* Waits for the stream when the call that holds it ends early: kernels that read or write pinned staging may still run,
+ * and the next call overwrites or frees it.  done(): the call has waited itself. */
+struct SettleStream {
+    hipStream_t stream;
+    bool armed = true;
+    explicit SettleStream(hipStream_t st) : stream(st) {}
+    SettleStream(const SettleStream &) = delete;
+    SettleStream &operator=(const SettleStream &) = delete;
+    ~SettleStream()
+    {
+        if (armed) (void)hipStreamSynchronize(stream);
+    }
+    int done()
+    {
+        armed = false;
+        return GWH_OK;
+    }
+};
+
 /* Bytes of a parameter record that a model's setup reads: the GR models none of the modified-gravity terms, which are
  * the last two thirds of it.  Records of a batch may lie that far apart. */
 inline int gwh_record_bytes(int model)

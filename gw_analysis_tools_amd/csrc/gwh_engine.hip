@@ -1482,16 +1482,14 @@ static int batch_from_host(const int *events, int events0, int model, int precis
         d_params = E.params.as<const gwh_params>();
         d_out = E.logl.as<double>();
     }
+    SettleStream settle(E.stream);
     rc = gwh_loglike_launch(events ? E.inst_event.as<const int>() : nullptr, events ? events[0] : events0, model,
                             precision, d_params, n, d_out, E.stream, false, nullptr, events, what, nullptr, &X);
-    if (rc != GWH_OK) {
-        (void)hipStreamSynchronize(E.stream); /* nothing in flight when the staging is used next */
-        return rc;
-    }
+    if (rc != GWH_OK) return rc;
     if (!staged) GWH_HIP(hipMemcpyAsync(out, d_out, res, hipMemcpyDeviceToHost, E.stream));
     GWH_HIP(hipStreamSynchronize(E.stream));
     if (staged) memcpy(out, E.stage.h + rec + ids, res);
-    return GWH_OK;
+    return settle.done();
 }
 
 int gwh_loglike_batch(const int *events, int events0, int model, int precision, const gwh_params *params, int n,
@@ -1833,10 +1831,12 @@ int gwh_fourier_waveform(const double *frequencies, int length, double *hplus, d
     if ((rc = check_common(frequencies, length, params, model)) != GWH_OK) return rc;
     if (!hplus || !hcross) return gwh_set_error(GWH_ERR_INVALID, "null output");
     SingleIO io;
+    SettleStream settle(E.stream);
     if ((rc = upload_single(frequencies, length, params, model, 0, 2, io)) != GWH_OK) return rc;
     launch_waveform(model, length, io, 0);
     GWH_HIP(hipGetLastError());
-    return download_single(io, length, hplus, hcross);
+    if ((rc = download_single(io, length, hplus, hcross)) != GWH_OK) return rc;
+    return settle.done();
 }
 
 int gwh_fourier_detector_response(const double *frequencies, int length, double *response, int detector, int model,
@@ -1851,10 +1851,12 @@ int gwh_fourier_detector_response(const double *frequencies, int length, double 
     if (detector < 0 || detector >= GWH_NDET_TABLE)
         return gwh_set_error(GWH_ERR_UNSUPPORTED, "unsupported detector (the reference exits here)");
     SingleIO io;
+    SettleStream settle(E.stream);
     if ((rc = upload_single(frequencies, length, params, model, detector, 1, io)) != GWH_OK) return rc;
     launch_waveform(model, length, io, 1);
     GWH_HIP(hipGetLastError());
-    return download_single(io, length, response, nullptr);
+    if ((rc = download_single(io, length, response, nullptr)) != GWH_OK) return rc;
+    return settle.done();
 }
 
 /* the host arrays of a call, all registered (gwh_host_data_register)? */
@@ -2426,6 +2428,7 @@ int gwh_create_coherent_GW_detection(const int *detectors, int num_detectors, co
         if (detectors[d] < 0 || detectors[d] >= GWH_NDET_TABLE)
             return gwh_set_error(GWH_ERR_UNSUPPORTED, "unsupported detector");
     SingleIO io;
+    SettleStream settle(E.stream);
     if ((rc = upload_single(frequencies, length, params, model, detectors[0], 1, io, detectors, num_detectors)) != GWH_OK)
         return rc;
     for (int d = 0; d < num_detectors; d++) {
@@ -2433,7 +2436,7 @@ int gwh_create_coherent_GW_detection(const int *detectors, int num_detectors, co
         GWH_HIP(hipGetLastError());
         if ((rc = download_single(io, length, responses + (size_t)2 * length * d, nullptr)) != GWH_OK) return rc;
     }
-    return GWH_OK;
+    return settle.done();
 }
 
 } /* extern "C" */

@@ -900,6 +900,7 @@ static int fisher_run(int event, int model, int basis, int precision, const gwh_
     if ((rc = F.misc.ensure(misc_max + 256)) != GWH_OK) return rc;
     /* the device waits for the host to build the first pass: of several, the first two are a quarter and a half of the
        others */
+    SettleStream settle(F.stream);
     int slot = 0, pass = (fused && n > chunk) ? std::max(1, chunk / 4) : chunk;
     for (int p0 = 0, np; p0 < n; p0 += np, slot ^= 1, pass = std::min(2 * pass, chunk)) {
         np = std::min(pass, n - p0);
@@ -981,7 +982,7 @@ static int fisher_run(int event, int model, int basis, int precision, const gwh_
             GWH_HIP(hipGetLastError());
             GWH_HIP(hipMemcpyAsync(raw, F.raw.p, (size_t)dim * N * 16, hipMemcpyDeviceToHost, F.stream));
             GWH_HIP(hipStreamSynchronize(F.stream));
-            return GWH_OK;
+            return settle.done();
         }
         int nb = nblk; /* partial Gram matrices of a point */
         if (fused) {
@@ -1015,7 +1016,7 @@ static int fisher_run(int event, int model, int basis, int precision, const gwh_
     for (int k = 0; k < 2; k++, slot ^= 1)
         if ((rc = collect(slot)) != GWH_OK) return rc;
     if (sigma) GWH_HIP(hipStreamSynchronize(F.stream));
-    return GWH_OK;
+    return settle.done();
 }
 
 int gwh_fisher_batch_with(int event, int model, int basis, int precision, const gwh_params *params, int n, int dim,

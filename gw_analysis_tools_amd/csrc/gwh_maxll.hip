@@ -440,6 +440,7 @@ int gwh_maximized_loglike_batch(int event, int model, const gwh_params *params, 
     const double dfac = ev.df_like / 3.0;
     const double df = ev.df_fisher;                      /* f[1] - f[0] */
     const double hh_scale = ev.df_fisher / ev.df_like;  /* the stored Simpson step -> f[1] - f[0] */
+    SettleStream settle(st);
     for (int i0 = 0; i0 < n; i0 += chunk) {
         const int m = std::min(chunk, n - i0);
         const gwh_params *d_params = staged ? (const gwh_params *)E.stage.g : E.params.as<const gwh_params>();
@@ -470,7 +471,7 @@ int gwh_maximized_loglike_batch(int event, int model, const gwh_params *params, 
     }
     GWH_HIP(hipStreamSynchronize(st));
     if (staged) memcpy(out, E.stage.h + rec, (size_t)n * 8);
-    return GWH_OK;
+    return settle.done();
 }
 
 } // extern "C"
