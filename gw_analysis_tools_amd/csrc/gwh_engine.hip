@@ -535,7 +535,6 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const char *__restrict__
             T.m2 = S.m2;
             T.M = S.M;
             T.eta = S.eta;
-            T.ieta = S.ieta;
             T.iM = S.iM;
             T.chi1 = S.chi1;
             T.chi2 = S.chi2;

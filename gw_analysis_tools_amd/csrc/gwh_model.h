@@ -408,7 +408,7 @@ __device__ __forceinline__ double gwh_erad0815(double eta, double chi1, double c
 /* Everything the setup needs while building the record */
 struct SetupState {
     double m1, m2, M, eta, chi1, chi2, chi_s, chi_a, delta, chi_pn, chi_eff, Mc, A0;
-    double ieta, iM; /* 1 / eta, 1 / M */
+    double iM; /* 1 / M */
     double fRD, fdamp, f1, f3, f1p, f2p;
     double rho[3], v2, g[3], sigma[5], beta[4], alpha[6];
     double pa[7];  /* amplitude PN coefficients (reference numbering) */
@@ -704,7 +704,6 @@ __device__ __forceinline__ void gwh_setup_base(const gwh_params &p, int ppe, Set
     S.chi_s = 0.5 * (S.chi1 + S.chi2);
     S.chi_a = 0.5 * (S.chi1 - S.chi2);
     S.delta = sqrt(1. - 4. * S.eta);
-    S.ieta = 1.0 / S.eta;
     S.iM = 1.0 / S.M;
     S.chi_eff = (S.m1 * S.chi1 + S.m2 * S.chi2) / S.M;
     S.chi_pn = S.chi_eff - (38. * S.eta / 113.) * (2. * S.chi_s);
