@@ -1,7 +1,7 @@
-"""The IMRPhenomPv2 twist-up collected by powers of e^{i alpha} (gwh_pv2_twist), restated operation by operation, against
+"""The identity behind gwh_pv2_twist: the IMRPhenomPv2 twist-up collected by powers of e^{i alpha}, restated here, against
 the sum over m of the rotation elements d^2_{m,+-2}(beta) and the -2Y_2m it stands for (IMRPhenomP.cpp:290-361), over
-small and large opening angles.  Every coefficient is a polynomial in cos beta and sin beta, so 8 ulp of the largest
-term covers its ~10 roundings."""
+small and large opening angles.  The kernel itself is compared with that sum in test_gpu_pv2_twist.py.  Every
+coefficient is a polynomial in cos beta and sin beta, so 8 ulp of the largest term covers its ~10 roundings."""
 import numpy as np
 import pytest
 
