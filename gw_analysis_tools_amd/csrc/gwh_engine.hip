@@ -785,17 +785,17 @@ __global__ __launch_bounds__(256) void gwh_setup_kernel(const char *__restrict__
             C->phic = 2 * X.phi_aligned;
             C->tc_total = GWH_2PI * p.tc;
             C->f_ref = p.f_ref;
-            /* t_c alignment: 1 / (2 pi) times the derivative at fRD of a 10-knot natural spline of -Psi_MR
+            /* t_c alignment: 2 pi times the time shift, that is the derivative at fRD of a 10-knot natural spline of -Psi_MR
              * (IMRPhenomP.cpp:550-606); the spline of a line is the line, so its alpha1 part is exact */
-            double t_corr = 0;
+            double slope = 0;
             if (p.shift_time) {
                 double q[10];
 #pragma unroll
                 for (int j = 0; j < 10; j++) q[j] = X.tq[j];
-                t_corr = -(gwh_setup_tcorr(S.fRD, q) + S.alpha[1] * M / eta);
-                if (!(S.fRD > 0)) t_corr = 0;
+                slope = -(gwh_setup_tcorr(S.fRD, q) + S.alpha[1] * M / eta);
+                if (!(S.fRD > 0)) slope = 0;
             }
-            C->t_corr_2pi = t_corr;
+            C->t_corr_2pi = slope;
         }
     }
 }

@@ -229,7 +229,7 @@ struct InstCoef {
     double beta[4];          /* beta_k / eta (beta_3 / (3 eta)) */
     double alpha[6];         /* alpha_k / eta ((4/3) alpha_3 / eta) ; alpha[5] = alpha_5 fRD */
     double tc_total, phic, f_ref; /* phi = Psi - tc_total (f - f_ref) - phic (Pv2: + t_corr term) */
-    double t_corr_2pi;       /* Pv2: 2 pi t_corr */
+    double t_corr_2pi;       /* Pv2: 2 pi times the t_c correction */
     /* Pv2 precession */
     double SP, SL, L_c1, L_c2; /* L2PN: eta (1 + L_c1 x + L_c2 x^2) / sqrt(x) */
     double a_c[5], e_c[5];   /* Euler alpha / epsilon coefficients */
@@ -1040,7 +1040,7 @@ __device__ __forceinline__ void gwh_setup_detectors(const gwh_params &p, bool pv
     }
 }
 
-/* role 2, phase 2: amplitude C1 connection, the Hermite quartic through (f1, v1, v1'), (f2, v2), (f3, v3, v3')
+/* role 3, phase 2: amplitude C1 connection, the Hermite quartic through (f1, v1, v1'), (f2, v2), (f3, v3, v3')
  * with f2 = (f1 + f3) / 2 (IMRPhenomD.cpp:1679-1702), as coefficients of powers of f */
 __device__ __forceinline__ void gwh_setup_amp_connection(double iM, double f1, double f3, double v1, double d1,
                                                          double v2, double v3, double d3, double *out)

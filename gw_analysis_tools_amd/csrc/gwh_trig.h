@@ -5,7 +5,7 @@
  * FP64 carries a large-argument (Payne-Hanek) reduction for every call; gwh_sincos_cw, for the per-instance setup,
  * reduces by Cody and Waite's method (W. J. Cody, W. Waite, Software Manual for the Elementary Functions, 1980):
  * q = rint(x 2/pi), r = (x - q p1) - q p2 with pi/2 = p1 + p2 split into two doubles and each step one
- * fused multiply-add (x - q p1 is exact by Sterbenz's lemma, the neglected part of pi/2 is 1e-33), then sin r and
+ * fused multiply-add (x - q p1 fits a double, so it is exact; the neglected part of pi/2 is 1.5e-33), then sin r and
  * cos r on [-pi/4, pi/4] by their Taylor series and the quadrant by q mod 4.
  *
  * gwh_sincos_table and gwh_exp_table trade the long series for a table lookup (gwh_trig_tables.h, 4.5 kB,
