@@ -573,17 +573,17 @@ __global__ __launch_bounds__(WAVES * 64) void gwh_fisher_fused_kernel(StencilArg
     if (a.row[wv][0] >= 0) {
         f = gwh_g(E.f)[k];
         bp = gwh_load_bin(E, k);
+#pragma unroll
+        for (int dd = 0; dd < (SKY ? 1 : GWH_MAXDET); dd++)
+            if (dd < a.d_count) sw[dd] = in ? sqrt(gwh_g(E.wS)[(size_t)(a.d_first + dd) * N + k]) : 0.0;
         /* a lane above the cutoff evaluates its bin with a zero amplitude, so the phase has to be finite: a bin of
-           infinite frequency, or none, is taken at 1e15 Hz, above every cutoff (a branch that no other wave enters; selects
-           in every wave took 2 % of the kernel) */
+           infinite frequency, or none, is taken at 1e15 Hz, above every cutoff (a branch that no other wave enters, behind the
+           loads: selects in every wave took 2 % of the kernel, the branch in front of the weights' loads 1.5 %) */
         if (!SKY && __ballot(!(f < HUGE_VAL))) {
             const bool none = !(f < HUGE_VAL);
             f = none ? 1e15 : f;
             bp = none ? BinPow{34.538776394910684, 1e5, 1e-5, 3.1622776601683795e-18, 1.7782794100389228e11} : bp;
         }
-#pragma unroll
-        for (int dd = 0; dd < (SKY ? 1 : GWH_MAXDET); dd++)
-            if (dd < a.d_count) sw[dd] = in ? sqrt(gwh_g(E.wS)[(size_t)(a.d_first + dd) * N + k]) : 0.0;
         if (SKY) {
             const InstCoef &Cc = C[a.dim * S];
             double ph;
