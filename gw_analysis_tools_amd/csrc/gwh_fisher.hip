@@ -518,8 +518,8 @@ __global__ __launch_bounds__(GWH_TPB) void gwh_gram_kernel(const float *__restri
 /* Column of the LDS plane that holds bin `col` of operand row `row` in the fused kernel: rows are rotated by two
  * bins each, so that the 32 lanes of a half wave, which read bins 4 q + {0, 1} or {2, 3} of all 16 rows, touch 32
  * different bank pairs.  Unrotated, the 16 rows (512 bytes apart) share their banks: SQ_LDS_BANK_CONFLICT was 9.4e7
- * of 1.2e8 LDS cycles of a 128-point pass of the 13-parameter IMRPhenomPv2 Fisher (846 -> 838 us: the vector ALU
- * covered most of them). */
+ * of 1.2e8 LDS cycles of a 128-point pass of the 13-parameter IMRPhenomPv2 Fisher (846 -> 838 us: the
+ * evaluations covered most of them). */
 __device__ __forceinline__ int fused_col(int row, int col) { return (col + 2 * row) & (GWH_FUSED_BINS - 1); }
 
 /* The stencil and the FP64 Gram in one kernel: one block of WAVES waves per (point, chunk of 64 bins).  Each wave
@@ -536,7 +536,8 @@ __device__ __forceinline__ int fused_col(int row, int col) { return (col + 2 * r
  * construction) is kept in registers instead of computed again, and rows that share are given to the same wave:
  * 12 instead of 22 evaluations of the waveform for the 11 IMRPhenomD parameters (4 rows change it, the other 7 lie
  * in 4 waves), 13 instead of 26 for the 13 of IMRPhenomPv2.  The arithmetic of an operand does not depend on which wave does it or after
- * what.  Bound by the vector ALU; per launch, every evaluation in full -> shared, over the live chunks only:
+ * what.  Two blocks share a CU by their LDS, 4 waves a SIMD, which issue 41 % (IMRPhenomPv2) and 46 % (IMRPhenomD) of
+ * the vector rate and wait for 62 and 50 % of their cycles.  Per launch, every evaluation in full -> shared, over the live chunks only:
  * IMRPhenomPv2, 128 points x 16225 bins x 3 detectors 838 -> 307 us, IMRPhenomD, 12 points x 65539 bins x 3 418 -> 238
  * us; the 7-parameter sky-averaged matrix of one point on 4017 bins, which went through operand rows in HBM, 36 ->
  * 8.5 us.
