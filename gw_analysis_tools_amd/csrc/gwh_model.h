@@ -888,8 +888,9 @@ __device__ __forceinline__ void gwh_setup_mass(const gwh_params &p, int ppe, Set
 struct Pv2Frame {
     double cJN, sJN, c2z, s2z, alpha0, phi_aligned;
 };
-/* cosine and sine of atan2(y, x), which is 0 or pi where x and y are zeros, by the sign of x.  Scaled by a power of 2, so
- * that no square under- or overflows. */
+/* cosine and sine of atan2(y, x), zeros and their signs included: atan2 of two zeros is 0 or pi by the sign of x, and next
+ * to a right angle it is the double pi/2, whose cosine is 6e-17 whatever the sign of x.  Scaled by a power of 2, so that no
+ * square under- or overflows. */
 __device__ __forceinline__ void gwh_direction(double x, double y, double &c, double &s)
 {
     const int e = -__builtin_amdgcn_frexp_exp(fmax(fabs(x), fabs(y)));
@@ -898,6 +899,7 @@ __device__ __forceinline__ void gwh_direction(double x, double y, double &c, dou
     y = ldexp(y, e);
     const double ih = none ? 0.0 : 1.0 / sqrt(x * x + y * y);
     c = none ? copysign(1.0, x) : x * ih;
+    c = fabs(c) < 4.98e-17 ? 6.123233995736766e-17 : c; /* pi/2 + |c| rounds to the double pi/2 = pi/2 - 6.12e-17 */
     s = y * ih;
 }
 __device__ __forceinline__ void gwh_rotz_cs(double c, double s, double &x, double &y)
@@ -940,7 +942,8 @@ __device__ __forceinline__ Pv2Frame gwh_setup_frame(const gwh_params &p, const S
     double cP, sP, cJ, sJ, cK, sK;
     gwh_direction(J0x, J0y, cP, sP);
     gwh_direction(J0z, J0x * cP + J0y * sP, cJ, sJ);
-    if (fabs(J0z) == J0 && J0 < HUGE_VAL) { /* a tilt that the reference's acos(J0z / J0) rounds to 0 or pi */
+    const bool flat = fabs(J0z) == J0 && J0 < HUGE_VAL; /* a tilt that the reference's acos(J0z / J0) rounds to 0 or pi */
+    if (flat) {
         cJ = copysign(1.0, J0z);
         sJ = J0z < 0 ? 1.2246467991473532e-16 : 0.0; /* sin of the double next to pi */
     }
@@ -952,8 +955,15 @@ __device__ __forceinline__ Pv2Frame gwh_setup_frame(const gwh_params &p, const S
     gwh_sincos_cw(p.incl, si, ci);
     gwh_sincos_cw(p.phiRef, sph, cph);
     /* line of sight N = (sin i cos(pi/2 - phi), sin i sin(pi/2 - phi), cos i), then rotated by kappa about z into the
-       x-z plane */
-    double tx = si * sph, ty = si * cph, tz = ci;
+       x-z plane; pi/2 - phi rounded as the reference rounds it where that shows: where phi is large, and where the sign of a
+       rounding error of N decides alpha0 */
+    double cr = sph, sr = cph;
+    if (flat || !(fabs(p.phiRef) < 1e6)) { /* the library's copy: no code in the way of the others */
+        const double2 r = gwh_sincos_huge(GWH_PI / 2. - p.phiRef);
+        sr = r.x;
+        cr = r.y;
+    }
+    double tx = si * cr, ty = si * sr, tz = ci;
     gwh_rotz_cs(cP, sP, tx, ty);
     gwh_roty_cs(cJ, sJ, tx, tz);
     gwh_direction(tx, -ty, cK, sK);

@@ -23,8 +23,8 @@ def net():
     ev.close()
 
 
-def _edges(kind):
-    base = W.precessing_params(1) if kind != "angles" else W.injection_params(1)
+def _edges(kind, model):
+    base = W.precessing_params(1) if model == G.IMRPHENOMPV2 else W.injection_params(1)
     out = []
 
     def add(**kw):
@@ -57,6 +57,12 @@ def _edges(kind):
                 add(mass1=30., mass2=30., spin1=[.5, x, .2], spin2=[-.5, 0, .2], incl=1.2, phiRef=phi)
                 add(mass1=30., mass2=30., spin1=[x, .5, .2], spin2=[0, -.5, .2], incl=1.2, phiRef=phi)
             add(mass1=30., mass2=30., spin1=[-0., .5, .2], spin2=[-0., -.5, .2], incl=1.2, phiRef=phi)
+        # the line of sight in a coordinate plane, where its azimuth is a rounding error away from a quadrant
+        for phi in (0., -0., np.pi / 2, np.pi, -np.pi / 2, 2 * np.pi):
+            for inc in (1.2, -1.2, 2.5, -2.5):
+                for a in (.5, -.3):
+                    add(mass1=30., mass2=30., spin1=[a, -.1, .2], spin2=[-a, .1, .2], incl=inc, phiRef=phi)
+                    add(mass1=30., mass2=30., spin1=[0, a, -.7], spin2=[0, -a, .7], incl=inc, phiRef=phi)
     elif kind == "reference":
         for fr in (5., 20., 60., 100., 200., 300., 500., 1000.):
             for st in (0, 1):
@@ -66,15 +72,19 @@ def _edges(kind):
         for k in ("incl", "psi", "RA", "DEC", "gmst"):
             for v in (-1e5, 2. ** 40, -2. ** 40 * (1 - 2. ** -53), 1e17, 1e300):
                 add(**{k: v})
+        if model == G.IMRPHENOMPV2:  # phiRef only places the line of sight there, as pi/2 - phiRef
+            for v in (1e5, -1e7, 1e10, 1e17, -1e300):
+                add(phiRef=v)
     return np.array(out, dtype=base.dtype)
 
 
 @pytest.mark.parametrize("kind,model", [("geometry", G.IMRPHENOMPV2), ("cancelling", G.IMRPHENOMPV2),
                                         ("reference", G.IMRPHENOMD),
-                                        ("reference", G.IMRPHENOMPV2), ("angles", G.IMRPHENOMD)])
+                                        ("reference", G.IMRPHENOMPV2), ("angles", G.IMRPHENOMD),
+                                        ("angles", G.IMRPHENOMPV2)])
 def test_degenerate_setups_match_oracle(net, kind, model):
     f, psd, data, ev = net
-    P = _edges(kind)
+    P = _edges(kind, model)
     a = G.loglike_batch(ev, P, model)
     for i, r in enumerate(P):
         p = O.make_params(**{k: (r[k].tolist() if r[k].shape else r[k].item()) for k in r.dtype.names})
