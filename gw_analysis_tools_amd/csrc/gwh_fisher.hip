@@ -535,12 +535,14 @@ __device__ __forceinline__ int fused_col(int row, int col) { return (col + 2 * r
  * phase in a detector.  What an evaluation shares with the one its wave did before (GWH_EV_SAME_*, equal bits by
  * construction) is kept in registers instead of computed again, and rows that share are given to the same wave:
  * 12 instead of 22 evaluations of the waveform for the 11 IMRPhenomD parameters (4 rows change it, the other 7 lie
- * in 4 waves), 13 instead of 26 for the 13 of IMRPhenomPv2.  The arithmetic of an operand does not depend on which wave does it or after
- * what.  Two blocks share a CU by their LDS, 4 waves a SIMD, which issue 41 % (IMRPhenomPv2) and 46 % (IMRPhenomD) of
- * the vector rate and wait for 62 and 50 % of their cycles.  Per launch, every evaluation in full -> shared, over the live chunks only:
+ * in 4 waves), 13 instead of 26 for the 13 of IMRPhenomPv2.  The arithmetic of an operand does not depend on which
+ * wave does it or after what.  Per launch, every evaluation in full -> shared, over the live chunks only:
  * IMRPhenomPv2, 128 points x 16225 bins x 3 detectors 838 -> 307 us, IMRPhenomD, 12 points x 65539 bins x 3 418 -> 238
  * us; the 7-parameter sky-averaged matrix of one point on 4017 bins, which went through operand rows in HBM, 36 ->
  * 8.5 us.
+ *
+ * Two blocks share a CU by their LDS: 4 waves a SIMD, which issue 41 % (IMRPhenomPv2) and 46 % (IMRPhenomD) of the
+ * vector rate and wait for 62 and 50 % of their cycles.
  *
  * SKY: the sky-averaged IMRPhenomD basis, d h = dA + i sign d(phase) A_central (fisher.cpp:292-316) in planes
  * (dA, d(phase) A) of one detector row. */

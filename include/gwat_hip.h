@@ -87,8 +87,8 @@ extern "C" {
 
 /* arithmetic of the batched kernels */
 #define GWH_FP64 0  /* everything in FP64 */
-#define GWH_MIXED 1 /* FP64 except the FP32 operations that are faster on gfx950: the IMRPhenomD merger-ringdown
-                       exponential and the IMRPhenomPv2 reciprocal square root's seed */
+#define GWH_MIXED 1 /* FP64 except the FP32 operation that is faster on gfx950, the IMRPhenomD merger-ringdown
+                       exponential; IMRPhenomPv2 and its modifications run the GWH_FP64 kernels */
 
 /* integration rules of Log_Likelihood_internal (mcmc_gw.cpp:801-868) */
 #define GWH_SIMPSONS 0

@@ -15,7 +15,7 @@ same constants and operation order, against 50-digit mpmath values:
   for seeds within 2^-26, as the hardware FP64 reciprocal's), and the reciprocal square root from an FP32 seed
   and two Newton steps (rsqrt_seeded) is within 4 ulp of z^(-1/2) over [1, 1e12] for any seed within 2^-22; a
   step with the wrong sign, or one step short, is caught;
-* the IMRPhenomPv2 half angle sin(b/2) = |s| cos b / (2 cos(b/2)) with cos b = (1 + s^2)^(-1/2) is within 4 ulp of
+* (of a form of the twist-up that no kernel uses any more) the IMRPhenomPv2 half angle sin(b/2) = |s| cos b / (2 cos(b/2)) with cos b = (1 + s^2)^(-1/2) is within 4 ulp of
   sin(atan(s) / 2) for s from 1e-8 to 1e4, where sqrt((1 - cos b) / 2) loses digits as s -> 0."""
 import os
 import re
